@@ -355,8 +355,8 @@ static TensorView kq_rows_view(const TensorView &v, int expert, int64_t r0, int6
 // is one they take, else the eight-row lane tiles. Every choice gives the reference's bits;
 // SPX_MV_MODE forces one (0: lane tiles, 1: row-parallel, 2: matrix cores where they apply).
 // Float formats: eight rows a wavefront (the reference's M = 1 order); Q8_0 with two or more
-// rows on the fp32 matrix cores (k_mv_fq, the multi-row order of quant_multi.rs's kernel,
-// within 1e-4 of it; a row's bits do not depend on the other rows of the batch).
+// rows on the bf16 matrix cores (k_fx_mv: within 1e-4 of quant_multi.rs's kernel; a row's bits do
+// not depend on the other rows of the batch).
 static int mv_launch(spx_ctx *ctx, const spx_tensor *w, int expert, int m, const float *x, int64_t ld_x, Q8KP y, float *out,
                      int64_t ld_out, int64_t r0, int64_t r1) {
   const bool kq = w->v.dtype == T_Q4K || w->v.dtype == T_Q6K;
@@ -393,7 +393,7 @@ static int mv_launch(spx_ctx *ctx, const spx_tensor *w, int expert, int m, const
   a.m = m;
   a.G = G;
   a.R = R;
-  a.fq = !kq && m >= FQ_MIN_ROWS ? 1 : 0;
+  a.fx = w->v.dtype == T_Q8_0 && m >= FX_MIN_ROWS ? 1 : 0;
   SPX_HIP(launch_mv(a, m, mode, nullptr, a.seg[0].wgs, ctx->stream));
   return 0;
 }

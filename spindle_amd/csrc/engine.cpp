@@ -23,6 +23,7 @@
 #include "../../include/spx.h"
 #include "decode.h"
 #include "fused.h"
+#include "fx.h"
 #include "internal.h"
 #include "persist.h"
 #include "kv.h"
@@ -95,6 +96,9 @@ struct spx_engine {
   // prologues and the residual adds in the producers' epilogues instead of last-workgroup
   // tails (the same bits; SPX_FPRO=0 keeps the tails)
   bool fpro = false;
+  // passes of 17..128 rows of a float model on the fused path's matrix-core kernels (fx.hip; attention
+  // on the multi-tile kernels): every row the bits of its pass of 2..16 rows
+  bool fx_pf = false;
   // one-row passes with their layers as cooperative launches (persist.hip), where the model
   // fits its tiles; off by default: measured slower than the pipeline (SPX_PERSIST=1 or
   // spx_engine_set_persist turns it on)
@@ -116,7 +120,7 @@ struct spx_engine {
   float *xA = nullptr, *xB = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *att = nullptr, *proj = nullptr, *ffn = nullptr;
   float *xn2 = nullptr, *h = nullptr, *rlog = nullptr, *logits = nullptr, *xn = nullptr, *part_ml = nullptr, *part_o = nullptr;
   Q8KP aq{}, xq2{}, hq{}, xq{};
-  int *amax = nullptr, *att_cnt = nullptr, *rt_cnt = nullptr, *gu_cnt = nullptr, *tail_cnt = nullptr, *dn_cnt = nullptr;
+  int *amax = nullptr, *att_cnt = nullptr, *rt_cnt = nullptr, *gu_cnt = nullptr, *tail_cnt = nullptr;
   unsigned long long *best = nullptr;
   int *hist = nullptr;  // token history of back-to-back decode passes [max_seq]
   int *chosen = nullptr, *nkeep = nullptr, *expert_count = nullptr;
@@ -264,7 +268,7 @@ int mv_run(spx_engine *E, MVArgs &a, int m, int mode, int grid_cap = 0) {
   if (grid_cap > 0 && grid > grid_cap) grid = grid_cap;
   a.m = m;
   a.nbest = grid;
-  a.fq = E->mq ? 1 : 0;
+  a.fx = E->mq ? 1 : 0;
   SPX_HIP(launch_mv(a, m, mode, E->st_dev, grid, E->ctx->stream));
   return 0;
 }
@@ -310,13 +314,38 @@ int mv_res(spx_engine *E, const spx_tensor *w, const float *x, int64_t ld_x, flo
   return mv_run(E, a, 1, 0);
 }
 
+// Integer matvec of m <= 16 rows of Q8_K activations, no step record (a slice of a longer pass).
+int mv_rows(spx_engine *E, const spx_tensor *w, int m, Q8KP y, float *out, int64_t ld_out) {
+  const int mode = mode_of(E, w, m);
+  MVArgs a{};
+  a.G = 8;
+  a.R = 1;
+  rp_shape(w->v.nb, a.G, a.R);
+  a.seg[0] = seg_of(w, out, ld_out, m, mode, a.R);
+  a.nseg = 1;
+  a.y = y;
+  a.lscale = E->c.logit_scale;
+  a.m = m;
+  SPX_HIP(launch_mv(a, m, mode, nullptr, a.seg[0].wgs, E->ctx->stream));
+  return 0;
+}
+
+// A MoE layer whose passes of 2..128 rows run on the bf16 matrix cores: float experts, and a row
+// width that the multi-row router and norm take.
+bool fx_moe(const spx_engine *E, const LayerW &ly) {
+  return ly.moe && fx_type(ly.gate->v.dtype) && fx_type(ly.up->v.dtype) && fx_type(ly.down->v.dtype) && ly.router->v.dtype == T_F32 &&
+         E->c.dim % 256 == 0 && E->c.dim <= 256 * DEC_MAXNB;
+}
+
 // One forward pass of m rows at the step record's start position: embeddings through the
 // LM head and the greedy pick (forward_slice / forward_batch_slice + compute_logits_batch).
 // Residual stream: the embedding writes xA; attn_output's norm tail adds its output to xA
 // and writes xB; the FFN's tail adds its output to xB and writes xA.
 // Attention of a pass of m unprepared rows: the multi-tile kernels (launch_attention_mt) from
-// att_mt_min rows, else the tile-per-workgroup kernel; both give the same bits.
+// att_mt_min rows (and for passes of more than 16), else the tile-per-workgroup kernel; both give
+// the same bits.
 hipError_t attn_launch(spx_engine *E, const AttnArgs &aa, int m, hipStream_t s) {
+  if (m > MAX_M) return launch_attention_mt(aa, m, E->st_dev, s);  // a float model's prefill pass (fx_pf)
   if (E->att_mt_min > 0 && m >= E->att_mt_min && m <= MAX_M && !aa.prepped && (aa.hd == 64 || aa.hd == 128) &&
       (!aa.q_bias || (aa.n_heads / aa.n_kv) * aa.hd <= 2048))
     return launch_attention_mt(aa, m, E->st_dev, s);
@@ -419,6 +448,36 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
     const int gmode = m <= 2 ? mode_of(E, ly.gate, m) : 0;  // grouped experts: row-parallel at decode, tiles for verify
     if (ly.moe) {  // moe_forward / moe_forward_batch (:925-1392)
       const int nu = c.n_expert_used, ne = c.n_expert;
+      if (fx_moe(E, ly) && E->mq && m >= FX_MIN_ROWS) {
+        // float experts, 2..128 rows: the router's rows, the routing and a job list of at most 16
+        // users a job (the K-quant prefill passes' kernels), the experts on the bf16 matrix cores,
+        // then the combine in choice order and the next norm in one launch
+        {
+          ProfScope ps(E, PC_ROUTER, wbytes(ly.router));
+          SPX_HIP(launch_dec_router_m(DecRouterMArgs{ly.router->v, E->xn2, E->rlog, ne, dim, m}, s));
+          SPX_HIP(launch_kp_route(DecRouteArgs{E->rlog, ne, nu, c.expert_norm, m, c.moe_prune, E->chosen, E->weights, E->nkeep, E->jobs, ly.njobs,
+                                               E->expert_count + (size_t)l * ne}, s));
+        }
+        const int max_jobs = std::min(512, std::min(ne, m * nu) + (m * nu) / MAX_M);
+        {
+          ProfScope ps(E, PC_GATEUP, wbytes(ly.gate) + wbytes(ly.up), l, true);  // one expert's slabs
+          GUArgs ga{};
+          ga.gate = ly.gate->v; ga.up = ly.up->v; ga.x = E->xn2; ga.jobs = E->jobs; ga.njobs = ly.njobs; ga.h = E->h; ga.n_ff = nff;
+          SPX_HIP(launch_fx_gateup(ga, m, E->st_dev, max_jobs, s));
+        }
+        {
+          ProfScope ps(E, PC_DOWN, wbytes(ly.down), l, true);
+          DownArgs da{};
+          da.w = ly.down->v; da.x = E->h; da.jobs = E->jobs; da.njobs = ly.njobs; da.yd = E->yd;
+          SPX_HIP(launch_fx_down(da, max_jobs, s));
+        }
+        ProfScope ps(E, PC_NORM, 0);
+        DecNormArgs na{};
+        na.x = E->xA; na.nw = tn.nw; na.eps = c.rms_eps; na.dim = dim; na.xn_out = tn.xn_out; na.q_out = tn.q_out;
+        na.yd = E->yd; na.cw = E->weights; na.nkeep = E->nkeep; na.res_in = E->xB; na.x_out = E->xA; na.n_used = nu; na.rscale = c.residual_scale;
+        SPX_HIP(launch_dec_norm(na, m, s));
+        continue;
+      }
       {
         ProfScope ps(E, PC_ROUTER, wbytes(ly.router));
         RouterArgs ra{};
@@ -430,10 +489,6 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
         SPX_HIP(launch_router(ra, m, E->st_dev, s));
       }
       const int max_gu_jobs = std::min(256, m * nu);  // jobs of at most GU_USERS users
-      // Q8_0 experts, 2..16 rows: gate/up and down on the fp32 matrix cores, a job per expert
-      const bool fq = E->mq && m >= FQ_MIN_ROWS && m <= MAX_M && ly.gate->v.dtype == T_Q8_0 && ly.up->v.dtype == T_Q8_0 &&
-                      ly.down->v.dtype == T_Q8_0;
-      const int max_dn_jobs = std::min(ne, m * nu);
       {
         ProfScope ps(E, PC_GATEUP, wbytes(ly.gate) + wbytes(ly.up), l, true);  // one expert's slabs
         GUArgs ga{};
@@ -447,12 +502,7 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
           rt.chosen = E->chosen; rt.weights = E->weights; rt.nkeep = E->nkeep; rt.jobs = E->jobs + 256; rt.njobs = ly.njobs;
           rt.expert_count = E->expert_count + (size_t)l * ne;
         }
-        if (fq) {
-          ga.jobs = E->jobs + 256; ga.njobs = ly.njobs; ga.vdiv = nu; ga.fq = 1;
-          SPX_HIP(launch_gateup(ga, m, 0, E->st_dev, max_dn_jobs, s));
-        } else {
-          SPX_HIP(launch_gateup(ga, std::min(m, GU_USERS), mode_of(E, ly.gate, m), E->st_dev, max_gu_jobs, s));
-        }
+        SPX_HIP(launch_gateup(ga, std::min(m, GU_USERS), mode_of(E, ly.gate, m), E->st_dev, max_gu_jobs, s));
       }
       {
         ProfScope ps(E, PC_DOWN, wbytes(ly.down), l, true);
@@ -461,12 +511,7 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
         da.nkeep = E->nkeep; da.n_used = nu; da.out = E->ffn;
         if (pro) { da.res_in = E->xB; da.res_out = E->xA; da.rscale = c.residual_scale; }
         else if (tails) da.tail = tn;
-        if (fq) {
-          da.yd = E->yd; da.counter = E->dn_cnt;
-          SPX_HIP(launch_down_fq(da, max_dn_jobs, E->st_dev, s));
-        } else {
-          SPX_HIP(launch_down(da, m, m > 2 && d_int && E->down_mode == 1 ? 1 : 0, E->st_dev, s));
-        }
+        SPX_HIP(launch_down(da, m, m > 2 && d_int && E->down_mode == 1 ? 1 : 0, E->st_dev, s));
       }
       if (!tails && !pro) { ProfScope ps(E, PC_NORM, 0); SPX_HIP(launch_norm(tn, E->st_dev, m, s)); }
     } else {  // ffn_forward / ffn_forward_multi (:590-646): k = 1, w = 1
@@ -474,15 +519,23 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
         ProfScope ps(E, PC_GATEUP, wbytes(ly.gate) + wbytes(ly.up));
         GUArgs ga{};
         ga.gate = ly.gate->v; ga.up = ly.up->v; ga.y = E->xq2; ga.x = E->xn2; ga.h = E->h; ga.counter = E->gu_cnt; ga.n_ff = nff;
-        ga.fq = E->mq && m >= FQ_MIN_ROWS ? 1 : 0;
-        if (d_int) ga.hq = E->hq;
-        if (pro) ga.pro = pro_of(E->xB, ly.ffn_norm, nullptr);
-        SPX_HIP(launch_gateup(ga, m, gmode, E->st_dev, 1, s));
+        if (E->mq && m >= FX_MIN_ROWS && fx_type(ly.gate->v.dtype) && fx_type(ly.up->v.dtype)) {
+          SPX_HIP(launch_fx_gateup(ga, m, E->st_dev, 1, s));
+          if (d_int) SPX_HIP(launch_q8kp_quantize(E->h, nff, nff, m, E->hq, s));
+        } else {
+          if (d_int) ga.hq = E->hq;
+          if (pro) ga.pro = pro_of(E->xB, ly.ffn_norm, nullptr);
+          SPX_HIP(launch_gateup(ga, m, gmode, E->st_dev, 1, s));
+        }
       }
       {
         ProfScope ps(E, PC_DOWN, wbytes(ly.down));
         if (pro) {
           if (int r = mv_res(E, ly.down, E->h, nff, E->ffn, E->xB, E->xA)) return r;
+        } else if (d_int && m > MAX_M) {  // a K-quant down of a float model's prefill pass: 16 rows a launch
+          for (int r0 = 0; r0 < m; r0 += MAX_M)
+            if (int r = mv_rows(E, ly.down, std::min(MAX_M, m - r0), q8kp_row(E->hq, r0, nff), E->ffn + (int64_t)r0 * dim, dim)) return r;
+          SPX_HIP(launch_norm(tn, E->st_dev, m, s));
         } else {
           if (int r = mv_one(E, ly.down, m, E->h, nff, E->hq, E->ffn, dim, &tn, tails, PC_NORM)) return r;
         }
@@ -518,7 +571,8 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
       SPX_HIP(launch_mv(a, 1, mode, nullptr, grid, s));
       E->nbest = grid;
     } else {
-      if (int r = mv_run(E, a, m, mode, mode == 0 ? E->lm_grid : 0)) return r;
+      const bool fx = E->mq && m >= FX_MIN_ROWS && fx_type(E->lm_head->v.dtype);
+      if (int r = mv_run(E, a, m, mode, fx ? fx_mv_wgs(E->lm_head->v, m) : mode == 0 ? E->lm_grid : 0)) return r;
       E->nbest = a.nbest;
     }
   }
@@ -1110,7 +1164,7 @@ int spx_engine_prepare(spx_engine *E) {
             (E->h = E->dalloc<float>((size_t)nv * nff)) && (E->yd = E->dalloc<float>((size_t)nv * c.dim)) && (E->rlog = E->dalloc<float>((size_t)M * std::max(1, c.n_expert))) &&
             (E->logits = E->dalloc<float>((size_t)M * c.vocab)) && (E->amax = E->dalloc<int>(M)) &&
             (E->best = E->dalloc<unsigned long long>((size_t)M * std::max<int64_t>(E->lm_grid, c.vocab / 4 + 1))) &&
-            (E->tail_cnt = E->dalloc<int>((size_t)(1 + CNT_SUB) * CNT_STRIDE)) && (E->dn_cnt = E->dalloc<int>((size_t)(2 + c.dim / 32) * CNT_STRIDE)) && (E->hist = E->dalloc<int>((size_t)c.max_seq)) &&
+            (E->tail_cnt = E->dalloc<int>((size_t)(1 + CNT_SUB) * CNT_STRIDE)) && (E->hist = E->dalloc<int>((size_t)c.max_seq)) &&
             (E->part_ml = E->dalloc<float>((size_t)c.n_kv_heads * (E->nch + ATT_GMAX) * ATT_QMAX * 2)) &&
             (E->part_o = E->dalloc<float>((size_t)c.n_kv_heads * (E->nch + ATT_GMAX) * ATT_QMAX * c.head_dim)) &&
             (E->att_cnt = E->dalloc<int>((size_t)c.n_kv_heads * ATT_QT * (1 + ATT_GMAX) * CNT_STRIDE)) && (E->rt_cnt = E->dalloc<int>((size_t)(1 + CNT_SUB) * CNT_STRIDE)) &&
@@ -1159,6 +1213,16 @@ int spx_engine_prepare(spx_engine *E) {
     }
     if (const char *v = std::getenv("SPX_FPRO")) fp = fp && atoi(v) != 0;
     E->fpro = fp;
+  }
+  {
+    bool ok = E->att_mt_min > 0 && c.n_heads / c.n_kv_heads >= 2 && fx_type(E->lm_head->v.dtype);
+    for (auto &ly : E->L) {
+      for (const spx_tensor *t : {ly.wq, ly.wk, ly.wv, ly.wo, ly.gate, ly.up}) ok = ok && fx_type(t->v.dtype);
+      ok = ok && ly.wk->v.dtype == ly.wq->v.dtype && ly.wv->v.dtype == ly.wq->v.dtype;
+      ok = ok && (ly.moe ? fx_moe(E, ly) : fx_type(ly.down->v.dtype) || is_kq(ly.down));
+      ok = ok && (!ly.q_bias || (c.n_heads / c.n_kv_heads) * c.head_dim <= 2048);
+    }
+    E->fx_pf = ok;
   }
   // passes of 2..16 rows: expert down rows of at most 4 blocks (n_ff <= 1024)
   // the down kernel stages every user's Q8_K h row in LDS: 16 rows x n_used users
@@ -1280,7 +1344,7 @@ int forward_sel(spx_engine *E, const int32_t *ids, int m, int start_pos, float *
   if (start_pos < 0 || start_pos + m > E->c.max_seq) return fail("spx_engine_forward: positions beyond max_seq (the KV window is full)");
   for (int i = 0; i < m; i++)
     if (ids[i] < 0 || ids[i] >= E->c.vocab) return fail("spx_engine_forward: token id out of range");
-  if (m > MAX_M && !(E->dec_ok && E->dec_on && E->mq && E->mq_shapes)) {
+  if (m > MAX_M && !(E->mq && (E->dec_ok && E->dec_on ? E->mq_shapes : E->fx_pf))) {
     // no prefill kernels for this model / setting: passes of at most 16 rows, one after the
     // other (a row's results do not depend on the rows that share its pass)
     for (int r0 = 0; r0 < m; r0 += MAX_M) {

@@ -69,9 +69,9 @@ struct MVArgs {
   int nbest;
   float lscale;
   NormTail tail;
-  // float path, passes of FQ_MIN_ROWS..16 rows: Q8_0 segments on the fp32 matrix cores
-  // (k_mv_fq) instead of the per-lane walk (the same products, summed in another order)
-  int fq;
+  // float path, FX_MIN_ROWS rows and more: Q8_0 or Q5_0 segments of one format and width on the bf16 matrix
+  // cores (launch_fx_mv) instead of the per-lane walk (the same products, summed in another order)
+  int fx;
   // one-row Q8_0 passes (k_mv_f1 only): pro.nw set: the input row is pro.x, normalised by every
   // workgroup as norm_rows would (workgroup 0 also writes pro.xn_out); res_out set: residual
   // epilogue res_out[r] = res_in[r] + rscale * y[r] (one segment)
@@ -80,7 +80,7 @@ struct MVArgs {
   float *res_out;
   float rscale;
 };
-constexpr int FQ_MIN_ROWS = 2;  // one-row passes keep the per-lane walk (a 16-vector tile would idle 15 columns)
+constexpr int FX_MIN_ROWS = 2;  // one-row passes keep the per-lane walk (a 16-vector tile would idle 15 columns)
 
 struct AttnArgs {
   const float *q, *k, *v;             // raw projections [m][q_dim], [m][kv_dim]
@@ -156,8 +156,6 @@ struct GUArgs {
   int *counter;                       // [vectors][n_ff/256][1 + GU_SUB][CNT_STRIDE], zero between passes
   int n_ff;
   int G;                              // row-parallel launch: lane groups per row
-  int fq;                             // Q8_0, 2..16 rows: on the fp32 matrix cores (k_gateup_fq)
-  int vdiv;                           // > 1: a job's vec entries are h indices (row * vdiv + slot), the input row their quotient
   NormTail pro;                       // one-row float passes (k_gateup_f): pro.nw set: x is pro.x, normalised in every workgroup
   F1Route rt;                         // one-row float passes (k_gateup_f): routing in the prologue
 };
@@ -174,8 +172,7 @@ struct DownArgs {
   float *out;                         // [m][dim]
   int G;                              // row-parallel launch: lane groups per row
   NormTail tail;
-  float *yd;                          // launch_down_fq: y per (row, slot) [m * n_used][dim]
-  int *counter;                       // launch_down_fq: arrivals per 32 output rows [dim / 32][CNT_STRIDE] (+ one), zero between passes
+  float *yd;                          // launch_fx_down: y per (row, slot) [m * n_used][dim]
   const float *res_in;                // k_down_f: residual epilogue res_out = res_in + rscale * out (instead of a tail)
   float *res_out;
   float rscale;
@@ -209,10 +206,6 @@ hipError_t launch_attention_mt(const AttnArgs &a, int m, const StepRec *st, hipS
 hipError_t launch_router(const RouterArgs &a, int mt, const StepRec *st, hipStream_t s);
 hipError_t launch_gateup(const GUArgs &a, int mt, int mode, const StepRec *st, int max_jobs, hipStream_t s);
 hipError_t launch_down(const DownArgs &a, int mt, int mode, const StepRec *st, hipStream_t s);
-// Routed experts' down projection of 2..16 rows, Q8_0 weights, on the fp32 matrix cores: a
-// workgroup per (32 output rows, down job), then per 32 rows the combine in choice order, then
-// the norm tail (a.tail.nw set) in the last of them
-hipError_t launch_down_fq(const DownArgs &a, int max_jobs, const StepRec *st, hipStream_t s);
 hipError_t launch_norm(const NormTail &t, const StepRec *st, int m, hipStream_t s);
 // hist non-null (m == 1): the pick advances the step record (next token and position) and is
 // appended to hist[step]

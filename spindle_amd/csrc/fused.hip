@@ -21,131 +21,14 @@
 
 #include <type_traits>
 #include "fused.h"
+#include "fx.h"
 #include "decode.h"
 #include "dev.h"
 #include "attn.h"
 #include "decode_dev.h"
+#include "norm_dev.h"
 
 namespace spx {
-
-// ------------------------------------------------------------------ norm tail
-// Rows [b0, b1) of a NormTail by all NW wavefronts of the workgroup. Wave w takes the
-// 256-value blocks w, w+NW, ...; lane j holds values 4j..4j+3 of a block.
-template <int NW>
-__device__ __forceinline__ void norm_rows(const NormTail &t, int b0, int b1) {
-  __shared__ float bsum[NORM_NT];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int dim = t.dim, n4 = dim >> 2, nblk = (n4 + 63) >> 6, nbq = dim >> 8;
-  const rsrc_t ra = rsrc_of(t.add ? t.add : t.x);
-  const float4 *x4 = reinterpret_cast<const float4 *>(t.x);
-  const float4 *w4 = reinterpret_cast<const float4 *>(t.nw);
-  float4 wn[NORM_NT / NW];  // the norm weights, loaded once with the first row's inputs
-#pragma unroll
-  for (int k = 0; k < NORM_NT / NW; k++) {
-    const int f = (wave + NW * k) * 64 + lane;
-    wn[k] = f < n4 ? w4[f] : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  for (int b = b0; b < b1; b++) {
-    float4 r[NORM_NT / NW];
-#pragma unroll
-    for (int k = 0; k < NORM_NT / NW; k++) {
-      const int tb = wave + NW * k, f = tb * 64 + lane;
-      r[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (tb < nblk) {
-        if (f < n4) {
-          float4 v = x4[(int64_t)b * n4 + f];
-          if (t.add) {
-            const f4v a = ld_coh4(ra, (b * n4 + f) * 16);
-            v.x = v.x + t.rscale * a.x; v.y = v.y + t.rscale * a.y; v.z = v.z + t.rscale * a.z; v.w = v.w + t.rscale * a.w;
-          }
-          r[k] = v;
-        }
-        float p = r[k].x * r[k].x;
-        p = fmaf(r[k].y, r[k].y, p);
-        p = fmaf(r[k].z, r[k].z, p);
-        p = fmaf(r[k].w, r[k].w, p);
-        p = wave_sum(p);
-        if (lane == 0) bsum[tb] = p;
-      }
-    }
-    __syncthreads();
-    float S = 0.0f;
-    for (int k = 0; k < nblk; k++) S = S + bsum[k];
-    const float inv = inv_rms(S, (float)dim, t.eps);
-#pragma unroll
-    for (int k = 0; k < NORM_NT / NW; k++) {
-      const int tb = wave + NW * k, f = tb * 64 + lane;
-      if (tb < nblk) {
-        float4 v = r[k];
-        if (f < n4) {
-          if (t.x_out) reinterpret_cast<float4 *>(t.x_out)[(int64_t)b * n4 + f] = v;
-          const float4 w = wn[k];
-          v.x = v.x * inv * w.x; v.y = v.y * inv * w.y; v.z = v.z * inv * w.z; v.w = v.w * inv * w.w;
-          if (t.xn_out) reinterpret_cast<float4 *>(t.xn_out)[(int64_t)b * n4 + f] = v;
-        }
-        if (t.q_out.q) {
-          const float am = q8k_amax(v);
-          const int64_t vb = (int64_t)b * nbq + tb;
-          q8k_block_store(v, am, t.q_out.q + vb * 64, t.q_out.d + vb, reinterpret_cast<int *>(t.q_out.bs + vb * 8));
-        }
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// The same RMSNorm of one row (t.x, no residual add) computed by a consumer's workgroup for
-// itself: the row and its weights loaded (load), then norm_rows's per-block fma chains and
-// wavefront trees, the blocks in order, x * inv * w (finish) into LDS lx (and memory, xn_out).
-// The bits are norm_rows's: a producer's residual epilogue plus this prologue replace its tail.
-template <int NW>
-struct NormRow {
-  float4 r[NORM_NT / NW], w[NORM_NT / NW];
-  __device__ __forceinline__ void load(const NormTail &t) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, n4 = t.dim >> 2, nblk = (n4 + 63) >> 6;
-#pragma unroll
-    for (int k = 0; k < NORM_NT / NW; k++) {
-      const int tb = wave + NW * k, f = tb * 64 + lane;
-      r[k] = w[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (tb < nblk && f < n4) {
-        r[k] = reinterpret_cast<const float4 *>(t.x)[f];
-        w[k] = reinterpret_cast<const float4 *>(t.nw)[f];
-      }
-    }
-  }
-  __device__ __forceinline__ void finish(const NormTail &t, float *lx, float *xn_out) {
-    __shared__ float bsum[NORM_NT];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, n4 = t.dim >> 2, nblk = (n4 + 63) >> 6;
-#pragma unroll
-    for (int k = 0; k < NORM_NT / NW; k++) {
-      const int tb = wave + NW * k;
-      if (tb < nblk) {
-        float p = r[k].x * r[k].x;
-        p = fmaf(r[k].y, r[k].y, p);
-        p = fmaf(r[k].z, r[k].z, p);
-        p = fmaf(r[k].w, r[k].w, p);
-        p = wave_sum(p);
-        if (lane == 0) bsum[tb] = p;
-      }
-    }
-    __syncthreads();
-    float S = 0.0f;
-    for (int k = 0; k < nblk; k++) S = S + bsum[k];
-    const float inv = inv_rms(S, (float)t.dim, t.eps);
-#pragma unroll
-    for (int k = 0; k < NORM_NT / NW; k++) {
-      const int tb = wave + NW * k, f = tb * 64 + lane;
-      if (tb < nblk && f < n4) {
-        float4 v = r[k];
-        const float4 ww = w[k];
-        v.x = v.x * inv * ww.x; v.y = v.y * inv * ww.y; v.z = v.z * inv * ww.z; v.w = v.w * inv * ww.w;
-        reinterpret_cast<float4 *>(lx)[f] = v;
-        if (xn_out) reinterpret_cast<float4 *>(xn_out)[f] = v;
-      }
-    }
-    __syncthreads();
-  }
-};
 
 // ------------------------------------------------------------------ activations in LDS
 __host__ __device__ inline size_t ldsq_dbytes(int mt, int dim) { return ((size_t)mt * (dim / 256) * 4 + 15) & ~(size_t)15; }
@@ -576,12 +459,6 @@ __device__ __forceinline__ void best_flush(const MVArgs &a, unsigned long long (
   }
 }
 
-// A launch output a norm tail will read is stored coherently.
-__device__ __forceinline__ void out_store(float *p, float v, bool coh) {
-  if (coh) st_dev(p, v);
-  else *p = v;
-}
-
 // Segment of workgroup task t and the task's index within it. The index is computed with
 // selects and made wave-uniform, so the segment's fields are read from the kernel arguments
 // directly (no branchy selection between argument sub-objects).
@@ -841,116 +718,6 @@ __global__ __launch_bounds__(MVF1_NW * 64) void k_mv_f1(const MVArgs a, const St
   }
   if (a.best) best_flush<1, MVF1_NW>(a, bestv, 1);
   if (coh && arrive_last(a.tail.counter, gridDim.x)) norm_rows<MVF1_NW>(a.tail, 0, 1);
-}
-
-// One wavefront's part of a Q8_0 16-row tile against up to 16 vectors on the fp32 matrix cores:
-// the batches of FQ_B 32-column blocks with index = kp mod FQ_KP (all of a batch's loads in flight),
-// eight v_mfma_f32_16x16x4f32 per block with A[vector j][kq] = x[j][32b + 8kq + s] and
-// B[kq][row j] = code[32b + 8kq + s] * d (an int8 times an f16 scale: exact in fp32), four
-// accumulator chains (block b in chain b mod 4) summed (0 + 1) + (2 + 3). cp / dp: row
-// lane & 15's codes (+ 8 (lane >> 4)) and scales; xr: vector lane & 15's values (+ 8 (lane >> 4)).
-// r[q]: row lane & 15 of vector 4 (lane >> 4) + q.
-constexpr int FQ_KP = 8;  // parts a tile's blocks are split into (wavefronts per tile)
-constexpr int FQ_B = 4;   // blocks a part loads at once
-__device__ __forceinline__ void fq_part(const uint8_t *cp, const uint16_t *dp, const float *xr, bool vin, int nb, int kp, float (&r)[4]) {
-  f4v acc[4];
-#pragma unroll
-  for (int u = 0; u < 4; u++) acc[u] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int b0 = FQ_B * kp; b0 < nb; b0 += FQ_B * FQ_KP) {
-    uint2 c[FQ_B];
-    uint32_t dh[FQ_B];
-    float4 x0[FQ_B], x1[FQ_B];
-#pragma unroll
-    for (int u = 0; u < FQ_B; u++) {
-      const int b = min(b0 + u, nb - 1);
-      c[u] = *reinterpret_cast<const uint2 *>(cp + (int64_t)b * 32);
-      dh[u] = dp[b];
-      x0[u] = *reinterpret_cast<const float4 *>(xr + (int64_t)b * 32);
-      x1[u] = *reinterpret_cast<const float4 *>(xr + (int64_t)b * 32 + 4);
-    }
-#pragma unroll
-    for (int u = 0; u < FQ_B; u++) {
-      if (b0 + u < nb) {
-        const float d = h2f(dh[u]);
-        const float xs[8] = {x0[u].x, x0[u].y, x0[u].z, x0[u].w, x1[u].x, x1[u].y, x1[u].z, x1[u].w};
-#pragma unroll
-        for (int s2 = 0; s2 < 8; s2++) {
-          const float w = (float)(int8_t)((s2 < 4 ? c[u].x : c[u].y) >> (8 * (s2 & 3))) * d;
-          acc[u & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vin ? xs[s2] : 0.0f, w, acc[u & 3], 0, 0, 0);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < 4; q++) r[q] = (acc[0][q] + acc[1][q]) + (acc[2][q] + acc[3][q]);
-}
-
-// Float matvec of 2..16 vectors on the fp32 matrix cores (Q8_0 weights): TPW 16-row tiles per
-// workgroup, eight wavefronts per tile (tasks stride over the grid as k_mv_f's): wavefront w
-// takes tile w / 8 and part w % 8 of its blocks (fq_part); the parts meet in LDS and are summed
-// in part order. Every product is the per-lane walk's; the sums run in a fixed order of their
-// own, so a row's result does not depend on the pass's other rows, nor on TPW (one tile a
-// workgroup for matrices of few rows: twice the workgroups).
-template <int TPW>
-__global__ __launch_bounds__(512 * TPW) void k_mv_fq(const MVArgs a, const StepRec *st) {
-  constexpr int NWV = 8 * TPW;
-  const int m = st ? st->m : a.m;
-  const bool coh = a.tail.nw != nullptr;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, kq = lane >> 4;
-  const int tile = wave / FQ_KP, kp = wave % FQ_KP;
-  __shared__ unsigned long long sbest[16];
-  __shared__ float part[FQ_KP][TPW][4][64];
-  if (threadIdx.x < 16) sbest[threadIdx.x] = 0;
-  __syncthreads();
-  // segments in units of TPW tiles (a segment's wgs counts 32-row tasks)
-  const int s0 = a.seg[0].wgs * 2 / TPW, s1 = a.nseg > 1 ? a.seg[1].wgs * 2 / TPW : 0, s2 = a.nseg > 2 ? a.seg[2].wgs * 2 / TPW : 0;
-  const int total = s0 + s1 + s2;
-  const bool vin = j < m;
-  for (int t = blockIdx.x; t < total; t += gridDim.x) {
-    const int si = __builtin_amdgcn_readfirstlane(t >= s0 ? (t >= s0 + s1 ? 2 : 1) : 0);
-    const int wg = t - (si > 0 ? s0 : 0) - (si > 1 ? s1 : 0);
-    const Seg &sg = a.seg[si];
-    const int64_t r0 = sg.r0 + ((int64_t)wg * TPW + tile) * 16;
-    float r[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (r0 < sg.r1) {
-      const int64_t grow = (int64_t)sg.expert * sg.w.rows + min(r0 + j, sg.r1 - 1);
-      const int nb = (int)sg.w.nb;
-      fq_part(sg.w.pl.p0 + grow * nb * 32 + 8 * kq, reinterpret_cast<const uint16_t *>(sg.w.pl.p3) + grow * nb,
-              a.x + (int64_t)(vin ? j : 0) * a.ld_x + 8 * kq, vin, nb, kp, r);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) part[kp][tile][q][lane] = r[q];
-    __syncthreads();
-    if (kp == 0 && r0 < sg.r1) {
-      const int64_t row = r0 + j;
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int v = 4 * kq + q;
-        float res = part[0][tile][q][lane];
-#pragma unroll
-        for (int p2 = 1; p2 < FQ_KP; p2++) res = res + part[p2][tile][q][lane];
-        unsigned long long key = 0;
-        if (v < m && row < sg.r1) {
-          out_store(sg.out + (int64_t)v * sg.ld_out + row, res, coh);
-          key = pick_key(res, a.lscale, row);
-        }
-        if (a.best) {  // the 16 rows' best key of vector v, then one atomic per vector
-#pragma unroll
-          for (int o = 1; o < 16; o <<= 1) {
-            const unsigned long long k2 = __shfl_xor(key, o, 64);
-            key = k2 > key ? k2 : key;
-          }
-          if (j == 0 && v < m) atomicMax(&sbest[v], key);
-        }
-      }
-    }
-    __syncthreads();
-  }
-  if (a.best) {
-    __syncthreads();
-    if ((int)threadIdx.x < m) a.best[(int64_t)threadIdx.x * a.nbest + blockIdx.x] = sbest[threadIdx.x];
-  }
-  if (coh && arrive_last(a.tail.counter, gridDim.x)) norm_rows<NWV>(a.tail, 0, m);
 }
 
 // ------------------------------------------------------------------ standalone kernels
@@ -2659,43 +2426,6 @@ __global__ __launch_bounds__(MVF1_NW * 64) void k_gateup_f1(const GUArgs a, cons
   }
 }
 
-// Gate / up + SwiGLU of 2..16 rows on the fp32 matrix cores (Q8_0), dense or one routed expert's
-// users a job (vdiv: the down jobs, whose entries are h indices): 16 rows of h per workgroup of
-// sixteen wavefronts: wavefront w takes part w >> 1 (fq_part) of the gate tile
-// (w even) or the up tile (w odd); the parts meet in LDS (summed in part order) and
-// h = silu(g) * u as k_gateup_f writes it.
-__global__ __launch_bounds__(1024) void k_gateup_fq(const GUArgs a, const StepRec *st) {
-  GUJob J;
-  if (!gu_job(a, st->m, J)) return;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, kq = lane >> 4, mat = wave & 1, kp = wave >> 1;
-  __shared__ float part[FQ_KP][2][4][64];
-  const TensorView &w = mat ? a.up : a.gate;
-  const int nb = (int)w.nb, n_ff = a.n_ff;
-  const int64_t r0 = (int64_t)blockIdx.x * 16, grow = (int64_t)J.expert * w.rows + min(r0 + j, (int64_t)n_ff - 1);
-  const bool vin = j < J.nvec;
-  const int xv = vin ? (J.jv ? (a.vdiv > 1 ? J.jv[j] / a.vdiv : J.jv[j]) : j) : 0;
-  float r[4];
-  fq_part(w.pl.p0 + grow * nb * 32 + 8 * kq, reinterpret_cast<const uint16_t *>(w.pl.p3) + grow * nb, a.x + (int64_t)xv * w.cols + 8 * kq,
-          vin, nb, kp, r);
-#pragma unroll
-  for (int q = 0; q < 4; q++) part[kp][mat][q][lane] = r[q];
-  __syncthreads();
-  if (wave == 0) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int v = 4 * kq + q;
-      const int64_t row = r0 + j;
-      if (v < J.nvec && row < n_ff) {
-        float g = part[0][0][q][lane], u = part[0][1][q][lane];
-#pragma unroll
-        for (int p2 = 1; p2 < FQ_KP; p2++) { g = g + part[p2][0][q][lane]; u = u + part[p2][1][q][lane]; }
-        st_dev(a.h + (int64_t)(J.jo ? J.jo[v] : v) * n_ff + row, g / (1.0f + expf(-g)) * u);
-      }
-    }
-  }
-  if (a.hq.q) gateup_quant_tail(a, J.nvec, J.jo, 16);
-}
-
 // ------------------------------------------------------------------ down + combine
 // One output row per wavefront; row slots take jobs eight at a time; each job's users get
 // y_e[r] in LDS, then out[b][r] = sum over b's chosen slots, in chosen order, of w * y
@@ -2835,64 +2565,6 @@ __global__ __launch_bounds__(256) void k_down_f(const DownArgs a, const StepRec 
   if (coh && arrive_last(a.tail.counter, gridDim.x)) norm_rows<4>(a.tail, 0, m);
 }
 
-// Routed experts' down projection of 2..16 rows on the fp32 matrix cores (Q8_0): workgroup
-// (32 output rows, down job) of sixteen wavefronts as k_mv_fq's (tile w & 1, part w >> 1, the
-// parts summed in part order), the job's users' h rows as the vectors; y of (user, row) goes to
-// yd through the L2. The last of a row block's job workgroups combines its 32 rows for every
-// pass row in choice order (down_combine's arithmetic), and the last row block runs the norm
-// tail.
-__global__ __launch_bounds__(1024) void k_down_fq(const DownArgs a, const StepRec *st) {
-  const int m = st->m, nj = *a.njobs;
-  if ((int)blockIdx.y >= nj) return;
-  const Job &J = a.jobs[blockIdx.y];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, kq = lane >> 4;
-  const int tile = wave & 1, kp = wave >> 1;
-  __shared__ float part[FQ_KP][2][4][64];
-  const int dim = (int)a.w.rows, nb = (int)a.w.nb, n_ff = (int)a.w.cols;
-  const bool coh = a.tail.nw != nullptr;
-  const int nvec = J.nvec;
-  const bool vin = j < nvec;
-  const int xv = vin ? J.vec[j] : 0;
-  const int64_t r0 = (int64_t)blockIdx.x * 32 + tile * 16;
-  float r[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (r0 < dim) {
-    const int64_t grow = (int64_t)J.expert * dim + min(r0 + j, (int64_t)dim - 1);
-    fq_part(a.w.pl.p0 + grow * nb * 32 + 8 * kq, reinterpret_cast<const uint16_t *>(a.w.pl.p3) + grow * nb, a.x + (int64_t)xv * n_ff + 8 * kq,
-            vin, nb, kp, r);
-  }
-#pragma unroll
-  for (int q = 0; q < 4; q++) part[kp][tile][q][lane] = r[q];
-  __syncthreads();
-  const rsrc_t ry = rsrc_of(a.yd);
-  if (kp == 0 && r0 < dim) {
-    const int64_t row = r0 + j;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int v = 4 * kq + q;
-      float res = part[0][tile][q][lane];
-#pragma unroll
-      for (int p2 = 1; p2 < FQ_KP; p2++) res = res + part[p2][tile][q][lane];
-      if (v < nvec && row < dim) st_coh1(ry, (int)(((int64_t)J.out[v] * dim + row) * 4), res);
-    }
-  }
-  int *tc = a.counter + (int64_t)(1 + blockIdx.x) * CNT_STRIDE;
-  if (arrive(tc) != nj - 1) return;
-  if (threadIdx.x == 0) *tc = 0;
-  for (int i = threadIdx.x; i < m * 32; i += 1024) {
-    const int b = i >> 5, row = blockIdx.x * 32 + (i & 31);
-    if (row < dim) {
-      const int nk = a.nkeep[b];
-      float acc = 0.0f;
-      for (int s2 = 0; s2 < nk; s2++) acc = acc + a.weights[b * 32 + s2] * ld_coh1(ry, (int)(((int64_t)(b * a.n_used + s2) * dim + row) * 4));
-      out_store(a.out + (int64_t)b * dim + row, acc, coh);
-    }
-  }
-  if (!coh) return;
-  if (arrive(a.counter) != (int)gridDim.x - 1) return;
-  if (threadIdx.x == 0) *a.counter = 0;
-  norm_rows<16>(a.tail, 0, m);
-}
-
 // ------------------------------------------------------------------ final greedy pick
 // With hist (one-row decode passes replayed back to back): the pick also becomes the next
 // pass's token at the next position, and is appended to hist.
@@ -2955,14 +2627,9 @@ hipError_t launch_mv(const MVArgs &a, int mt, int mode, const StepRec *st, int g
   const bool f1_only = a.pro.nw || a.res_out;  // prologue norm / residual epilogue: k_mv_f1 only
   if (f1_only && (kq_type(dt) || mt != 1 || (a.res_out && a.nseg != 1))) return hipErrorInvalidValue;
   if (!kq_type(dt)) {
-    bool fq = a.fq && a.m >= FQ_MIN_ROWS;
-    for (int i = 0; i < a.nseg; i++) fq = fq && a.seg[i].w.dtype == T_Q8_0;
-    if (fq) {
-      // one tile a workgroup (two tiles: Qwen3-0.6B M = 9 2.82 vs 2.26 ms a pass): twice the
-      // workgroups when the grid covers the tasks, else the same grid (greedy-key slots follow it)
-      hipLaunchKernelGGL(k_mv_fq<1>, dim3(!a.best && grid == mv_total(a) ? 2 * grid : grid), dim3(512), 0, s, a, st);
-      return hipGetLastError();
-    }
+    bool fx = a.fx && a.m >= FX_MIN_ROWS;
+    for (int i = 0; i < a.nseg; i++) fx = fx && fx_type(a.seg[i].w.dtype) && a.seg[i].w.dtype == a.seg[0].w.dtype && a.seg[i].w.cols == a.seg[0].w.cols;
+    if (fx) return launch_fx_mv(a, a.m, st, a.best ? grid : 0, s);
     if (mt == 1) {  // one row over Q8_0 segments: k_mv_f1 (the only kernel that takes pro / res_out)
       bool q8 = true;
       for (int i = 0; i < a.nseg; i++) q8 = q8 && a.seg[i].w.dtype == T_Q8_0 && a.seg[i].w.cols == a.seg[0].w.cols;
@@ -3187,8 +2854,6 @@ static hipError_t launch_gu_t(const GUArgs &a, int mode, const StepRec *st, int 
     const size_t sm = (MT <= 2 ? ldsq_bytes(MT, dim) : 0) + (size_t)4 * 8 * nb * tile_bpb();
     SPX_LDS((k_gateup_kq<T, MT>), sm);
     hipLaunchKernelGGL((k_gateup_kq<T, MT>), dim3((unsigned)((a.n_ff + 15) / 16), jobs), dim3(256), sm, s, a, st);
-  } else if (T == T_Q8_0 && MT >= 4 && a.fq) {
-    hipLaunchKernelGGL(k_gateup_fq, dim3((unsigned)((a.n_ff + 15) / 16), jobs), dim3(1024), 0, s, a, st);
   } else if (T == T_Q8_0 && MT == 1 && !a.hq.q && a.gate.nb <= 128 && gu_f1_on()) {
     // one row: k_gateup_f1, RW rows a wavefront (fewer for more workgroups, up to 2 a CU)
     const int blocks = (a.n_ff + 15) / 16, nb = (int)a.gate.nb;
@@ -3287,12 +2952,6 @@ hipError_t launch_down(const DownArgs &a, int mt, int mode, const StepRec *st, h
   case T_Q5K: return launch_down_dt<T_Q5K>(a, mt, mode, st, s);
   default: return hipErrorInvalidValue;
   }
-}
-
-hipError_t launch_down_fq(const DownArgs &a, int max_jobs, const StepRec *st, hipStream_t s) {
-  if (a.w.dtype != T_Q8_0 || !a.yd || !a.counter || max_jobs < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_down_fq, dim3((unsigned)((a.w.rows + 31) / 32), (unsigned)max_jobs), dim3(1024), 0, s, a, st);
-  return hipGetLastError();
 }
 
 hipError_t launch_embed(const TensorView &e, const StepRec *st, float escale, const NormTail &t, int m, hipStream_t s) {

@@ -1,0 +1,108 @@
+"""Float-activation products on the bf16 matrix cores (fx.hip): Q8_0 matvecs of 2..16 rows against
+float64 at the edges of their tiles and parts, non-finite activations, and prefill passes of float
+models (17..128 rows) against the same rows in passes of at most 16, bitwise."""
+import numpy as np
+import pytest
+
+from spindle_amd import model as M
+from oracle import ffi
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from spindle_amd import ops
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    c = ops.Context(0)
+    yield c
+    c.close()
+
+
+def _q8_0(rng, cols, rows):
+    raw = rng.integers(0, 256, M.row_bytes(M.Q8_0, cols) * rows, dtype=np.uint8)
+    raw.reshape(-1, 34)[:, 0:2] = np.float16(rng.uniform(0.001, 0.05, raw.size // 34)).view(np.uint8).reshape(-1, 2)
+    return raw, ffi.dequant(M.Q8_0, raw, rows, cols).astype(np.float64).reshape(rows, cols)
+
+
+# widths of 1 and 2 blocks (empty parts), odd part lengths, 8 and 16 parts; row counts around a
+# tile of 16, a workgroup's 32 rows and the four-tile shape of large matrices
+@pytest.mark.parametrize("cols,rows", [(32, 17), (64, 1), (96, 65), (576, 33), (992, 16), (1024, 200), (1056, 15), (2016, 64), (2048, 31),
+                                       (3072, 48), (4096, 95), (576, 33000), (2080, 33001)])
+def test_q8_0_edges(ctx, cols, rows):
+    """Within the rounding of a row's fp32 additions: at most 96 in a block (32 products in three
+    parts, exact), one a block and one a part, each off by at most one unit in the last place
+    (2^-23) of a partial sum that sum |w x| bounds; a vector's bits the same in any batch."""
+    from spindle_amd import ops
+    rng = np.random.default_rng(cols + rows)
+    raw, wd = _q8_0(rng, cols, rows)
+    w = ops.Tensor(ctx, M.Q8_0, cols, rows, raw)
+    x = (rng.standard_normal((16, cols)) * np.exp(rng.uniform(-8, 8, (16, 1)))).astype(np.float32)
+    full = ops.matvec(ctx, w, torch.from_numpy(x).cuda()).cpu().numpy()
+    want, scale = x.astype(np.float64) @ wd.T, np.abs(x.astype(np.float64)) @ np.abs(wd).T
+    assert np.all(np.abs(full - want) <= (96 + cols // 32 + 16) * 2.0 ** -23 * scale)
+    for m, v0 in ((2, 3), (9, 5), (15, 0)):
+        part = ops.matvec(ctx, w, torch.from_numpy(x[v0:v0 + m]).cuda()).cpu().numpy()
+        assert np.array_equal(part.view(np.uint32), full[v0:v0 + m].view(np.uint32)), m
+    w.free()
+
+
+def test_q8_0_non_finite(ctx):
+    """An infinite activation gives what IEEE products and sums give (an infinity, or a NaN where
+    its code is 0), a NaN a NaN, and the batch's other vectors keep their bits."""
+    from spindle_amd import ops
+    rng = np.random.default_rng(5)
+    raw, wd = _q8_0(rng, 1024, 64)
+    w = ops.Tensor(ctx, M.Q8_0, 1024, 64, raw)
+    x = rng.standard_normal((9, 1024)).astype(np.float32)
+    clean = ops.matvec(ctx, w, torch.from_numpy(x).cuda()).cpu().numpy()
+    x[2, 77], x[4, 500], x[7, 1023] = np.inf, np.nan, -np.inf
+    got = ops.matvec(ctx, w, torch.from_numpy(x).cuda()).cpu().numpy()
+    for v in (0, 1, 3, 5, 6, 8):
+        assert np.array_equal(got[v].view(np.uint32), clean[v].view(np.uint32)), v
+    with np.errstate(invalid="ignore"):
+        for v, c in ((2, 77), (7, 1023)):
+            want = x[v, c].astype(np.float64) * wd[:, c]
+            assert np.array_equal(got[v], want.astype(np.float32), equal_nan=True), v
+    assert np.isnan(got[4]).all()
+    w.free()
+
+
+# dense Q8_0 (attention with q/k norms), dense Q5_0 with a Q6_K ffn_down, Q8_0 experts, Q5_0 experts
+CASES = {
+    "qwen3": M.TINY["tiny-qwen3"].replace(sigma=0.05, max_seq=320),
+    "llama": M.TINY["tiny-llama"].replace(sigma=0.05, max_seq=320),
+    "granite": M.TINY["tiny-granite"].replace(sigma=0.05, max_seq=320),
+    "granite-q5_0": M.TINY["tiny-granite"].replace(sigma=0.05, max_seq=320, t_gate=M.Q5_0, t_up=M.Q5_0, t_down=M.Q5_0, moe_prune=0.3),
+    "wide": M.TINY["tiny-qwen3"].replace(sigma=0.03, max_seq=320, dim=1024, n_heads=16, n_kv_heads=8, head_dim=128, n_ff=2048),
+}
+
+
+@pytest.mark.parametrize("case", list(CASES))
+def test_float_prefill_equals_16_row_passes(ctx, case):
+    cfg = CASES[case]
+    w = M.synth_model(cfg, seed=71)
+    a, b = M.Engine(ctx, cfg, w), M.Engine(ctx, cfg, w)
+    ids, pos = np.random.default_rng(72).integers(0, cfg.vocab, 320), 0
+    for m in (17, 128, 33, 2, 100, 32):
+        am0, h0, l0 = a.forward(ids[pos:pos + m], pos, hidden=True, logits=True)
+        for s in range(0, m, 16):
+            n = min(16, m - s) if m - s != 17 else 15  # (no last pass of one row: those sum in the one-row order)
+            if m - s == 1:
+                break
+            am1, h1, l1 = b.forward(ids[pos + s:pos + s + n], pos + s, hidden=True, logits=True)
+            assert np.array_equal(h0[s:s + n].view(np.uint32), h1.view(np.uint32)), (case, m, s, "hidden")
+            assert np.array_equal(l0[s:s + n].view(np.uint32), l1.view(np.uint32)) and np.array_equal(am0[s:s + n], am1), (case, m, s)
+        if m % 16 == 1:  # the odd row through a two-row pass with its predecessor
+            am1, h1, l1 = b.forward(ids[pos + m - 2:pos + m], pos + m - 2, hidden=True, logits=True)
+            assert np.array_equal(h0[m - 2:].view(np.uint32), h1.view(np.uint32)) and np.array_equal(l0[m - 2:].view(np.uint32), l1.view(np.uint32))
+        pos += m
+    ka, va = a.kv_cache()
+    kb, vb = b.kv_cache()
+    assert np.array_equal(ka, kb) and np.array_equal(va, vb)
+    if cfg.moe:
+        assert all(0 < n <= cfg.n_expert for n in a.last_experts())
+    a.close()
+    b.close()
