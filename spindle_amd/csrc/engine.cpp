@@ -99,6 +99,10 @@ struct spx_engine {
   // passes of 17..128 rows of a float model on the fused path's matrix-core kernels (fx.hip; attention
   // on the multi-tile kernels): every row the bits of its pass of 2..16 rows
   bool fx_pf = false;
+  // no K-quant matrix: Q5_0 passes of more than one row take the matrix cores too. (A model that
+  // re-quantizes some activations to Q8_K keeps the per-lane order for its Q5_0 matrices: a last-bit
+  // change before them can move a Q8_K code by a step, ~2e-3 of SmolLM2's logits.)
+  bool all_float = false;
   // one-row passes with their layers as cooperative launches (persist.hip), where the model
   // fits its tiles; off by default: measured slower than the pipeline (SPX_PERSIST=1 or
   // spx_engine_set_persist turns it on)
@@ -268,7 +272,7 @@ int mv_run(spx_engine *E, MVArgs &a, int m, int mode, int grid_cap = 0) {
   if (grid_cap > 0 && grid > grid_cap) grid = grid_cap;
   a.m = m;
   a.nbest = grid;
-  a.fx = E->mq ? 1 : 0;
+  a.fx = !E->mq ? 0 : E->all_float ? 2 : 1;
   SPX_HIP(launch_mv(a, m, mode, E->st_dev, grid, E->ctx->stream));
   return 0;
 }
@@ -314,26 +318,15 @@ int mv_res(spx_engine *E, const spx_tensor *w, const float *x, int64_t ld_x, flo
   return mv_run(E, a, 1, 0);
 }
 
-// Integer matvec of m <= 16 rows of Q8_K activations, no step record (a slice of a longer pass).
-int mv_rows(spx_engine *E, const spx_tensor *w, int m, Q8KP y, float *out, int64_t ld_out) {
-  const int mode = mode_of(E, w, m);
-  MVArgs a{};
-  a.G = 8;
-  a.R = 1;
-  rp_shape(w->v.nb, a.G, a.R);
-  a.seg[0] = seg_of(w, out, ld_out, m, mode, a.R);
-  a.nseg = 1;
-  a.y = y;
-  a.lscale = E->c.logit_scale;
-  a.m = m;
-  SPX_HIP(launch_mv(a, m, mode, nullptr, a.seg[0].wgs, E->ctx->stream));
-  return 0;
+// A matrix whose passes of two rows and more run on the bf16 matrix cores (fx.hip).
+bool fx_on(const spx_engine *E, const spx_tensor *t) {
+  return E->mq && (t->v.dtype == T_Q8_0 || (t->v.dtype == T_Q5_0 && E->all_float));
 }
 
 // A MoE layer whose passes of 2..128 rows run on the bf16 matrix cores: float experts, and a row
 // width that the multi-row router and norm take.
 bool fx_moe(const spx_engine *E, const LayerW &ly) {
-  return ly.moe && fx_type(ly.gate->v.dtype) && fx_type(ly.up->v.dtype) && fx_type(ly.down->v.dtype) && ly.router->v.dtype == T_F32 &&
+  return ly.moe && fx_on(E, ly.gate) && fx_on(E, ly.up) && fx_on(E, ly.down) && ly.router->v.dtype == T_F32 &&
          E->c.dim % 256 == 0 && E->c.dim <= 256 * DEC_MAXNB;
 }
 
@@ -448,7 +441,7 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
     const int gmode = m <= 2 ? mode_of(E, ly.gate, m) : 0;  // grouped experts: row-parallel at decode, tiles for verify
     if (ly.moe) {  // moe_forward / moe_forward_batch (:925-1392)
       const int nu = c.n_expert_used, ne = c.n_expert;
-      if (fx_moe(E, ly) && E->mq && m >= FX_MIN_ROWS) {
+      if (fx_moe(E, ly) && m >= FX_MIN_ROWS) {
         // float experts, 2..128 rows: the router's rows, the routing and a job list of at most 16
         // users a job (the K-quant prefill passes' kernels), the experts on the bf16 matrix cores,
         // then the combine in choice order and the next norm in one launch
@@ -519,7 +512,7 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
         ProfScope ps(E, PC_GATEUP, wbytes(ly.gate) + wbytes(ly.up));
         GUArgs ga{};
         ga.gate = ly.gate->v; ga.up = ly.up->v; ga.y = E->xq2; ga.x = E->xn2; ga.h = E->h; ga.counter = E->gu_cnt; ga.n_ff = nff;
-        if (E->mq && m >= FX_MIN_ROWS && fx_type(ly.gate->v.dtype) && fx_type(ly.up->v.dtype)) {
+        if (m >= FX_MIN_ROWS && fx_on(E, ly.gate) && fx_on(E, ly.up)) {
           SPX_HIP(launch_fx_gateup(ga, m, E->st_dev, 1, s));
           if (d_int) SPX_HIP(launch_q8kp_quantize(E->h, nff, nff, m, E->hq, s));
         } else {
@@ -532,10 +525,6 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
         ProfScope ps(E, PC_DOWN, wbytes(ly.down));
         if (pro) {
           if (int r = mv_res(E, ly.down, E->h, nff, E->ffn, E->xB, E->xA)) return r;
-        } else if (d_int && m > MAX_M) {  // a K-quant down of a float model's prefill pass: 16 rows a launch
-          for (int r0 = 0; r0 < m; r0 += MAX_M)
-            if (int r = mv_rows(E, ly.down, std::min(MAX_M, m - r0), q8kp_row(E->hq, r0, nff), E->ffn + (int64_t)r0 * dim, dim)) return r;
-          SPX_HIP(launch_norm(tn, E->st_dev, m, s));
         } else {
           if (int r = mv_one(E, ly.down, m, E->h, nff, E->hq, E->ffn, dim, &tn, tails, PC_NORM)) return r;
         }
@@ -571,7 +560,7 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
       SPX_HIP(launch_mv(a, 1, mode, nullptr, grid, s));
       E->nbest = grid;
     } else {
-      const bool fx = E->mq && m >= FX_MIN_ROWS && fx_type(E->lm_head->v.dtype);
+      const bool fx = m >= FX_MIN_ROWS && fx_on(E, E->lm_head);
       if (int r = mv_run(E, a, m, mode, fx ? fx_mv_wgs(E->lm_head->v, m) : mode == 0 ? E->lm_grid : 0)) return r;
       E->nbest = a.nbest;
     }
@@ -856,7 +845,7 @@ int enqueue_pass_m(spx_engine *E, int m) {
       {
         ProfScope ps(E, PC_DOWN, wbytes(ly.down), l, true);
         DecDownMArgs da{ly.down->v, E->h, E->jobs, ly.njobs, E->yd, big ? maxj : std::min(m * nu, c.n_expert)};
-        SPX_HIP(mqk(spx_engine::MQ_DOWN) ? launch_dec_down_mq(da, s) : launch_dec_down_m(da, s));
+        SPX_HIP(mqk(spx_engine::MQ_DOWN) ? launch_kp_down_mq(da, s) : launch_dec_down_m(da, s));
         combine = true;  // + weighted combine + residual in the next norm (xB -> xA)
       }
     } else {  // ffn_forward_multi (:616-646)
@@ -1215,11 +1204,14 @@ int spx_engine_prepare(spx_engine *E) {
     E->fpro = fp;
   }
   {
-    bool ok = E->att_mt_min > 0 && c.n_heads / c.n_kv_heads >= 2 && fx_type(E->lm_head->v.dtype);
+    E->all_float = !is_kq(E->lm_head);
+    for (auto &ly : E->L)
+      for (const spx_tensor *t : {ly.wq, ly.wk, ly.wv, ly.wo, ly.gate, ly.up, ly.down}) E->all_float = E->all_float && !is_kq(t);
+    bool ok = E->all_float && E->att_mt_min > 0 && c.n_heads / c.n_kv_heads >= 2 && fx_type(E->lm_head->v.dtype);
     for (auto &ly : E->L) {
-      for (const spx_tensor *t : {ly.wq, ly.wk, ly.wv, ly.wo, ly.gate, ly.up}) ok = ok && fx_type(t->v.dtype);
+      for (const spx_tensor *t : {ly.wq, ly.wk, ly.wv, ly.wo, ly.gate, ly.up, ly.down}) ok = ok && fx_type(t->v.dtype);
       ok = ok && ly.wk->v.dtype == ly.wq->v.dtype && ly.wv->v.dtype == ly.wq->v.dtype;
-      ok = ok && (ly.moe ? fx_moe(E, ly) : fx_type(ly.down->v.dtype) || is_kq(ly.down));
+      ok = ok && (!ly.moe || (ly.router->v.dtype == T_F32 && c.dim % 256 == 0 && c.dim <= 256 * DEC_MAXNB));
       ok = ok && (!ly.q_bias || (c.n_heads / c.n_kv_heads) * c.head_dim <= 2048);
     }
     E->fx_pf = ok;

@@ -69,8 +69,8 @@ struct MVArgs {
   int nbest;
   float lscale;
   NormTail tail;
-  // float path, FX_MIN_ROWS rows and more: Q8_0 or Q5_0 segments of one format and width on the bf16 matrix
-  // cores (launch_fx_mv) instead of the per-lane walk (the same products, summed in another order)
+  // float path, FX_MIN_ROWS rows and more: Q8_0 (2: and Q5_0) segments of one format and width on the
+  // bf16 matrix cores (launch_fx_mv) instead of the per-lane walk (the same products, summed in another order)
   int fx;
   // one-row Q8_0 passes (k_mv_f1 only): pro.nw set: the input row is pro.x, normalised by every
   // workgroup as norm_rows would (workgroup 0 also writes pro.xn_out); res_out set: residual

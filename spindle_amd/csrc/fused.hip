@@ -2628,7 +2628,7 @@ hipError_t launch_mv(const MVArgs &a, int mt, int mode, const StepRec *st, int g
   if (f1_only && (kq_type(dt) || mt != 1 || (a.res_out && a.nseg != 1))) return hipErrorInvalidValue;
   if (!kq_type(dt)) {
     bool fx = a.fx && a.m >= FX_MIN_ROWS;
-    for (int i = 0; i < a.nseg; i++) fx = fx && fx_type(a.seg[i].w.dtype) && a.seg[i].w.dtype == a.seg[0].w.dtype && a.seg[i].w.cols == a.seg[0].w.cols;
+    for (int i = 0; i < a.nseg; i++) fx = fx && (a.seg[i].w.dtype == T_Q8_0 || (a.fx == 2 && a.seg[i].w.dtype == T_Q5_0)) && a.seg[i].w.dtype == a.seg[0].w.dtype && a.seg[i].w.cols == a.seg[0].w.cols;
     if (fx) return launch_fx_mv(a, a.m, st, a.best ? grid : 0, s);
     if (mt == 1) {  // one row over Q8_0 segments: k_mv_f1 (the only kernel that takes pro / res_out)
       bool q8 = true;
