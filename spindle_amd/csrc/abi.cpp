@@ -620,7 +620,7 @@ extern "C" int spx_moe(spx_ctx *ctx, const spx_tensor *gate, const spx_tensor *u
 // The routed experts with the routing in device memory: nothing waits on the host. The routing
 // goes into the pipeline's layout (kp_moe_in), the job list is built on the device (kp_jobs: at
 // most 16 users a job), x is quantized to Q8_K, and the prefill pass's grouped kernels run on
-// the int8 matrix cores (kp_gateup_mq, kd_down_mq: the reference's per-lane integer dots and fp32
+// the int8 matrix cores (kp_gateup_mq, kp_down_mq or kd_down_m: the reference's per-lane integer dots and fp32
 // chains); kp_moe_combine sums each row's choices in order.
 extern "C" int spx_moe_dev(spx_ctx *ctx, const spx_tensor *gate, const spx_tensor *up, const spx_tensor *down, const float *x,
                            int64_t ld_x, int m, int k, const int32_t *chosen, const float *weights, float *y, int64_t ld_y) {
@@ -661,7 +661,14 @@ extern "C" int spx_moe_dev(spx_ctx *ctx, const spx_tensor *gate, const spx_tenso
   ga.gate = gate->v; ga.up = up->v; ga.y = yq; ga.h = h; ga.n_ff = (int)n_ff; ga.m = m;
   SPX_HIP(launch_kp_gateup_mq(ga, jobs, njobs, max_jobs, s));
   DecDownMArgs da{down->v, h, jobs, njobs, yd, max_jobs};
-  SPX_HIP(launch_dec_down_mq(da, s));
+  // below 12 rows the lane kernel (as the passes choose; 128 experts, 8 a row, us a call with it / on
+  // the matrix cores: 1 row 43.5 / 46.7, 4 rows 64.0 / 71.5, 9 rows 87.5 / 93.5, 16 rows 114.5 / 113.0)
+  if (m < 12) {
+    da.max_jobs = std::min(ne, nv);  // (at most 16 rows: one job an expert)
+    SPX_HIP(launch_dec_down_m(da, s));
+  } else {
+    SPX_HIP(launch_kp_down_mq(da, s));
+  }
   SPX_HIP(launch_kp_moe_combine(yd, w32, nkeep, m, k, (int)dim, y, ld_y, s));
   return 0;
 }

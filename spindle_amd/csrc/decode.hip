@@ -1359,30 +1359,6 @@ __device__ __forceinline__ void q6_wsplit(uint32_t q, uint32_t s16, uint32_t &hi
   hi = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, ho), __builtin_bit_cast(uint32_t, he), 0x06020400u);
 }
 
-// 4 x 4 transpose over the wavefront's four 16-lane rows: row g of r[c] holds M[g][c] on entry
-// and M[c][g] on return (v_permlane32_swap: rows 2, 3 of the first operand <-> rows 0, 1 of the
-// second; v_permlane16_swap: rows 1, 3 of the first <-> rows 0, 2 of the second).
-__device__ __forceinline__ void mw_t4(uint32_t (&r)[4]) {
-  const auto p = __builtin_amdgcn_permlane32_swap(r[0], r[2], false, false);
-  const auto q = __builtin_amdgcn_permlane32_swap(r[1], r[3], false, false);
-  const auto u = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
-  const auto v = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
-  r[0] = u[0];
-  r[1] = u[1];
-  r[2] = v[0];
-  r[3] = v[1];
-}
-// The same for rows (a, a, b, b): three swaps.
-__device__ __forceinline__ void mw_t4d(uint32_t a, uint32_t b, uint32_t (&r)[4]) {
-  const auto p = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-  const auto u = __builtin_amdgcn_permlane16_swap(p[0], p[0], false, false);
-  const auto v = __builtin_amdgcn_permlane16_swap(p[1], p[1], false, false);
-  r[0] = u[0];
-  r[1] = u[1];
-  r[2] = v[0];
-  r[3] = v[1];
-}
-
 // The LDS image of a tile's vectors (at most 16): codes lq (vector v's block b at dword
 // v mw_vs + 64 b; eight pad dwords a vector put the sixteen vectors' reads of one class word in
 // different banks), block scales ld [v nb + b], the correction words lc (vector v's block b at
@@ -1438,57 +1414,6 @@ __device__ __forceinline__ void mq_corr_stage(int m, int nb, const SPX_L int2 *l
   }
 }
 
-// One block of a tile as lane c16 + 16 k4 loads it, from matrix row c16's bytes in 16-byte
-// pieces (the row's four lanes read its 128 code bytes as two 64-byte halves): Q4_K c[e] = code
-// dwords 16 e + 4 k4 .. + 3; Q6_K c[e] = ql dwords 16 e + 4 k4 .. + 3 and h[e] = qh dwords
-// 8 e + 2 k4, + 1; s = the row's scale line (Q4_K: 8 scales, 8 mins; Q6_K: 16 int8 scales);
-// d = Q4_K d | dmin << 16, Q6_K d.
-struct MwRaw {
-  uint4 c[2], s;
-  uint2 h[2];
-  uint32_t d;
-};
-// A tile's planes at its first row (wave-uniform: scalar registers) and this lane's row as a
-// block offset from there, so the loads take a scalar base and a 32-bit lane offset.
-struct MwSrc {
-  const uint8_t *p0, *p1, *p2, *p3;
-  int rb;  // (row c16, clamped to the tile) x nb
-  int dt;
-};
-__device__ __forceinline__ int64_t mw_uni64(int64_t v) {
-  const uint64_t u = (uint64_t)v;
-  return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)u));
-}
-__device__ __forceinline__ MwSrc mw_src(const Planes &pl, int dt, int64_t row0, int nrows, int nb) {
-  const int64_t r0 = mw_uni64(row0) * nb;
-  MwSrc s;
-  s.dt = __builtin_amdgcn_readfirstlane(dt);
-  s.p0 = pl.p0 + r0 * 128;
-  s.p2 = pl.p2 + r0 * 16;
-  if (s.dt == T_Q4K) {
-    s.p1 = pl.p1 + r0 * 16;
-    s.p3 = s.p1;
-  } else {
-    s.p1 = pl.p1 + r0 * 64;
-    s.p3 = pl.p3 + r0 * 2;
-  }
-  s.rb = min((int)(threadIdx.x & 15), __builtin_amdgcn_readfirstlane(nrows) - 1) * nb;
-  return s;
-}
-template <int TT>  // TT: the tile's format when fixed for the launch, 0: s.dt at run time
-__device__ __forceinline__ void mw_fetch(MwRaw &r, const MwSrc &s, int b) {
-  const uint32_t k4 = (threadIdx.x & 63) >> 4, ob = (uint32_t)(s.rb + b);
-  r.c[0] = gld<uint4>(s.p0 + (ob * 128u + 16u * k4));
-  r.c[1] = gld<uint4>(s.p0 + (ob * 128u + 16u * k4 + 64u));
-  r.s = gld<uint4>(s.p2 + ob * 16u);
-  if (TT == T_Q4K || (TT == 0 && s.dt == T_Q4K)) {
-    r.d = gld<uint32_t>(s.p1 + ob * 16u);
-  } else {
-    r.h[0] = gld<uint2>(s.p1 + (ob * 64u + 8u * k4));
-    r.h[1] = gld<uint2>(s.p1 + (ob * 64u + 8u * k4 + 32u));
-    r.d = gld<uint16_t>(s.p3 + ob * 2u);
-  }
-}
 // The tile's LDS operands for this lane: A (vector lane & 15's class words, dword 2 k4 of each),
 // its correction words, the block scales of vectors 4 (lane >> 4) + t. Rows of A past the
 // vectors read vector 0's: a row of A reaches only the same row of D, never stored.
@@ -1535,112 +1460,6 @@ struct MwProd {
   float dx[4], cf[4];
 };
 
-// Q6_K classes 4 E .. 4 E + 3 of a block (those of part C) from its ql words c (dwords
-// 16 E + 4 k4 ..) and qh words h (dwords 8 E + 2 k4, + 1); sw = the lane's four int8 scales
-// (groups 4 k4 .. 4 k4 + 3). Each 6-bit code c times its group's scale sc, W = c sc = 128 hi +
-// lo (q6_wsplit: lo 0..127, hi -63..62, both int8): P = 128 D(hi) + D(lo), accumulated on the
-// matrix core (exact in int32, the same integer as the digit products of c and sc).
-template <int E, int WPT, int C>
-__device__ __forceinline__ void mw_q6_half(const uint4 &c, const uint2 &h, uint32_t sw, const SPX_L uint32_t *py, mq_v4i (&P)[8 / WPT]) {
-  const int sh = 4 * ((threadIdx.x >> 4) & 1);
-  uint32_t q0[4], q1[4], qh[4];
-  mw_t4d(c.x, c.z, q0);
-  mw_t4d(c.y, c.w, q1);
-  mw_t4d(h.x, h.y, qh);
-  const uint32_t s0 = (uint32_t)(uint16_t)(int16_t)(int8_t)(sw >> (8 * E)), s1 = (uint32_t)(uint16_t)(int16_t)(int8_t)(sw >> (16 + 8 * E));
-  uint32_t wh0[4], wl0[4], wh1[4], wl1[4];
-  uint2 y[4];
-#pragma unroll
-  for (int a = 0; a < 4; a++) {
-    if (mw_slot<WPT, C>(4 * E + a) < 0) continue;
-    const uint32_t c0 = ((q0[a] >> sh) & 0x0F0F0F0Fu) | (((qh[a] >> sh) & 0x03030303u) << 4);
-    const uint32_t c1 = ((q1[a] >> sh) & 0x0F0F0F0Fu) | (((qh[a] >> (sh + 2)) & 0x03030303u) << 4);
-    q6_wsplit(c0, s0, wh0[a], wl0[a]);
-    q6_wsplit(c1, s1, wh1[a], wl1[a]);
-    y[a] = lld<uint2>(py + 8 * (4 * E + a));
-  }
-  // the classes' contractions interleaved, one dependent step at a time
-#pragma unroll
-  for (int a = 0; a < 4; a++) {
-    const int j = mw_slot<WPT, C>(4 * E + a);
-    if (j >= 0) P[j] = mq_mfma(y[a].x, y[a].y, wh0[a], wh1[a]) * 128;
-  }
-#pragma unroll
-  for (int a = 0; a < 4; a++) {
-    const int j = mw_slot<WPT, C>(4 * E + a);
-    if (j >= 0) P[j] = mq_mfma_c(y[a].x, y[a].y, wl0[a], wl1[a], P[j]);
-  }
-}
-
-// Block b of a tile, part C: its integers (mw_prod). The class words are regrouped across the
-// four 16-lane rows (mw_t4): lane row k4 then holds, for class l, the code word of sub-blocks
-// 2 k4, 2 k4 + 1 (Q4_K dword 4 l + k4; Q6_K ql dwords 4 l + 2 (k4 >> 1) + 0, 1 and qh dword
-// 2 l + (k4 >> 1)).
-template <int T, int WPT, int C>
-__device__ __forceinline__ void mw_prod(const MwRaw &r, const MwDst &d, int b, MwProd<WPT> &o) {
-  const int k4 = (threadIdx.x & 63) >> 4;
-  const SPX_L uint32_t *py = d.py + b * 64, *pw = d.pw + b * MQ_CW;
-  float xd[4];
-  const float dd = h2f(r.d);
-#pragma unroll
-  for (int t = 0; t < 4; t++) {
-    xd[t] = d.px[t][b];
-    o.dx[t] = dd * xd[t];
-  }
-  if constexpr (T == T_Q4K) {
-    uint32_t w[2][4] = {{r.c[0].x, r.c[0].y, r.c[0].z, r.c[0].w}, {r.c[1].x, r.c[1].y, r.c[1].z, r.c[1].w}};
-    mw_t4(w[0]);
-    mw_t4(w[1]);
-    const uint32_t sw = k4 < 2 ? r.s.x : r.s.y, sp = (k4 & 1) ? sw >> 16 : sw;
-    const uint32_t s0 = sp & 0xFFu, s1 = (sp >> 8) & 0xFFu;
-    const uint32_t lo0 = s0 & 7u, hi0 = s0 >> 3, lo1 = s1 & 7u, hi1 = s1 >> 3;
-    // P = D(q sl) + 8 D(q sh), the digits accumulated on the matrix core (exact in int32); the
-    // classes interleaved four at a time
-    constexpr int CG = 8 / WPT < 4 ? 8 / WPT : 4;
-#pragma unroll
-    for (int j0 = 0; j0 < 8 / WPT; j0 += CG) {
-      uint32_t c0[CG], c1[CG];
-      uint2 y[CG];
-#pragma unroll
-      for (int q = 0; q < CG; q++) {
-        const int l = mw_cls<WPT, C>(j0 + q);
-        const uint32_t wl = w[l >> 2][l & 3];
-        c0[q] = wl & 0x0F0F0F0Fu;
-        c1[q] = (wl >> 4) & 0x0F0F0F0Fu;
-        y[q] = lld<uint2>(py + 8 * l);
-      }
-#pragma unroll
-      for (int q = 0; q < CG; q++) o.P[j0 + q] = mq_mfma(y[q].x, y[q].y, mx_pmul(c0[q], hi0), mx_pmul(c1[q], hi1)) * 8;
-#pragma unroll
-      for (int q = 0; q < CG; q++) o.P[j0 + q] = mq_mfma_c(y[q].x, y[q].y, mx_pmul(c0[q], lo0), mx_pmul(c1[q], lo1), o.P[j0 + q]);
-    }
-    if (C == 0) {
-      // C = sum_s mn_s (bsum_2s + bsum_2s+1): K 0-7 the sums' lo, 8-15 their hi, against the mins
-      const uint2 cw = lld<uint2>(pw + 8 + 2 * (k4 & 1));
-      const uint32_t a0 = k4 < 2 ? cw.x : 0u, a1 = k4 < 2 ? cw.y : 0u;
-      o.Cc = mq_mfma_c(a0, a1, r.s.z, r.s.w, mq_mfma(k4 == 1 ? a0 : 0u, k4 == 1 ? a1 : 0u, r.s.z, r.s.w) * 63);
-      const float dm = h2f(r.d >> 16);
-#pragma unroll
-      for (int t = 0; t < 4; t++) o.cf[t] = dm * xd[t];
-    }
-  } else {
-    // the lane's scale dword k4, by shifts of the line (a select among the raw fields would have
-    // the compiler index the block buffer in scratch memory)
-    const uint64_t s01 = ((uint64_t)r.s.y << 32) | r.s.x, s23 = ((uint64_t)r.s.w << 32) | r.s.z;
-    const uint32_t sw = (uint32_t)(((k4 & 2) ? s23 : s01) >> (32 * (k4 & 1)));
-    mw_q6_half<0, WPT, C>(r.c[0], r.h[0], sw, py, o.P);
-    mw_q6_half<1, WPT, C>(r.c[1], r.h[1], sw, py, o.P);
-    if (C == 0) {
-      // C = sum_g sc_g bsum_g: K 0-15 the bsums' lo, 16-31 their hi, against the scales
-      const uint2 cw = lld<uint2>(pw + 2 * k4);
-      const uint32_t b0 = (k4 & 1) ? r.s.z : r.s.x, b1 = (k4 & 1) ? r.s.w : r.s.y;
-      const bool lo = k4 < 2;
-      o.Cc = mq_mfma_c(cw.x, cw.y, b0, b1, mq_mfma(lo ? 0u : cw.x, lo ? 0u : cw.y, b0, b1) * 63) * 32;
-#pragma unroll
-      for (int t = 0; t < 4; t++) o.cf[t] = dd * xd[t];
-    }
-  }
-}
 // The chains advance by one block: acc_l = fma(d xd, float(P_l), acc_l) and, part 0,
 // corr = corr + (dmin xd) float(C) (Q6_K (d xd) float(32 C)).
 template <int WPT, int C>
@@ -1654,95 +1473,6 @@ __device__ __forceinline__ void mw_chain(const MwProd<WPT> &o, float (&acc)[8 / 
     for (int t = 0; t < 4; t++) cr[t] = cr[t] + o.cf[t] * (float)o.Cc[t];
 }
 
-// The walk of one wavefront (part C of WPT) over its tiles 0 .. ntiles - 1: tile i's bytes from
-// src(i), its LDS operands from dst(i). A tile's blocks are taken in stages of PD (mw_pd: NB up
-// to three blocks a row, two at four, else four); each block's bytes are requested one stage
-// ahead of its arithmetic into a ring of PD buffers (the next tile's first stage during the last
-// one, the last tile's first stage again at the end), the same loads on every path, so the
-// compiler's wait for a block leaves the PD later blocks in flight. done(i, part, cr) takes
-// tile i's partial sums part[t] (WPT 1: the whole hsum less the correction; matrix row lane & 15,
-// vector 4 (lane >> 4) + t) and, part 0, the correction chain cr; a done() with barriers is met
-// by every wavefront of the workgroup as long as they walk the same number of tiles.
-template <int NB>
-constexpr int mw_pd() { return NB <= 3 ? NB : NB == 4 ? 2 : 4; }
-template <int NB, int TT, int WPT, int C, int PD = mw_pd<NB>(), class Src, class Dst, class Done>
-__device__ __forceinline__ void mw_walk(int ntiles, Src src, Dst dst, Done done) {
-  constexpr int NS = NB / PD, CPW = 8 / WPT;
-  constexpr int BB = WPT == 4 ? PD : WPT == 2 && PD % 2 == 0 ? 2 : 1;  // blocks whose integers are issued together
-  static_assert(NB % PD == 0, "whole stages");
-  if (ntiles <= 0) return;
-  MwRaw r[PD];
-  MwSrc sc = src(0);
-#pragma unroll
-  for (int p = 0; p < PD; p++) mw_fetch<TT>(r[p], sc, p);
-  for (int i = 0; i < ntiles; i++) {
-    const MwDst dc = dst(i);
-    const MwSrc sn = i + 1 < ntiles ? src(i + 1) : sc;
-    float acc[CPW][4], cr[4];
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-      cr[t] = 0.0f;
-#pragma unroll
-      for (int j = 0; j < CPW; j++) acc[j][t] = 0.0f;
-    }
-    for (int st = 0; st < NS; st++) {
-      const bool last = st == NS - 1;
-      // the stage's integers in groups of BB blocks, then their chains in block order
-#pragma unroll
-      for (int p0 = 0; p0 < PD; p0 += BB) {
-        MwProd<WPT> pr[BB];
-#pragma unroll
-        for (int q = 0; q < BB; q++) {
-          if (TT == T_Q4K || (TT == 0 && dc.dt == T_Q4K)) mw_prod<T_Q4K, WPT, C>(r[p0 + q], dc, st * PD + p0 + q, pr[q]);
-          else mw_prod<T_Q6K, WPT, C>(r[p0 + q], dc, st * PD + p0 + q, pr[q]);
-        }
-#pragma unroll
-        for (int q = 0; q < BB; q++) mw_chain<WPT, C>(pr[q], acc, cr);
-      }
-#pragma unroll
-      for (int p = 0; p < PD; p++) {
-        const int b = st * PD + p;
-        MwSrc fs;
-        fs.p0 = last ? sn.p0 : sc.p0;
-        fs.p1 = last ? sn.p1 : sc.p1;
-        fs.p2 = last ? sn.p2 : sc.p2;
-        fs.p3 = last ? sn.p3 : sc.p3;
-        fs.rb = last ? sn.rb : sc.rb;
-        fs.dt = last ? sn.dt : sc.dt;
-        mw_fetch<TT>(r[p], fs, last ? p : b + PD);
-      }
-    }
-    float part[4];
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-      if constexpr (WPT == 1)
-        part[t] = (((acc[0][t] + acc[4][t]) + (acc[2][t] + acc[6][t])) + ((acc[1][t] + acc[5][t]) + (acc[3][t] + acc[7][t]))) - cr[t];
-      else if constexpr (WPT == 2)
-        part[t] = (acc[0][t] + acc[2][t]) + (acc[1][t] + acc[3][t]);
-      else
-        part[t] = acc[0][t] + acc[1][t];
-    }
-    done(i, part, cr);
-    sc = sn;
-  }
-}
-// The walk of part c (wave-uniform) of WPT: one instance per part.
-template <int NB, int TT, int WPT, class Src, class Dst, class Done>
-__device__ __forceinline__ void mw_walk_part(int c, int ntiles, Src src, Dst dst, Done done) {
-  if constexpr (WPT == 1) {
-    mw_walk<NB, TT, 1, 0>(ntiles, src, dst, done);
-  } else if constexpr (WPT == 2) {
-    if (c == 0) mw_walk<NB, TT, 2, 0>(ntiles, src, dst, done);
-    else mw_walk<NB, TT, 2, 1>(ntiles, src, dst, done);
-  } else {
-    switch (c) {
-    case 0: mw_walk<NB, TT, 4, 0>(ntiles, src, dst, done); break;
-    case 1: mw_walk<NB, TT, 4, 1>(ntiles, src, dst, done); break;
-    case 2: mw_walk<NB, TT, 4, 2>(ntiles, src, dst, done); break;
-    default: mw_walk<NB, TT, 4, 3>(ntiles, src, dst, done); break;
-    }
-  }
-}
 // The parts' partial sums of a tile meet in LDS (xch: [WPT][4][64] floats of the tile's parts, one
 // barrier; the caller alternates two such areas between tiles): part 0 returns the tile's
 // results (hsum order as at mw_cls, less the correction), other parts return zeros.
@@ -1861,14 +1591,15 @@ struct MsLoad {
     }
   }
 };
-// Block b of a staged tile, part C: its integers (MwProd), as mw_prod from the LDS image.
+// Block b of the vectors against block wb of a staged tile, part C: its integers and scale
+// factors.
 template <int T, int NB, bool Q6, int WPT, int C>
-__device__ __forceinline__ void ms_prod(const SPX_L uint8_t *tl, const MwDst &d, int b, MwProd<WPT> &o) {
+__device__ __forceinline__ void ms_prod(const SPX_L uint8_t *tl, const MwDst &d, int b, int wb, MwProd<WPT> &o) {
   using G = MsGeo<NB, Q6>;
   const int lane = threadIdx.x & 63, k4 = lane >> 4, c16 = lane & 15;
   const SPX_L uint32_t *py = d.py + b * 64, *pw = d.pw + b * MQ_CW;
-  const SPX_L uint8_t *rc = tl + G::OC + c16 * G::CR + 128 * b, *rs = tl + G::OS + c16 * G::SR + 16 * b;
-  const uint32_t dw = lld<uint32_t>((const SPX_L uint32_t *)(tl + G::OD + 4 * (c16 * NB + b)));
+  const SPX_L uint8_t *rc = tl + G::OC + c16 * G::CR + 128 * wb, *rs = tl + G::OS + c16 * G::SR + 16 * wb;
+  const uint32_t dw = lld<uint32_t>((const SPX_L uint32_t *)(tl + G::OD + 4 * (c16 * NB + wb)));
   float xd[4];
   const float dd = h2f(dw);
 #pragma unroll
@@ -1910,7 +1641,7 @@ __device__ __forceinline__ void ms_prod(const SPX_L uint8_t *tl, const MwDst &d,
       for (int t = 0; t < 4; t++) o.cf[t] = dm * xd[t];
     }
   } else {
-    const SPX_L uint8_t *rh = tl + G::OH + c16 * G::HR + 64 * b;
+    const SPX_L uint8_t *rh = tl + G::OH + c16 * G::HR + 64 * wb;
     const int h = k4 >> 1, sh = 4 * (k4 & 1);
     const uint32_t sw = lld<uint32_t>((const SPX_L uint32_t *)(rs + 4 * k4));
     uint32_t wh0[8 / WPT], wl0[8 / WPT], wh1[8 / WPT], wl1[8 / WPT];
@@ -1958,8 +1689,8 @@ __device__ __forceinline__ void ms_tile(const SPX_L uint8_t *tl, int dt, const M
     MwProd<WPT> pr[BB];
 #pragma unroll
     for (int q = 0; q < BB; q++) {
-      if (TT == T_Q4K || (TT == 0 && dt == T_Q4K)) ms_prod<T_Q4K, NB, TT != T_Q4K, WPT, C>(tl, d, b0 + q, pr[q]);
-      else ms_prod<T_Q6K, NB, true, WPT, C>(tl, d, b0 + q, pr[q]);
+      if (TT == T_Q4K || (TT == 0 && dt == T_Q4K)) ms_prod<T_Q4K, NB, TT != T_Q4K, WPT, C>(tl, d, b0 + q, b0 + q, pr[q]);
+      else ms_prod<T_Q6K, NB, true, WPT, C>(tl, d, b0 + q, b0 + q, pr[q]);
     }
 #pragma unroll
     for (int q = 0; q < BB; q++) mw_chain<WPT, C>(pr[q], acc, cr);
@@ -1989,6 +1720,134 @@ __device__ __forceinline__ void ms_tile_part(int c, const SPX_L uint8_t *tl, int
   }
 }
 
+// ---- one wavefront's walk over tiles, staged in its own LDS. In the operand layout consecutive
+// lanes hold different matrix rows: a load straight into it is 64 requests of 16 bytes (and 64
+// each for the scale lines, the high bits and d), and one CU's address unit takes about one a
+// cycle, ~256 cycles a (tile, 256-block) of Q4_K and ~380 of Q6_K against ~190 of vector
+// instructions: what bounded the prefill expert kernels and the LM head (gate/up 56 us a 128-row
+// layer, down 46, the 9-row LM head 90). So the wavefront loads a block of the tile along its rows
+// (whole 128-byte lines), parks it in its own LDS (MsGeo<1>'s layout: no two rows' words of a class
+// in one bank; no barrier, one wavefront's LDS accesses run in order), and reads its classes' words
+// there, the next two blocks' loads in flight meanwhile.
+__device__ __forceinline__ int64_t mw_uni64(int64_t v) {
+  const uint64_t u = (uint64_t)v;
+  return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)u));
+}
+struct WsSrc {  // a tile's planes at its first row (wave-uniform); lim = (rows of the tile - 1) x nb
+  const uint8_t *p0, *p1, *p2, *p3;
+  int lim, dt;
+};
+__device__ __forceinline__ WsSrc ws_src(const Planes &pl, int dt, int64_t row0, int nrows, int nb) {
+  const int64_t r0 = mw_uni64(row0) * nb;
+  WsSrc s;
+  s.dt = __builtin_amdgcn_readfirstlane(dt);
+  s.p0 = pl.p0 + r0 * 128;
+  s.p2 = pl.p2 + r0 * 16;
+  if (s.dt == T_Q4K) {
+    s.p1 = pl.p1 + r0 * 16;
+    s.p3 = s.p1;
+  } else {
+    s.p1 = pl.p1 + r0 * 64;
+    s.p3 = pl.p3 + r0 * 2;
+  }
+  s.lim = (__builtin_amdgcn_readfirstlane(nrows) - 1) * nb;
+  return s;
+}
+// One block of a tile on its way to LDS: rows lane >> 3 and 8 + (lane >> 3), 16-byte piece lane & 7
+// of their codes; row lane >> 2, piece lane & 3 of the Q6_K high bits; lanes 0-15 their row's scale
+// line and d.
+template <int NB, int TT>
+struct WsRaw {
+  static constexpr bool Q6 = TT != T_Q4K;
+  using G = MsGeo<1, Q6>;
+  uint4 c[2], s, h;
+  uint32_t d;
+  __device__ __forceinline__ void get(const WsSrc &w, int b) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t o0 = (uint32_t)(min((lane >> 3) * NB, w.lim) + b), o1 = (uint32_t)(min((8 + (lane >> 3)) * NB, w.lim) + b);
+    c[0] = gld<uint4>(w.p0 + (o0 * 128u + 16u * (lane & 7)));
+    c[1] = gld<uint4>(w.p0 + (o1 * 128u + 16u * (lane & 7)));
+    const bool q4 = TT == T_Q4K || (TT == 0 && w.dt == T_Q4K);
+    if (Q6 && !q4) h = gld<uint4>(w.p1 + ((uint32_t)(min((lane >> 2) * NB, w.lim) + b) * 64u + 16u * (lane & 3)));
+    if (lane < 16) {
+      const uint32_t o = (uint32_t)(min(lane * NB, w.lim) + b);
+      s = gld<uint4>(w.p2 + o * 16u);
+      d = q4 ? gld<uint32_t>(w.p1 + o * 16u) : (uint32_t)gld<uint16_t>(w.p3 + o * 2u);
+    }
+  }
+  __device__ __forceinline__ void put(SPX_L uint8_t *tl, int dt) const {
+    const int lane = threadIdx.x & 63;
+    __builtin_amdgcn_wave_barrier();
+    lst<uint4>(tl + G::OC + (lane >> 3) * G::CR + 16 * (lane & 7), c[0]);
+    lst<uint4>(tl + G::OC + (8 + (lane >> 3)) * G::CR + 16 * (lane & 7), c[1]);
+    if (Q6 && dt != T_Q4K) lst<uint4>(tl + G::OH + (lane >> 2) * G::HR + 16 * (lane & 3), h);
+    if (lane < 16) {
+      lst<uint2>(tl + G::OS + lane * G::SR, make_uint2(s.x, s.y));
+      lst<uint2>(tl + G::OS + lane * G::SR + 8, make_uint2(s.z, s.w));
+      lst<uint32_t>(tl + G::OD + 4 * lane, d);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+};
+template <int TT>
+constexpr int WS_BYTES = MsGeo<1, TT != T_Q4K>::BYTES;  // a wavefront's LDS
+__host__ __device__ inline size_t ws_bytes(int tt) { return tt == T_Q4K ? WS_BYTES<T_Q4K> : WS_BYTES<0>; }
+
+// The walk of one wavefront over its tiles 0 .. ntiles - 1, all eight classes: tile i's bytes from src(i), its vectors from dst(i), done(i, out) with the tile's
+// results (matrix row lane & 15, vector 4 (lane >> 4) + t). tl: the wavefront's WS_BYTES.
+template <int NB, int TT, class Src, class Dst, class Done>
+__device__ __forceinline__ void ws_walk(SPX_L uint8_t *tl, int ntiles, Src src, Dst dst, Done done) {
+  if (ntiles <= 0) return;
+  WsRaw<NB, TT> ra, rb;
+  int fi = 0, fb = 0, i = 0, b = 0;  // the next block to request, the block in hand
+  WsSrc fs = src(0);
+  MwDst dc = dst(0);
+  float acc[8][4], cr[4];
+  auto clear = [&]() SPX_AI {
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      cr[t] = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 8; j++) acc[j][t] = 0.0f;
+    }
+  };
+  auto fetch = [&](WsRaw<NB, TT> &r) SPX_AI {
+    if (fi >= ntiles) return;
+    r.get(fs, fb);
+    if (++fb == NB) {
+      fb = 0;
+      if (++fi < ntiles) fs = src(fi);
+    }
+  };
+  auto step = [&](WsRaw<NB, TT> &r) SPX_AI {
+    r.put(tl, dc.dt);
+    fetch(r);
+    MwProd<1> pr;
+    if (TT == T_Q4K || (TT == 0 && dc.dt == T_Q4K)) ms_prod<T_Q4K, 1, TT != T_Q4K, 1, 0>(tl, dc, b, 0, pr);
+    else ms_prod<T_Q6K, 1, true, 1, 0>(tl, dc, b, 0, pr);
+    mw_chain<1, 0>(pr, acc, cr);
+    if (++b < NB) return;
+    b = 0;
+    float out[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+      out[t] = (((acc[0][t] + acc[4][t]) + (acc[2][t] + acc[6][t])) + ((acc[1][t] + acc[5][t]) + (acc[3][t] + acc[7][t]))) - cr[t];
+    done(i, out);
+    clear();
+    if (++i < ntiles) dc = dst(i);
+  };
+  clear();
+  fetch(ra);
+  fetch(rb);
+  for (;;) {
+    step(ra);
+    if (i >= ntiles) break;
+    step(rb);
+    if (i >= ntiles) break;
+  }
+}
+
 // A unit of kd_mq: tile t (segment si, rows row0 .. row0 + nrows - 1). The bookkeeping is
 // wave-uniform and kept scalar (readfirstlane), so the segment's fields are read from the
 // arguments with scalar loads.
@@ -2004,23 +1863,19 @@ __device__ __forceinline__ void mq_locate(const DecMMArgs &a, int total, MqPos &
 }
 // Multi-vector matvec on the matrix cores: tiles of 16 rows over up to three segments (the
 // formats may differ by segment), the m vectors' Q8_K staged in LDS with their correction
-// words. A tile is walked by WPT wavefronts (mw_walk, each a part of the lane classes; their
-// partial sums meet in LDS), so a workgroup of MW_NW walks TP = MW_NW / WPT tiles at a time:
-// round i of workgroup r takes tiles (r + R i) TP .. + TP - 1. Part 0 runs the epilogue
-// (residual, greedy keys). Few tiles (q|k|v, the attention output) take WPT 4: a quarter of the
-// classes' arithmetic on each wavefront's path; many (the LM head) WPT 1 (mq_wpt).
+// words. A wavefront walks whole tiles (ws_walk): wavefront w of workgroup r takes tiles
+// r MW_NW + w, + R MW_NW, .... Taller matrices (the LM head) and prefill passes; few tiles at up to
+// 16 rows take kd_mqs.
 //
 // Passes of more than 16 rows (prefill) take the vectors in groups of 16: the launch holds
 // R x groups workgroups; workgroup i = 8k + x (x: its XCD) takes group k mod groups and tile
 // range r = 8 (k / groups) + x, so the groups' workgroups of one tile range share an XCD and its
 // L2: the weights come from HBM about once.
 constexpr int MW_NW = 4;  // wavefronts a workgroup of kd_mq
-template <int NB, int TT, int WPT>  // TT: the segments' one format, or 0 when they differ
+template <int NB, int TT>  // TT: the segments' one format, or 0 when they differ
 __global__ __launch_bounds__(MW_NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void kd_mq(const DecMMArgs a) {
-  constexpr int TP = MW_NW / WPT;
   extern __shared__ __align__(16) uint8_t smem[];
   __shared__ unsigned long long sbest[MAX_M];
-  __shared__ float xch[WPT > 1 ? 2 : 1][MW_NW][4][64];
   const int nvg = (a.m + 15) >> 4;
   int vg = 0, r0 = blockIdx.x, R = gridDim.x;
   if (nvg > 1) {
@@ -2037,30 +1892,27 @@ __global__ __launch_bounds__(MW_NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
   const MwLds L = mw_lds(smem, m, nb);
   const int total = a.tiles[0] + (a.nseg > 1 ? a.tiles[1] : 0) + (a.nseg > 2 ? a.tiles[2] : 0);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c16 = lane & 15;
-  const int g = wave / WPT, c = wave - g * WPT;
+  SPX_L uint8_t *tl = (SPX_L uint8_t *)(smem + mw_tail_off(m, nb)) + wave * WS_BYTES<TT>;  // (over lbs, once lc is built)
   if (threadIdx.x < MAX_M) sbest[threadIdx.x] = 0;
   stage_q8<MW_NW * 64>(y, (const int *)nullptr, m, cols, L.lq, L.ld, L.lbs, mw_vs(nb) / 4);
   __syncthreads();
   mq_corr_stage(m, nb, L.lbs, L.lc);
   __syncthreads();
   const MqVec vv = mq_vecs(m, MqIdentity{});
-  const int base = r0 * TP, S = R * TP, nr = base < total ? (total - base + S - 1) / S : 0;
+  const int base = r0 * MW_NW + wave, S = R * MW_NW, nr = base < total ? (total - base + S - 1) / S : 0;
   auto pos_of = [&](int i) SPX_AI {
     MqPos p;
-    p.t = base + i * S + g;  // (past the last tile: mq_locate's clamp, results not stored)
+    p.t = base + i * S;
     mq_locate(a, total, p);
     return p;
   };
   auto src = [&](int i) SPX_AI {
     const MqPos p = pos_of(i);
     const TensorView &w = a.w[p.si];
-    return mw_src(w.pl, w.dtype, p.row0, p.nrows, NB);
+    return ws_src(w.pl, w.dtype, p.row0, p.nrows, NB);
   };
   auto dst = [&](int i) SPX_AI { return mw_dst(L, vv, NB, a.w[pos_of(i).si].dtype); };
-  auto done = [&](int i, const float(&part)[4], const float(&cr)[4]) SPX_AI {
-    float out[4];
-    mw_meet<WPT>((SPX_L float *)&xch[WPT > 1 ? (i & 1) : 0][g * WPT][0][0], c, part, cr, out);
-    if (c != 0 || base + i * S + g >= total) return;
+  auto done = [&](int i, const float (&out)[4]) SPX_AI {
     const MqPos p = pos_of(i);
     float *const o = a.out[p.si];
     const int64_t wrows = a.w[p.si].rows, ldo = a.ld_out[p.si];
@@ -2078,7 +1930,7 @@ __global__ __launch_bounds__(MW_NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
       }
     }
   };
-  mw_walk_part<NB, TT, WPT>(c, nr, src, dst, done);
+  ws_walk<NB, TT>(tl, nr, src, dst, done);
   if (a.best) {  // per vector, the best key of each tile range
     __syncthreads();
     if ((int)threadIdx.x < m) gst<unsigned long long>(a.best + (int64_t)(v0 + threadIdx.x) * a.nbest + r0, sbest[threadIdx.x]);
@@ -2155,74 +2007,8 @@ __global__ __launch_bounds__(MW_NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
 }
 
 // Routing + gate/up + SwiGLU over the jobs on the matrix cores (kd_gateup_m's prologue and job
-// list): items (job, 16 h rows), TP = NW / WPT of them a round: round i of workgroup b takes
-// items (b + G i) TP .. + TP - 1, each walked (gate tile, then up tile) by WPT wavefronts whose
-// partial sums meet in LDS; part 0 applies SwiGLU.
-template <int T, int NB, int WPT>
-__global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void kd_gateup_mq(const DecGateUpMArgs a) {
-  constexpr int NW = DEC_MM_NW, JR = 2 + 2 * MAX_M, TP = NW / WPT;
-  extern __shared__ __align__(16) uint8_t smem[];
-  __shared__ signed char slot_of[MAX_M * 256];
-  __shared__ int wcount[NW];
-  __shared__ float xch[WPT > 1 ? 2 : 1][NW][4][64];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int g = wave / WPT, c = wave - g * WPT;
-  const int n_ff = a.n_ff, cols = (int)a.gate.cols, nb = cols >> 8, m = a.m;
-  const int TX = (n_ff + 15) / 16;
-  const MwLds L = mw_lds(smem, m, nb);
-  SPX_L int *sj = (SPX_L int *)(smem + mw_act_bytes(m, nb));  // [max jobs][JR]
-  int nj = 1;
-  {
-    StageQ8<NW * 64> st;
-    if (a.rt.logits) {
-      float lv[2][4];
-      route_load<NW>(a.rt, lv);
-      st.get(a.y, m, cols);
-      nj = route_jobs<NW>(a.rt, lv, sj, (SPX_L signed char *)slot_of, (SPX_L int *)wcount, blockIdx.x == 0);
-    } else {
-      st.get(a.y, m, cols);
-      for (int i = threadIdx.x; i < JR; i += blockDim.x) sj[i] = i == 0 ? 0 : i == 1 ? m : i < 2 + MAX_M ? i - 2 : i - 2 - MAX_M;
-    }
-    st.put(m, cols, L.lq, L.ld, L.lbs, mw_vs(nb) / 4);
-  }
-  __syncthreads();
-  mq_corr_stage(m, nb, L.lbs, L.lc);
-  __syncthreads();
-  const int n = TX * nj, base = blockIdx.x * TP, S = gridDim.x * TP, nr = base < n ? (n - base + S - 1) / S : 0;
-  auto item = [&](int k) SPX_AI { return min(base + S * (k >> 1) + g, n - 1); };  // tile k: gate (k even) or up
-  float gv[4];
-  auto src = [&](int k) SPX_AI {
-    const int i = item(k), j = i / TX, x = i - j * TX;
-    const int e = min(max(sj[j * JR], 0), a.gate.n_expert - 1);
-    return mw_src((k & 1) ? a.up.pl : a.gate.pl, T, (int64_t)e * a.gate.rows + (int64_t)x * 16, min(16, n_ff - x * 16), NB);
-  };
-  auto dst = [&](int k) SPX_AI {
-    const int j = item(k) / TX;
-    return mw_dst(L, mq_vecs(sj[j * JR + 1], MqRows{sj + j * JR + 2}), NB, T);
-  };
-  auto done = [&](int k, const float(&part)[4], const float(&cr)[4]) SPX_AI {
-    float out[4];
-    mw_meet<WPT>((SPX_L float *)&xch[WPT > 1 ? (k & 1) : 0][g * WPT][0][0], c, part, cr, out);
-    if (c != 0) return;
-    if (!(k & 1)) {
-#pragma unroll
-      for (int t = 0; t < 4; t++) gv[t] = out[t];
-      return;
-    }
-    if (base + S * (k >> 1) + g >= n) return;
-    const int i = item(k), j = i / TX, x = i - j * TX, nv = sj[j * JR + 1], r = lane & 15;
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-      const int v = 4 * (lane >> 4) + t;
-      if (v < nv && x * 16 + r < n_ff)
-        gst<float>(a.h + (int64_t)sj[j * JR + 2 + MAX_M + v] * n_ff + x * 16 + r, gv[t] / (1.0f + expf(-gv[t])) * out[t]);
-    }
-  };
-  mw_walk_part<NB, T, WPT>(c, 2 * nr, src, dst, done);
-}
-
-// kd_gateup_mq on staged tiles: rounds of two items' gate tiles, then their up tiles (MsLoad: a
-// round's bytes come into LDS at once, the next round's loads fly during this one); wavefronts
+// list) on staged tiles: items (job, 16 h rows), rounds of two items' gate tiles, then their up
+// tiles (MsLoad: a round's bytes come into LDS at once, the next round's loads fly during this one); wavefronts
 // 0-3 take the first item's tile, 4-7 the second's, a quarter of the lane classes each, their
 // partial sums meeting in LDS; part 0 applies SwiGLU. Workgroup b takes item pairs b, b + G, ...
 template <int T, int NB>
@@ -2290,174 +2076,6 @@ __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(
       if (v < nv && x * 16 + r < n_ff)
         gst<float>(a.h + (int64_t)sj[j * JR + 2 + MAX_M + v] * n_ff + x * 16 + r, gv[t] / (1.0f + expf(-gv[t])) * out[t]);
     }
-  }
-}
-
-// Down projection of the jobs' users on the matrix cores: items (job, DOWN_MQ_ROWS = 8 tiles),
-// workgroup b the items b, b + G, ...; at each item the job's users' h rows are quantized into
-// LDS (quantize_avx2 per 256 block) as kd_down_m does, and the item's tiles are walked TP =
-// NW / WPT at a time (WPT wavefronts a tile, their partial sums meeting in LDS; mw_walk: the
-// next item's bytes are requested before its staging); y per (row, choice) to yd.
-constexpr int DOWN_MQ_ROWS = 16 * DEC_MM_NW, DOWN_MQ_ITEMS = 64;
-template <int T, int NB, int WPT>
-__global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void kd_down_mq(const DecDownMArgs a) {
-  constexpr int NW = DEC_MM_NW, JF = 2 + MAX_M, TP = NW / WPT, RI = NW / TP;  // RI: rounds an item
-  extern __shared__ __align__(16) uint8_t smem[];
-  __shared__ int s_job[JF];
-  __shared__ int ihead[DOWN_MQ_ITEMS][2];  // expert, users of the workgroup's items
-  __shared__ float xch[WPT > 1 ? 2 : 1][NW][4][64];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int g = wave / WPT, c = wave - g * WPT;
-  const int dim = (int)a.w.rows, n_ff = (int)a.w.cols, TX = (dim + DOWN_MQ_ROWS - 1) / DOWN_MQ_ROWS, G = gridDim.x;
-  const MwLds L = mw_lds(smem, MAX_M, NB);
-  const int n = TX * gld<int>(a.njobs), nit = (int)blockIdx.x < n ? (n - (int)blockIdx.x + G - 1) / G : 0;
-  for (int k = threadIdx.x; k < min(nit, DOWN_MQ_ITEMS); k += blockDim.x) {
-    const int j = ((int)blockIdx.x + G * k) / TX;
-    ihead[k][0] = min(max(gld<int>(reinterpret_cast<const int *>(a.jobs + j)), 0), a.w.n_expert - 1);
-    ihead[k][1] = min(max(gld<int>(reinterpret_cast<const int *>(a.jobs + j) + 1), 0), MAX_M);
-  }
-  auto stage = [&](int k) SPX_AI {  // item k's users' h rows, quantized
-    __syncthreads();
-    const int j = ((int)blockIdx.x + G * k) / TX;
-    if ((int)threadIdx.x < JF) {
-      const int f = threadIdx.x;
-      s_job[f] = gld<int>(reinterpret_cast<const int *>(a.jobs + j) + (f < 2 ? f : 2 + MAX_M + (f - 2)));
-    }
-    __syncthreads();
-    const int nv = min(max(s_job[1], 0), MAX_M), nq = nv * NB;
-    for (int q0 = wave; q0 < nq; q0 += 4 * NW) {
-      float4 hv[4];
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const int q = q0 + NW * t;
-        if (q < nq) {
-          const int u = q / NB, i = q - u * NB;
-          hv[t] = gld<float4>(a.h + (int64_t)s_job[2 + u] * n_ff + i * 256 + 4 * lane);
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const int q = q0 + NW * t;
-        if (q < nq) {
-          const int u = q / NB, i = q - u * NB;
-          const float am = q8k_amax(hv[t]);
-          q8k_block_store(hv[t], am, L.lq + u * mw_vs(NB) + i * 64, L.ld + q, (SPX_L int *)L.lbs + q * 16);
-        }
-      }
-    }
-    __syncthreads();
-    mq_corr_stage(nv, NB, L.lbs, L.lc);
-    __syncthreads();
-  };
-  auto row0 = [&](int k) SPX_AI {  // tile k: item k / RI, its tile (k % RI) TP + g
-    const int it = (int)blockIdx.x + G * (k / RI);
-    return (it - (it / TX) * TX) * DOWN_MQ_ROWS + 16 * ((k % RI) * TP + g);
-  };
-  auto src = [&](int k) SPX_AI {
-    const int r0 = row0(k);
-    return mw_src(a.w.pl, T, (int64_t)ihead[k / RI][0] * dim + min(r0, dim - 1), max(1, min(16, dim - r0)), NB);
-  };
-  auto dst = [&](int k) SPX_AI { return mw_dst(L, mq_vecs(ihead[k / RI][1], MqIdentity{}), NB, T); };
-  auto done = [&](int k, const float(&part)[4], const float(&cr)[4]) SPX_AI {
-    float out[4];
-    mw_meet<WPT>((SPX_L float *)&xch[WPT > 1 ? (k & 1) : 0][g * WPT][0][0], c, part, cr, out);
-    if (c == 0) {
-      const int r0 = row0(k), nv = ihead[k / RI][1], r = lane & 15;
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const int v = 4 * (lane >> 4) + t;
-        if (v < nv && r0 + r < dim) gst<float>(a.yd + (int64_t)s_job[2 + v] * dim + r0 + r, out[t]);
-      }
-    }
-    if (k % RI == RI - 1 && k / RI + 1 < nit) stage(k / RI + 1);  // (its first barrier: every reader of s_job is done)
-  };
-  if (nit > 0) stage(0);
-  mw_walk_part<NB, T, WPT>(c, nit * RI, src, dst, done);
-}
-
-// kd_down_mq for passes of up to 16 rows on staged tiles: an item's eight tiles in four rounds
-// of two (MsLoad; the next round's loads, the next item's included, fly during this one),
-// wavefronts 0-3 on the first tile, 4-7 on the second, a quarter of the lane classes each.
-template <int T, int NB>
-__global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void kd_down_mqs(const DecDownMArgs a) {
-  constexpr int NW = DEC_MM_NW, JF = 2 + MAX_M, RI = 4;  // RI: rounds an item
-  static_assert(DOWN_MQ_ROWS == 16 * 2 * RI, "eight tiles an item");
-  using G = MsGeo<NB, T == T_Q6K>;
-  extern __shared__ __align__(16) uint8_t smem[];
-  __shared__ int s_job[JF];
-  __shared__ int ihead[DOWN_MQ_ITEMS][2];  // expert, users of the workgroup's items
-  __shared__ float xch[2][NW][4][64];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int g = wave >> 2, c = wave & 3;
-  const int dim = (int)a.w.rows, n_ff = (int)a.w.cols, TX = (dim + DOWN_MQ_ROWS - 1) / DOWN_MQ_ROWS, R = gridDim.x;
-  const MwLds L = mw_lds(smem, MAX_M, NB);
-  SPX_L uint8_t *tl = (SPX_L uint8_t *)(smem + mw_tail_off(MAX_M, NB));  // (over lbs between the items' stagings)
-  const int n = TX * gld<int>(a.njobs), nit = (int)blockIdx.x < n ? (n - (int)blockIdx.x + R - 1) / R : 0;
-  for (int k = threadIdx.x; k < min(nit, DOWN_MQ_ITEMS); k += blockDim.x) {
-    const int j = ((int)blockIdx.x + R * k) / TX;
-    ihead[k][0] = min(max(gld<int>(reinterpret_cast<const int *>(a.jobs + j)), 0), a.w.n_expert - 1);
-    ihead[k][1] = min(max(gld<int>(reinterpret_cast<const int *>(a.jobs + j) + 1), 0), MAX_M);
-  }
-  __syncthreads();
-  // round k: item k / RI, its tiles 2 (k % RI) + u
-  auto row0 = [&](int k, int u) SPX_AI {
-    const int it = (int)blockIdx.x + R * (k / RI);
-    return (it - (it / TX) * TX) * DOWN_MQ_ROWS + 16 * (2 * (k % RI) + u);
-  };
-  auto msrc = [&](int k, int u) SPX_AI {
-    const int r0 = row0(k, u);
-    return MsSrc{a.w.pl, (int64_t)ihead[k / RI][0] * dim + min(r0, dim - 1), max(1, min(16, dim - r0))};
-  };
-  MsLoad<NB, NW * 64, T == T_Q6K, 2> ld;
-  if (nit > 0) ld.get(T, msrc(0, 0), msrc(0, 1));
-  for (int k = 0; k < nit * RI; k++) {
-    if (k % RI == 0) {  // item k / RI: its users' h rows, quantized (quantize_avx2 per 256 block)
-      const int j = ((int)blockIdx.x + R * (k / RI)) / TX;
-      if ((int)threadIdx.x < JF) {
-        const int f = threadIdx.x;
-        s_job[f] = gld<int>(reinterpret_cast<const int *>(a.jobs + j) + (f < 2 ? f : 2 + MAX_M + (f - 2)));
-      }
-      __syncthreads();
-      const int nv = min(max(s_job[1], 0), MAX_M), nq = nv * NB;
-      for (int q0 = wave; q0 < nq; q0 += 4 * NW) {
-        float4 hv[4];
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const int q = q0 + NW * t;
-          if (q < nq) {
-            const int u = q / NB, i = q - u * NB;
-            hv[t] = gld<float4>(a.h + (int64_t)s_job[2 + u] * n_ff + i * 256 + 4 * lane);
-          }
-        }
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const int q = q0 + NW * t;
-          if (q < nq) {
-            const int u = q / NB, i = q - u * NB;
-            const float am = q8k_amax(hv[t]);
-            q8k_block_store(hv[t], am, L.lq + u * mw_vs(NB) + i * 64, L.ld + q, (SPX_L int *)L.lbs + q * 16);
-          }
-        }
-      }
-      __syncthreads();
-      mq_corr_stage(nv, NB, L.lbs, L.lc);
-      __syncthreads();  // lbs read: the tiles may take its place
-    }
-    ld.put(tl, T);
-    __syncthreads();
-    if (k + 1 < nit * RI) ld.get(T, msrc(k + 1, 0), msrc(k + 1, 1));
-    float part[4], cr[4], out[4];
-    ms_tile_part<NB, T, 4>(c, tl + g * G::BYTES, T, mw_dst(L, mq_vecs(ihead[k / RI][1], MqIdentity{}), NB, T), part, cr);
-    mw_meet<4>((SPX_L float *)&xch[k & 1][4 * g][0][0], c, part, cr, out);  // (its barrier: the tiles are read)
-    if (c == 0) {
-      const int r0 = row0(k, g), nv = ihead[k / RI][1], r = lane & 15;
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const int v = 4 * (lane >> 4) + t;
-        if (v < nv && r0 + r < dim) gst<float>(a.yd + (int64_t)s_job[2 + v] * dim + r0 + r, out[t]);
-      }
-    }
-    if (k % RI == RI - 1) __syncthreads();  // every reader of s_job and the staged h is done
   }
 }
 
@@ -2595,12 +2213,10 @@ __global__ __launch_bounds__(256) void kp_moe_combine(const float *yd, const flo
 
 // Gate / up + SwiGLU of a prefill pass on the matrix cores over a job list of at most sixteen
 // users a job (MoE: kp_route's, in global memory; dense, jobs null: rows 16j .. 16j + 15 as
-// job j): items (job, 16 h rows) as kd_gateup_mq takes them, workgroup b the items
+// job j): items (job, 16 h rows), workgroup b the items
 // [b n / G, (b + 1) n / G), job by job: the job's users' Q8_K rows are staged in LDS (slot =
 // the user's place in the job), then wavefront w walks the job's items w, w + NW, ... of the
-// range. An item's arithmetic, and so each h value, is kd_gateup_mq's.
-template <int NB>
-constexpr int KP_PD() { return NB >= 8 ? 2 : mw_pd<NB>(); }
+// range (ws_walk). Each h value has the bits of kd_gateup_mqs's.
 template <int T, int NB>
 __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void kp_gateup_mq(const DecGateUpMArgs a,
                                                                                                      const Job *jobs,
@@ -2612,6 +2228,7 @@ __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(
   const int n_ff = a.n_ff, cols = (int)a.gate.cols, nb = cols >> 8, m = a.m;
   const int TX = (n_ff + 15) / 16;
   const MwLds L = mw_lds(smem, MAX_M, nb);
+  SPX_L uint8_t *tl = (SPX_L uint8_t *)(smem + mw_tail_off(MAX_M, nb)) + wave * WS_BYTES<T>;  // (over lbs, once lc is built)
   const int nj = jobs ? gld<int>(njobs) : (m + MAX_M - 1) / MAX_M;
   const int n = TX * nj, G = gridDim.x;
   const int i0 = (int)((int64_t)blockIdx.x * n / G), i1 = (int)((int64_t)(blockIdx.x + 1) * n / G);
@@ -2635,10 +2252,10 @@ __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(
     float g[4];
     auto src = [&](int k) SPX_AI {  // tile k: item s0 + wave + NW (k / 2), gate (k even) or up
       const int x = s0 + wave + NW * (k >> 1) - j * TX;
-      return mw_src((k & 1) ? a.up.pl : a.gate.pl, T, (int64_t)e * a.gate.rows + (int64_t)x * 16, min(16, n_ff - x * 16), NB);
+      return ws_src((k & 1) ? a.up.pl : a.gate.pl, T, (int64_t)e * a.gate.rows + (int64_t)x * 16, min(16, n_ff - x * 16), NB);
     };
     auto dst = [&](int) SPX_AI { return mw_dst(L, vv, NB, T); };
-    auto done = [&](int k, const float (&out)[4], const float (&)[4]) SPX_AI {
+    auto done = [&](int k, const float (&out)[4]) SPX_AI {
 #pragma unroll
       for (int t = 0; t < 4; t++)
         if (!(k & 1)) g[t] = out[t];
@@ -2650,17 +2267,16 @@ __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(
         if (v < nv && x * 16 + r < n_ff) gst<float>(a.h + (int64_t)sj[2 + MAX_M + v] * n_ff + x * 16 + r, g[t] / (1.0f + expf(-g[t])) * out[t]);
       }
     };
-    mw_walk<NB, T, 1, 0, KP_PD<NB>()>(2 * nit, src, dst, done);
+    ws_walk<NB, T>(tl, 2 * nit, src, dst, done);
     s0 = s1;
   }
 }
 
 // Down projection of a prefill pass over its job list: tiles (job, 16 rows of the expert's down
 // matrix), workgroup b the tiles [b n / G, (b + 1) n / G), job by job as kp_gateup_mq takes its
-// items: the job's users' h rows are quantized into LDS once (kd_down_mq's staging, quantize_avx2
+// items: the job's users' h rows are quantized into LDS once (quantize_avx2
 // per 256 block), then wavefront w walks the job's tiles w, w + NW, ... of the range with no
-// barrier between tiles. A tile's arithmetic is kd_down_mq's one-wavefront tile, so each y value
-// has its bits; y per (row, choice) to yd.
+// barrier between tiles. Each y value has the bits of kd_down_m's; y per (row, choice) to yd.
 template <int T, int NB>
 __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void kp_down_mq(const DecDownMArgs a) {
   constexpr int NW = DEC_MM_NW, JF = 2 + MAX_M;  // job fields: expert, nvec, out[]
@@ -2669,6 +2285,7 @@ __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int dim = (int)a.w.rows, n_ff = (int)a.w.cols, TX = (dim + 15) / 16, G = gridDim.x;
   const MwLds L = mw_lds(smem, MAX_M, NB);
+  SPX_L uint8_t *tl = (SPX_L uint8_t *)(smem + mw_tail_off(MAX_M, NB)) + wave * WS_BYTES<T>;  // (over lbs, once lc is built)
   const int n = TX * gld<int>(a.njobs);
   const int i0 = (int)((int64_t)blockIdx.x * n / G), i1 = (int)((int64_t)(blockIdx.x + 1) * n / G);
   for (int s0 = i0; s0 < i1;) {
@@ -2709,10 +2326,10 @@ __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(
     auto row0 = [&](int k) SPX_AI { return (s0 + wave + NW * k - j * TX) * 16; };
     auto src = [&](int k) SPX_AI {
       const int r0 = row0(k);
-      return mw_src(a.w.pl, T, (int64_t)e * dim + r0, min(16, dim - r0), NB);
+      return ws_src(a.w.pl, T, (int64_t)e * dim + r0, min(16, dim - r0), NB);
     };
     auto dst = [&](int) SPX_AI { return mw_dst(L, vv, NB, T); };
-    auto done = [&](int k, const float (&out)[4], const float (&)[4]) SPX_AI {
+    auto done = [&](int k, const float (&out)[4]) SPX_AI {
       const int r0 = row0(k), r = lane & 15;
 #pragma unroll
       for (int t = 0; t < 4; t++) {
@@ -2720,7 +2337,7 @@ __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(
         if (v < nv && r0 + r < dim) gst<float>(a.yd + (int64_t)s_job[2 + v] * dim + r0 + r, out[t]);
       }
     };
-    mw_walk<NB, T, 1, 0, 1>(nit, src, dst, done);
+    ws_walk<NB, T>(tl, nit, src, dst, done);
     s0 = s1;
   }
 }
@@ -2935,11 +2552,9 @@ static size_t ms_tile_bytes(int nb, bool q6) {
   default: return q6 ? MsGeo<16, true>::BYTES : MsGeo<16, false>::BYTES;
   }
 }
-// kd_mq's form: up to 16 vectors and up to four tiles a CU, the staged tiles (kd_mqs: four
-// wavefronts a tile); taller matrices (the LM head), one wavefront a tile (kd_mq's walk, WPT 1);
-// prefill, two (WPT 2: the walk's eight chains and block ring exceed the registers of one
-// wavefront when the formats are mixed).
-static int mq_wpt(int tiles, int m) { return m > MAX_M ? 2 : tiles > 4 * cu_count() ? 1 : 4; }
+// Up to 16 vectors and up to four tiles a CU: a tile shared by four wavefronts (kd_mqs); taller
+// matrices (the LM head) and prefill passes: a wavefront a tile (kd_mq).
+static bool mq_tiled(int tiles, int m) { return m <= MAX_M && tiles <= 4 * cu_count(); }
 
 hipError_t launch_dec_mq(const DecMMArgs &a, int grid, hipStream_t s) {
   const int nb = a.cols >> 8, nvg = (a.m + 15) / 16;
@@ -2949,19 +2564,19 @@ hipError_t launch_dec_mq(const DecMMArgs &a, int grid, hipStream_t s) {
     if ((a.w[i].dtype != T_Q4K && a.w[i].dtype != T_Q6K) || a.w[i].nb != nb) return hipErrorInvalidValue;
   if (a.res_out && a.nseg != 1) return hipErrorInvalidValue;
   if (a.best && a.nbest != grid) return hipErrorInvalidValue;
-  const size_t sm = mw_act_bytes(std::min(a.m, MAX_M), nb);
-  const int total = a.tiles[0] + (a.nseg > 1 ? a.tiles[1] : 0) + (a.nseg > 2 ? a.tiles[2] : 0), wpt = mq_wpt(total, a.m);
+  const int total = a.tiles[0] + (a.nseg > 1 ? a.tiles[1] : 0) + (a.nseg > 2 ? a.tiles[2] : 0);
   int tt = a.w[0].dtype;
   for (int i = 1; i < a.nseg; i++)
     if (a.w[i].dtype != tt) tt = 0;
+  const int mx = std::min(a.m, MAX_M);
+  const size_t sm = mw_tail_off(mx, nb) + std::max((size_t)mx * nb * 64, MW_NW * ws_bytes(tt));
   const dim3 g(grid * nvg), b(MW_NW * 64);
   auto go = [&](auto kern) {
     SPX_DLDS(kern, sm);
     hipLaunchKernelGGL(kern, g, b, sm, s, a);
     return hipGetLastError();
   };
-  const int mv = std::min(a.m, MAX_M);
-  const size_t sms = mw_tail_off(mv, nb) + std::max((size_t)mv * nb * 64, ms_tile_bytes(nb, tt != T_Q4K));
+  const size_t sms = mw_tail_off(mx, nb) + std::max((size_t)mx * nb * 64, ms_tile_bytes(nb, tt != T_Q4K));
   auto gos = [&](auto kern) {
     SPX_DLDS(kern, sms);
     hipLaunchKernelGGL(kern, g, b, sms, s, a);
@@ -2971,7 +2586,7 @@ hipError_t launch_dec_mq(const DecMMArgs &a, int grid, hipStream_t s) {
     constexpr int NB = decltype(NBc)::value;
     auto by_wpt = [&](auto TTc) {
       constexpr int TT = decltype(TTc)::value;
-      return wpt == 4 ? gos(kd_mqs<NB, TT>) : wpt == 2 ? go(kd_mq<NB, TT, 2>) : go(kd_mq<NB, TT, 1>);
+      return mq_tiled(total, a.m) ? gos(kd_mqs<NB, TT>) : go(kd_mq<NB, TT>);
     };
     if (tt == T_Q4K) return by_wpt(std::integral_constant<int, T_Q4K>{});
     if (tt == T_Q6K) return by_wpt(std::integral_constant<int, T_Q6K>{});
@@ -2981,9 +2596,9 @@ hipError_t launch_dec_mq(const DecMMArgs &a, int grid, hipStream_t s) {
 
 bool dec_mq_nb_ok(int nb) { return nb == 1 || nb == 2 || nb == 3 || nb == 4 || nb == 8 || nb == 16; }
 
-// kd_mq's workgroups: MW_NW wavefronts, MW_NW / mq_wpt tiles at a time, two workgroups a CU.
+// kd_mq's workgroups: MW_NW wavefronts, a tile each (kd_mqs: one tile a workgroup), two a CU.
 int dec_mq_grid(int tiles, int m) {
-  const int slots = 2 * cu_count(), tp = MW_NW / mq_wpt(tiles, m), need = (tiles + tp - 1) / tp;
+  const int slots = 2 * cu_count(), tp = mq_tiled(tiles, m) ? 1 : MW_NW, need = (tiles + tp - 1) / tp;
   if (m <= MAX_M) return std::max(1, std::min(need, slots));
   const int nvg = (m + 15) / 16, per = (slots / nvg + 7) / 8 * 8;
   return std::max(8, std::min((need + 7) / 8 * 8, per));
@@ -3052,7 +2667,7 @@ hipError_t launch_kp_gateup_mq(const DecGateUpMArgs &a, const Job *jobs, const i
   if (a.gate.cols % 256 || nb > DEC_MAXNB || a.gate.nb != nb || a.up.nb != nb || a.gate.dtype != a.up.dtype || a.m < 1 || a.m > PMAX ||
       max_jobs < 1 || max_jobs > 512 || (jobs && !njobs))
     return hipErrorInvalidValue;
-  const size_t sm = mw_act_bytes(MAX_M, nb);
+  const size_t sm = mw_tail_off(MAX_M, nb) + std::max((size_t)MAX_M * nb * 64, DEC_MM_NW * ws_bytes(a.gate.dtype));
   const int njob = jobs ? max_jobs : (a.m + MAX_M - 1) / MAX_M, items = ((a.n_ff + 15) / 16) * njob;
   const dim3 grid((unsigned)std::max(1, std::min((items + DEC_MM_NW - 1) / DEC_MM_NW, cu_count()))), b(DEC_MM_NW * 64);
   if (a.gate.dtype != T_Q4K && a.gate.dtype != T_Q6K) return hipErrorInvalidValue;
@@ -3069,51 +2684,13 @@ hipError_t launch_kp_down_mq(const DecDownMArgs &a, hipStream_t s) {
   if (a.w.dtype != T_Q4K && a.w.dtype != T_Q6K) return hipErrorInvalidValue;
   const int items = (int)((a.w.rows + 15) / 16) * a.max_jobs;
   const dim3 grid((unsigned)std::max(1, std::min((items + DEC_MM_NW - 1) / DEC_MM_NW, cu_count()))), b(DEC_MM_NW * 64);
-  const size_t sm = mw_act_bytes(MAX_M, (int)a.w.nb);
+  const size_t sm = mw_tail_off(MAX_M, (int)a.w.nb) + std::max((size_t)MAX_M * a.w.nb * 64, DEC_MM_NW * ws_bytes(a.w.dtype));
   return with_nb((int)a.w.nb, [&](auto NBc) {
     constexpr int NB = decltype(NBc)::value;
     auto kern = a.w.dtype == T_Q4K ? kp_down_mq<T_Q4K, NB> : kp_down_mq<T_Q6K, NB>;
     SPX_DLDS(kern, sm);
     hipLaunchKernelGGL(kern, grid, b, sm, s, a);
     return hipGetLastError();
-  });
-}
-
-// passes of more than 128 jobs on kp_down_mq (SPX_PF_DOWN=0: kd_down_mq, the same bits)
-static bool pf_down_on() {
-  static const bool on = [] {
-    const char *v = std::getenv("SPX_PF_DOWN");
-    return !v || atoi(v) != 0;
-  }();
-  return on;
-}
-
-hipError_t launch_dec_down_mq(const DecDownMArgs &a, hipStream_t s) {
-  if (a.w.cols % 256 || a.w.nb > 4 || a.max_jobs < 1 || a.max_jobs > 512 || !a.h || !a.yd) return hipErrorInvalidValue;
-  const int tx = (int)((a.w.rows + DOWN_MQ_ROWS - 1) / DOWN_MQ_ROWS), G = std::min(tx * a.max_jobs, cu_count());
-  if ((tx * a.max_jobs + G - 1) / G > DOWN_MQ_ITEMS) return hipErrorInvalidValue;  // items a workgroup, cached in LDS
-  const dim3 grid((unsigned)G), b(DEC_MM_NW * 64);
-  const size_t sm = mw_act_bytes(MAX_M, (int)a.w.nb);
-  if (a.w.dtype != T_Q4K && a.w.dtype != T_Q6K) return hipErrorInvalidValue;
-  auto go = [&](auto kern) {
-    SPX_DLDS(kern, sm);
-    hipLaunchKernelGGL(kern, grid, b, sm, s, a);
-    return hipGetLastError();
-  };
-  // a pass of up to 16 rows (at most 128 jobs): staged tiles, four wavefronts a tile; prefill:
-  // one wavefront a tile
-  const size_t sms = mw_tail_off(MAX_M, (int)a.w.nb) + std::max((size_t)MAX_M * a.w.nb * 64, 2 * ms_tile_bytes((int)a.w.nb, a.w.dtype == T_Q6K));
-  auto gos = [&](auto kern) {
-    SPX_DLDS(kern, sms);
-    hipLaunchKernelGGL(kern, grid, b, sms, s, a);
-    return hipGetLastError();
-  };
-  const bool staged = a.max_jobs <= 128;
-  if (!staged && pf_down_on()) return launch_kp_down_mq(a, s);  // prefill: contiguous tile ranges, job by job
-  return with_nb((int)a.w.nb, [&](auto NBc) {
-    constexpr int NB = decltype(NBc)::value;
-    if (a.w.dtype == T_Q4K) return staged ? gos(kd_down_mqs<T_Q4K, NB>) : go(kd_down_mq<T_Q4K, NB, 1>);
-    return staged ? gos(kd_down_mqs<T_Q6K, NB>) : go(kd_down_mq<T_Q6K, NB, 1>);
   });
 }
 
