@@ -120,7 +120,11 @@ struct spx_engine {
   // device state
   __half *kc = nullptr, *vc = nullptr;
   float2 *rope = nullptr;
+  // host memory that the device reads and writes: a pass's step record, its picks, hidden rows (up to
+  // 16) and one row of logits
   StepRec *st_dev = nullptr, *st_host = nullptr;
+  int *picks_host = nullptr;
+  float *hidden_host = nullptr, *logits_host = nullptr;
   float *xA = nullptr, *xB = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *att = nullptr, *proj = nullptr, *ffn = nullptr;
   float *xn2 = nullptr, *h = nullptr, *rlog = nullptr, *logits = nullptr, *xn = nullptr, *part_ml = nullptr, *part_o = nullptr;
   Q8KP aq{}, xq2{}, hq{}, xq{};
@@ -318,6 +322,17 @@ int mv_res(spx_engine *E, const spx_tensor *w, const float *x, int64_t ld_x, flo
   return mv_run(E, a, 1, 0);
 }
 
+// Where a pass of m rows finds its step record: in host memory (the embedding kernel brings it), or, for
+// longer passes and the one-row passes that advance it on the device, already in st_dev (null). A
+// 128-row pass would read the bus from 128 workgroups; a copy before it costs 5 us of its 860.
+const StepRec *step_src(const spx_engine *E, int m, bool advance = false) { return advance || m > MAX_M ? nullptr : E->st_host; }
+
+// Where the last kernel of a pass leaves n rows' picks and (up to 16 rows) their hidden states, rows
+// row0 .. of xn.
+HostOut host_out(spx_engine *E, int n, int row0) {
+  return HostOut{E->picks_host, n <= MAX_M ? E->hidden_host : nullptr, E->xn + (int64_t)row0 * E->c.dim, E->c.dim};
+}
+
 // A matrix whose passes of two rows and more run on the bf16 matrix cores (fx.hip).
 bool fx_on(const spx_engine *E, const spx_tensor *t) {
   return E->mq && (t->v.dtype == T_Q8_0 || (t->v.dtype == T_Q5_0 && E->all_float));
@@ -388,7 +403,7 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
     ProfScope ps(E, PC_EMBED, 0);
     NormTail t = norm_next(E, 0, E->xA, nullptr, nullptr);
     if (pro) t.nw = nullptr;  // the embedding row only
-    SPX_HIP(launch_embed(E->embed->v, E->st_dev, c.embedding_scale, t, m, s));
+    SPX_HIP(launch_embed(E->embed->v, E->st_dev, step_src(E, m, advance), c.embedding_scale, t, m, s));
   }
   for (int l = 0; l < c.n_layers; l++) {
     const LayerW &ly = E->L[l];
@@ -567,7 +582,7 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
   }
   {
     ProfScope ps(E, PC_ARGMAX, 0);
-    SPX_HIP(launch_argmax_final(E->best, E->nbest, E->amax, last ? nullptr : E->st_dev, advance ? E->hist : nullptr, lm, s));
+    SPX_HIP(launch_argmax_final(E->best, E->nbest, E->amax, last ? nullptr : E->st_dev, advance ? E->hist : nullptr, lm, advance ? HostOut{} : host_out(E, lm, m - lm), s));
   }
   return 0;
 }
@@ -591,7 +606,7 @@ int enqueue_decode(spx_engine *E, bool advance, int nv = 1) {
     NormTail t{};
     t.x = E->xA;
     t.dim = dim;
-    SPX_HIP(launch_embed(E->embed->v, E->st_dev, c.embedding_scale, t, nv, s));
+    SPX_HIP(launch_embed(E->embed->v, E->st_dev, step_src(E, nv, advance), c.embedding_scale, t, nv, s));
   }
   for (int l = 0; l < c.n_layers; l++) {
     const LayerW &ly = E->L[l];
@@ -703,7 +718,7 @@ int enqueue_decode(spx_engine *E, bool advance, int nv = 1) {
   E->nbest = grid;
   {
     ProfScope ps(E, PC_ARGMAX, 0);
-    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, last ? nullptr : E->st_dev, advance ? E->hist : nullptr, nl, s));
+    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, last ? nullptr : E->st_dev, advance ? E->hist : nullptr, nl, advance ? HostOut{} : host_out(E, nl, 0), s));
   }
   return 0;
 }
@@ -749,7 +764,7 @@ int enqueue_pass_m(spx_engine *E, int m) {
     NormTail t{};
     t.x = E->xA;
     t.dim = dim;
-    SPX_HIP(launch_embed(E->embed->v, E->st_dev, c.embedding_scale, t, m, s));
+    SPX_HIP(launch_embed(E->embed->v, E->st_dev, step_src(E, m), c.embedding_scale, t, m, s));
   }
   for (int l = 0; l < c.n_layers; l++) {
     const LayerW &ly = E->L[l];
@@ -881,7 +896,7 @@ int enqueue_pass_m(spx_engine *E, int m) {
     SPX_HIP(launch_dec_mv(a, grid, s));
     E->nbest = grid;
     ProfScope pa(E, PC_ARGMAX, 0);
-    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, nullptr, nullptr, 1, s));
+    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, nullptr, nullptr, 1, host_out(E, 1, 0), s));
     return 0;
   }
   {
@@ -898,7 +913,7 @@ int enqueue_pass_m(spx_engine *E, int m) {
   E->nbest = grid;
   {
     ProfScope ps(E, PC_ARGMAX, 0);
-    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, E->st_dev, nullptr, m, s));
+    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, E->st_dev, nullptr, m, host_out(E, m, 0), s));
   }
   return 0;
 }
@@ -913,7 +928,7 @@ int enqueue_persist(spx_engine *E, bool advance) {
     NormTail t{};
     t.x = E->xA;
     t.dim = c.dim;
-    SPX_HIP(launch_embed(E->embed->v, E->st_dev, c.embedding_scale, t, 1, s));
+    SPX_HIP(launch_embed(E->embed->v, E->st_dev, step_src(E, 1, advance), c.embedding_scale, t, 1, s));
   }
   SPX_HIP(hipMemsetAsync(E->pa.bar, 0, PERSIST_BAR_WORDS * sizeof(unsigned), s));
   unsigned epoch = 0;
@@ -937,7 +952,7 @@ int enqueue_persist(spx_engine *E, bool advance) {
   E->nbest = grid;
   {
     ProfScope ps(E, PC_ARGMAX, 0);
-    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, E->st_dev, advance ? E->hist : nullptr, 1, s));
+    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, E->st_dev, advance ? E->hist : nullptr, 1, advance ? HostOut{} : host_out(E, 1, 0), s));
   }
   return 0;
 }
@@ -1167,6 +1182,9 @@ int spx_engine_prepare(spx_engine *E) {
   for (auto &ly : E->L)
     if (ly.moe && !(ly.njobs = E->dalloc<int>(3))) return fail("out of device memory");
   SPX_HIP(hipHostMalloc(&E->st_host, sizeof(StepRec)));
+  SPX_HIP(hipHostMalloc(&E->picks_host, sizeof(int) * PMAX));
+  SPX_HIP(hipHostMalloc(&E->hidden_host, sizeof(float) * MAX_M * c.dim));
+  SPX_HIP(hipHostMalloc(&E->logits_host, sizeof(float) * ((c.vocab + 3) / 4 * 4)));
   // RoPE table: inv_freq = 1/theta^(2i/hd) (Rope::new :1399-1402); angle = pos * inv_freq.
   const int half = c.head_dim / 2;
   std::vector<float2> tab((size_t)c.max_seq * half);
@@ -1356,29 +1374,40 @@ int forward_sel(spx_engine *E, const int32_t *ids, int m, int start_pos, float *
   }
   hipStream_t s = E->ctx->stream;
   SPX_HIP(hipSetDevice(E->ctx->device));
-  SPX_HIP(hipStreamSynchronize(s));
+  // (a pass is waited for before its call returns: the record is free to be written)
   E->st_host->m = m;
   E->st_host->start = start_pos;
   E->st_host->step = 0;
   for (int i = 0; i < m; i++) E->st_host->ids[i] = ids[i];
   E->last_m = m;
-  SPX_HIP(hipMemcpyAsync(E->st_dev, E->st_host, sizeof(StepRec), hipMemcpyHostToDevice, s));
+  if (!step_src(E, m)) SPX_HIP(hipMemcpyAsync(E->st_dev, E->st_host, sizeof(StepRec), hipMemcpyHostToDevice, s));
   E->lm_sel = sel;
   const int rf = run_forward(E, m);
   E->lm_sel = 0;
-  if (rf) return rf;
+  if (rf) {
+    (void)hipStreamSynchronize(s);  // what was queued still reads the record
+    return rf;
+  }
   const int nr = sel ? 1 : m;  // rows copied out (sel 1: the last row's, at row 0; the decode pipeline's norm writes row 0)
   const int64_t hrow = sel && !(E->dec_ok && E->dec_on) ? m - 1 : 0;
+  // up to 16 hidden rows and the picks are in host memory when the pass ends; one row of logits takes
+  // the same way, more take a copy
+  const bool one_row = logits && nr == 1, hid_host = nr <= MAX_M;
   if (sel != 2) {
-    if (hidden) SPX_HIP(hipMemcpyAsync(hidden, E->xn + hrow * E->c.dim, sizeof(float) * nr * E->c.dim, hipMemcpyDeviceToHost, s));
-    if (logits) SPX_HIP(hipMemcpyAsync(logits, E->logits, sizeof(float) * nr * E->c.vocab, hipMemcpyDeviceToHost, s));
-    if (argmax) SPX_HIP(hipMemcpyAsync(argmax, E->amax, sizeof(int) * nr, hipMemcpyDeviceToHost, s));
+    if (hidden && !hid_host) SPX_HIP(hipMemcpyAsync(hidden, E->xn + hrow * E->c.dim, sizeof(float) * nr * E->c.dim, hipMemcpyDeviceToHost, s));
+    if (one_row) SPX_HIP(launch_to_host(E->logits, E->logits_host, (E->c.vocab + 3) / 4 * 4, s));
+    else if (logits) SPX_HIP(hipMemcpyAsync(logits, E->logits, sizeof(float) * nr * E->c.vocab, hipMemcpyDeviceToHost, s));
   }
   const bool pers = persist_used(E, m);
   if (pers) SPX_HIP(hipMemcpyAsync(E->perr_host, E->pa.err, sizeof(int), hipMemcpyDeviceToHost, s));
   SPX_HIP(hipStreamSynchronize(s));
   if (pers)
     if (int r = persist_check(E)) return r;
+  if (sel != 2) {
+    if (hidden && hid_host) memcpy(hidden, E->hidden_host, sizeof(float) * nr * E->c.dim);
+    if (one_row) memcpy(logits, E->logits_host, sizeof(float) * E->c.vocab);
+    if (argmax) memcpy(argmax, E->picks_host, sizeof(int) * nr);
+  }
   if (E->profiling && !E->prof.empty()) {
     std::vector<int32_t> nj(E->c.n_layers, 0);  // experts run per layer (their slabs' bytes)
     for (int l = 0; l < E->c.n_layers; l++)
@@ -1457,13 +1486,8 @@ int spx_engine_decode(spx_engine *E, int32_t token, int start_pos, int n, int32_
   if (n == 0) return 0;
   hipStream_t s = E->ctx->stream;
   SPX_HIP(hipSetDevice(E->ctx->device));
-  SPX_HIP(hipStreamSynchronize(s));
-  E->st_host->m = 1;
-  E->st_host->start = start_pos;
-  E->st_host->ids[0] = token;
-  E->st_host->step = 0;
   E->last_m = 1;
-  SPX_HIP(hipMemcpyAsync(E->st_dev, E->st_host, sizeof(StepRec), hipMemcpyHostToDevice, s));
+  SPX_HIP(launch_step(E->st_dev, 1, start_pos, token, s));
   const bool pers = persist_used(E, 1);
   for (int i = 0; i < n; i++)
     if (int r = run_forward(E, 1, true)) return r;
@@ -1607,11 +1631,7 @@ int spx_engine_attention(spx_engine *E, int layer, const float *q, const float *
   const int hd = c.head_dim;
   hipStream_t s = E->ctx->stream;
   SPX_HIP(hipSetDevice(E->ctx->device));
-  SPX_HIP(hipStreamSynchronize(s));
-  E->st_host->m = m;
-  E->st_host->start = start_pos;
-  E->st_host->step = 0;
-  SPX_HIP(hipMemcpyAsync(E->st_dev, E->st_host, sizeof(StepRec), hipMemcpyHostToDevice, s));
+  SPX_HIP(launch_step(E->st_dev, m, start_pos, 0, s));
   AttnArgs aa{};
   aa.q = q; aa.k = k; aa.v = v;
   aa.q_bias = ly.q_bias; aa.k_bias = ly.k_bias; aa.v_bias = ly.v_bias; aa.q_norm = ly.q_norm; aa.k_norm = ly.k_norm;
@@ -1886,7 +1906,8 @@ int spx_engine_destroy(spx_engine *E) {
   for (auto ev : E->ev_pool) (void)hipEventDestroy(ev);
   for (auto &kv : E->mats) spx_tensor_free(E->ctx, kv.second);
   for (void *p : E->allocs) (void)hipFree(p);
-  if (E->st_host) (void)hipHostFree(E->st_host);
+  for (void *h : {(void *)E->st_host, (void *)E->picks_host, (void *)E->hidden_host, (void *)E->logits_host})
+    if (h) (void)hipHostFree(h);
   if (E->perr_host) (void)hipHostFree(E->perr_host);
   delete E;
   return 0;

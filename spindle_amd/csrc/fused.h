@@ -178,7 +178,21 @@ struct DownArgs {
   float rscale;
 };
 
-hipError_t launch_embed(const TensorView &e, const StepRec *st, float escale, const NormTail &t, int m, hipStream_t s);
+// The pass's embedding rows (and their norm, t.nw set). src non-null (host memory, up to 16
+// rows): the pass's step record is read from there and left in st for the kernels after it.
+hipError_t launch_embed(const TensorView &e, StepRec *st, const StepRec *src, float escale, const NormTail &t, int m, hipStream_t s);
+// The step record of a call whose pass is not captured: m rows from position start (m == 1: of token tok).
+hipError_t launch_step(StepRec *st, int m, int start, int tok, hipStream_t s);
+// n floats (a multiple of 4) to host memory.
+hipError_t launch_to_host(const float *src, float *host, int64_t n, hipStream_t s);
+// Where a pass's last kernel leaves what the host reads (null: not left there): the picks, and rows of dim
+// values from rows on (the hidden states).
+struct HostOut {
+  int *picks;
+  float *hidden;
+  const float *rows;
+  int dim;
+};
 // mode 0: eight rows per wavefront (tiles); 1: row-parallel (integer only)
 hipError_t launch_mv(const MVArgs &a, int mt, int mode, const StepRec *st, int grid, hipStream_t s);
 hipError_t launch_attention(const AttnArgs &a, int m, const StepRec *st, hipStream_t s);
@@ -209,7 +223,7 @@ hipError_t launch_down(const DownArgs &a, int mt, int mode, const StepRec *st, h
 hipError_t launch_norm(const NormTail &t, const StepRec *st, int m, hipStream_t s);
 // hist non-null (m == 1): the pick advances the step record (next token and position) and is
 // appended to hist[step]
-hipError_t launch_argmax_final(const unsigned long long *best, int nbest, int *out, StepRec *st, int *hist, int m, hipStream_t s);
+hipError_t launch_argmax_final(const unsigned long long *best, int nbest, int *out, StepRec *st, int *hist, int m, const HostOut &ho, hipStream_t s);
 hipError_t launch_q8kp_quantize(const float *x, int64_t n, int64_t ld_x, int m, Q8KP out, hipStream_t s);
 hipError_t launch_q8kp_from_ref(const float *d, const int8_t *qs, const int16_t *bs, int64_t n, int m, Q8KP out, hipStream_t s);
 hipError_t launch_kq_block_sums(const TensorView &w, int expert, int64_t row, Q8KP y, int32_t *sums, hipStream_t s);

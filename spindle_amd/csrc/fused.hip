@@ -772,22 +772,43 @@ __global__ __launch_bounds__(64) void k_kq_block_sums(TensorView w, int expert, 
 // ------------------------------------------------------------------ embedding
 // dequant_row (quant.rs:1548-1660) of token rows, times embedding_scale (:3381-3388), into
 // t.x; then the row's norm tail (layer 0's attn_norm). One workgroup per row.
-__global__ __launch_bounds__(256) void k_embed(TensorView e, const StepRec *st, float escale, const NormTail t) {
+// (256 threads with a norm, up to 1024 without.) The step record of a captured pass comes from host
+// memory (src) with the ids that this kernel needs anyway, so a pass starts with no copy of its own.
+__global__ __launch_bounds__(1024) void k_embed(TensorView e, StepRec *st, const StepRec *src, float escale, const NormTail t) {
   const int b = blockIdx.x;
-  if (b >= st->m) return;
-  const int64_t tok = st->ids[b];
+  int m, tok;
+  if (src) {  // one thread's reads: a read of host memory is a trip over the bus for each wavefront that makes it
+    __shared__ int rec[2];
+    auto host = [](const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+    const bool one = b == 0 && threadIdx.x < MAX_M;  // the first workgroup also leaves the record for the pass
+    const int id = one ? host(&src->ids[threadIdx.x]) : threadIdx.x == 0 ? host(&src->ids[b]) : 0;
+    const int hm = threadIdx.x == 0 ? host(&src->m) : 0, hs = b == 0 && threadIdx.x == 0 ? host(&src->start) : 0;
+    if (one) st->ids[threadIdx.x] = id;
+    if (threadIdx.x == 0) {
+      if (b == 0) { st->m = hm; st->start = hs; st->step = 0; }
+      rec[0] = hm;
+      rec[1] = id;
+    }
+    __syncthreads();
+    m = rec[0];
+    tok = rec[1];
+  } else {
+    m = st->m;
+    tok = st->ids[b];
+  }
+  if (b >= m) return;
   const int64_t cols = e.cols;
   float *out = const_cast<float *>(t.x) + b * cols;
-  for (int64_t j = threadIdx.x; j < cols; j += 256) {
+  for (int64_t j = threadIdx.x; j < cols; j += blockDim.x) {
     float v = 0.0f;
     if (e.dtype == T_F32) {
-      v = reinterpret_cast<const float *>(e.pl.p0)[tok * cols + j];
+      v = reinterpret_cast<const float *>(e.pl.p0)[(int64_t)tok * cols + j];
     } else if (e.dtype == T_Q8_0) {
-      const int64_t g = tok * e.nb + j / 32;
+      const int64_t g = (int64_t)tok * e.nb + j / 32;
       const float dd = h2f(*reinterpret_cast<const uint16_t *>(e.pl.p3 + g * 2));
       v = (float)(int8_t)e.pl.p0[g * 32 + j % 32] * dd;
     } else if (e.dtype == T_Q5_0) {
-      const int64_t g = tok * e.nb + j / 32;
+      const int64_t g = (int64_t)tok * e.nb + j / 32;
       const int k = (int)(j % 32), l = k & 15;
       const float dd = h2f(*reinterpret_cast<const uint16_t *>(e.pl.p3 + g * 2));
       const uint32_t qh = *reinterpret_cast<const uint32_t *>(e.pl.p1 + g * 4);
@@ -796,7 +817,7 @@ __global__ __launch_bounds__(256) void k_embed(TensorView e, const StepRec *st, 
       const int q = nib | (int)(((qh >> k) & 1u) << 4);
       v = (float)(q - 16) * dd + 0.0f;
     } else if (e.dtype == T_Q4K) {  // element 64c + 32hi + t: byte qs[32c + t] (device offset 16(t/4) + 4c + t%4)
-      const int64_t g = tok * e.nb + j / 256;
+      const int64_t g = (int64_t)tok * e.nb + j / 256;
       const int k = (int)(j % 256), c = k / 64, tt = k % 32, hi = (k % 64) >= 32;
       const uint8_t *hd = e.pl.p1 + g * 16;
       const float dd = h2f(hd[0] | (hd[1] << 8)), dm = h2f(hd[2] | (hd[3] << 8));
@@ -809,7 +830,7 @@ __global__ __launch_bounds__(256) void k_embed(TensorView e, const StepRec *st, 
       const int q = hi ? (byte >> 4) : (byte & 0xF);
       v = dd * (float)sc * (float)q - dm * (float)mn;
     } else if (e.dtype == T_Q5K) {  // element 64c + 32h + t: qs[32c + t] (device 16(t%8) + 4c + t/8), qh[t] bit 2c+h
-      const int64_t g = tok * e.nb + j / 256;
+      const int64_t g = (int64_t)tok * e.nb + j / 256;
       const int k = (int)(j % 256), c = k / 64, tt = k % 32, hi = (k % 64) >= 32;
       const uint8_t *hd = e.pl.p2 + g * 16;
       const float dd = h2f(hd[0] | (hd[1] << 8)), dm = h2f(hd[2] | (hd[3] << 8));
@@ -823,7 +844,7 @@ __global__ __launch_bounds__(256) void k_embed(TensorView e, const StepRec *st, 
       const int q = (hi ? (byte >> 4) : (byte & 0xF)) | (((qhb >> jj) & 1) << 4);
       v = dd * (float)sc * (float)q - dm * (float)mn;
     } else if (e.dtype == T_Q6K) {  // element 128h + 32mq + t
-      const int64_t g = tok * e.nb + j / 256;
+      const int64_t g = (int64_t)tok * e.nb + j / 256;
       const int k = (int)(j % 256), h = k / 128, r = k % 128, mq = r / 32, tt = r % 32;
       const int lb = 16 * (tt >> 2) + 8 * h + 4 * (mq & 1) + (tt & 3);
       const int hb = 8 * (tt >> 2) + 4 * h + (tt & 3);
@@ -2568,9 +2589,13 @@ __global__ __launch_bounds__(256) void k_down_f(const DownArgs a, const StepRec 
 // ------------------------------------------------------------------ final greedy pick
 // With hist (one-row decode passes replayed back to back): the pick also becomes the next
 // pass's token at the next position, and is appended to hist.
-__global__ __launch_bounds__(256) void k_argmax_final(const unsigned long long *best, int nbest, int *out, StepRec *st, int *hist) {
+// What the host reads of a pass goes straight to its memory (ho): the picks and the hidden rows.
+__global__ __launch_bounds__(256) void k_argmax_final(const unsigned long long *best, int nbest, int *out, StepRec *st, int *hist, const HostOut ho) {
   const int b = blockIdx.x;
   if (st && b >= st->m) return;
+  if (ho.hidden)
+    for (int i = threadIdx.x; i < ho.dim / 4; i += 256)
+      reinterpret_cast<float4 *>(ho.hidden + (int64_t)b * ho.dim)[i] = reinterpret_cast<const float4 *>(ho.rows + (int64_t)b * ho.dim)[i];
   unsigned long long v = 0;
   for (int i = threadIdx.x; i < nbest; i += 256) { const unsigned long long w = best[(int64_t)b * nbest + i]; v = w > v ? w : v; }
   v = wave_max_u64(v);
@@ -2582,6 +2607,7 @@ __global__ __launch_bounds__(256) void k_argmax_final(const unsigned long long *
     for (int w = 1; w < 4; w++) r = sb[w] > r ? sb[w] : r;
     const int tok = (int)(uint32_t)(r & 0xffffffffull);
     out[b] = tok;
+    if (ho.picks) ho.picks[b] = tok;
     if (hist) {
       hist[st->step] = tok;
       st->step += 1;
@@ -2589,6 +2615,15 @@ __global__ __launch_bounds__(256) void k_argmax_final(const unsigned long long *
       st->start += 1;
     }
   }
+}
+
+__global__ __launch_bounds__(64) void k_step(StepRec *st, int m, int start, int tok) {
+  if (threadIdx.x == 0) { st->m = m; st->start = start; st->step = 0; st->ids[0] = tok; }
+}
+
+__global__ __launch_bounds__(256) void k_to_host(const float *src, float *host, int64_t n4) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)gridDim.x * 256)
+    reinterpret_cast<float4 *>(host)[i] = reinterpret_cast<const float4 *>(src)[i];
 }
 
 // ------------------------------------------------------------------ launchers
@@ -2954,8 +2989,23 @@ hipError_t launch_down(const DownArgs &a, int mt, int mode, const StepRec *st, h
   }
 }
 
-hipError_t launch_embed(const TensorView &e, const StepRec *st, float escale, const NormTail &t, int m, hipStream_t s) {
-  hipLaunchKernelGGL(k_embed, dim3(m), dim3(256), 0, s, e, st, escale, t);
+hipError_t launch_embed(const TensorView &e, StepRec *st, const StepRec *src, float escale, const NormTail &t, int m, hipStream_t s) {
+  // without a norm two values a thread (2048 columns of Q4_K: 9.0 us with 256 threads, a chain of
+  // eight dependent rounds of byte loads)
+  const int nt = t.nw ? 256 : (int)std::min<int64_t>(1024, std::max<int64_t>(256, (e.cols / 2 + 63) / 64 * 64));
+  if (src && m > MAX_M) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_embed, dim3(m), dim3(nt), 0, s, e, st, src, escale, t);
+  return hipGetLastError();
+}
+
+hipError_t launch_step(StepRec *st, int m, int start, int tok, hipStream_t s) {
+  hipLaunchKernelGGL(k_step, dim3(1), dim3(64), 0, s, st, m, start, tok);
+  return hipGetLastError();
+}
+
+hipError_t launch_to_host(const float *src, float *host, int64_t n, hipStream_t s) {
+  if (n < 4 || n % 4) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_to_host, dim3((unsigned)std::min<int64_t>((n / 4 + 255) / 256, 512)), dim3(256), 0, s, src, host, n / 4);
   return hipGetLastError();
 }
 
@@ -2964,9 +3014,9 @@ hipError_t launch_norm(const NormTail &t, const StepRec *st, int m, hipStream_t 
   return hipGetLastError();
 }
 
-hipError_t launch_argmax_final(const unsigned long long *best, int nbest, int *out, StepRec *st, int *hist, int m, hipStream_t s) {
-  if (hist && m != 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_argmax_final, dim3(m), dim3(256), 0, s, best, nbest, out, st, hist);
+hipError_t launch_argmax_final(const unsigned long long *best, int nbest, int *out, StepRec *st, int *hist, int m, const HostOut &ho, hipStream_t s) {
+  if ((hist && m != 1) || (ho.hidden && ho.dim % 4)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_argmax_final, dim3(m), dim3(256), 0, s, best, nbest, out, st, hist, ho);
   return hipGetLastError();
 }
 
