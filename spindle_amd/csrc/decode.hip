@@ -1674,6 +1674,99 @@ __device__ __forceinline__ void ms_prod(const SPX_L uint8_t *tl, const MwDst &d,
     }
   }
 }
+// All eight classes' chains of a tile advance by one block: ms_prod's integers and mw_chain's fp32
+// steps, four classes at a time, so that at most half of the integers are in registers (a walk in
+// 128 registers, four wavefronts a SIMD).
+template <int T, bool Q6>
+__device__ __forceinline__ void ms_step(const SPX_L uint8_t *tl, const MwDst &d, int b, float (&acc)[8][4], float (&cr)[4]) {
+  using G = MsGeo<1, Q6>;
+  constexpr int CG = 4;
+  const int lane = threadIdx.x & 63, k4 = lane >> 4, c16 = lane & 15;
+  const SPX_L uint32_t *py = d.py + b * 64, *pw = d.pw + b * MQ_CW;
+  const SPX_L uint8_t *rc = tl + G::OC + c16 * G::CR, *rs = tl + G::OS + c16 * G::SR;
+  const uint32_t dw = lld<uint32_t>((const SPX_L uint32_t *)(tl + G::OD + 4 * c16));
+  float xd[4], dx[4];
+  const float dd = h2f(dw);
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    xd[t] = d.px[t][b];
+    dx[t] = dd * xd[t];
+  }
+  auto chain = [&](int l, const mq_v4i &P) SPX_AI {
+#pragma unroll
+    for (int t = 0; t < 4; t++) acc[l][t] = fmaf(dx[t], (float)P[t], acc[l][t]);
+  };
+  if constexpr (T == T_Q4K) {
+    {
+      const uint2 mn = lld<uint2>((const SPX_L uint2 *)(rs + 8));
+      const uint2 cw = lld<uint2>(pw + 8 + 2 * (k4 & 1));
+      const uint32_t a0 = k4 < 2 ? cw.x : 0u, a1 = k4 < 2 ? cw.y : 0u;
+      const mq_v4i C = mq_mfma_c(a0, a1, mn.x, mn.y, mq_mfma(k4 == 1 ? a0 : 0u, k4 == 1 ? a1 : 0u, mn.x, mn.y) * 63);
+      const float dm = h2f(dw >> 16);
+#pragma unroll
+      for (int t = 0; t < 4; t++) cr[t] = cr[t] + (dm * xd[t]) * (float)C[t];
+    }
+    const uint32_t sp = lld<uint16_t>((const SPX_L uint16_t *)(rs + 2 * k4));
+    const uint32_t s0 = sp & 0xFFu, s1 = (sp >> 8) & 0xFFu;
+    const uint32_t lo0 = s0 & 7u, hi0 = s0 >> 3, lo1 = s1 & 7u, hi1 = s1 >> 3;
+#pragma unroll
+    for (int j0 = 0; j0 < 8; j0 += CG) {
+      uint32_t c0[CG], c1[CG];
+      uint2 y[CG];
+      mq_v4i P[CG];
+#pragma unroll
+      for (int q = 0; q < CG; q++) {
+        const uint32_t wl = lld<uint32_t>((const SPX_L uint32_t *)(rc + 16 * (j0 + q) + 4 * k4));
+        c0[q] = wl & 0x0F0F0F0Fu;
+        c1[q] = (wl >> 4) & 0x0F0F0F0Fu;
+        y[q] = lld<uint2>(py + 8 * (j0 + q));
+      }
+#pragma unroll
+      for (int q = 0; q < CG; q++) P[q] = mq_mfma(y[q].x, y[q].y, mx_pmul(c0[q], hi0), mx_pmul(c1[q], hi1)) * 8;
+#pragma unroll
+      for (int q = 0; q < CG; q++) P[q] = mq_mfma_c(y[q].x, y[q].y, mx_pmul(c0[q], lo0), mx_pmul(c1[q], lo1), P[q]);
+#pragma unroll
+      for (int q = 0; q < CG; q++) chain(j0 + q, P[q]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    const SPX_L uint8_t *rh = tl + G::OH + c16 * G::HR;
+    const int h = k4 >> 1, sh = 4 * (k4 & 1);
+    {
+      const uint2 bb = lld<uint2>((const SPX_L uint2 *)(rs + 8 * (k4 & 1)));
+      const uint2 cw = lld<uint2>(pw + 2 * k4);
+      const bool lo = k4 < 2;
+      const mq_v4i C = mq_mfma_c(cw.x, cw.y, bb.x, bb.y, mq_mfma(lo ? 0u : cw.x, lo ? 0u : cw.y, bb.x, bb.y) * 63) * 32;
+#pragma unroll
+      for (int t = 0; t < 4; t++) cr[t] = cr[t] + dx[t] * (float)C[t];
+    }
+    const uint32_t sw = lld<uint32_t>((const SPX_L uint32_t *)(rs + 4 * k4));
+#pragma unroll
+    for (int j0 = 0; j0 < 8; j0 += CG) {
+      uint32_t wl0[CG], wl1[CG];
+      uint2 y[CG];
+      mq_v4i P[CG];
+#pragma unroll
+      for (int q = 0; q < CG; q++) {
+        const int l = j0 + q, hb = l >= 4 ? 8 : 0;
+        const uint2 ql = lld<uint2>((const SPX_L uint2 *)(rc + 16 * l + 8 * h));
+        const uint32_t qh = lld<uint32_t>((const SPX_L uint32_t *)(rh + 8 * l + 4 * h));
+        const uint32_t c0 = ((ql.x >> sh) & 0x0F0F0F0Fu) | (((qh >> sh) & 0x03030303u) << 4);
+        const uint32_t c1 = ((ql.y >> sh) & 0x0F0F0F0Fu) | (((qh >> (sh + 2)) & 0x03030303u) << 4);
+        uint32_t h0, h1;
+        q6_wsplit(c0, (uint32_t)(uint16_t)(int16_t)(int8_t)(sw >> hb), h0, wl0[q]);
+        q6_wsplit(c1, (uint32_t)(uint16_t)(int16_t)(int8_t)(sw >> (16 + hb)), h1, wl1[q]);
+        y[q] = lld<uint2>(py + 8 * l);
+        P[q] = mq_mfma(y[q].x, y[q].y, h0, h1) * 128;
+      }
+#pragma unroll
+      for (int q = 0; q < CG; q++) P[q] = mq_mfma_c(y[q].x, y[q].y, wl0[q], wl1[q], P[q]);
+#pragma unroll
+      for (int q = 0; q < CG; q++) chain(j0 + q, P[q]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
 // Part C's chains over a staged tile's NB blocks (integers of BB blocks issued together).
 template <int NB, int TT, int WPT, int C>
 __device__ __forceinline__ void ms_tile(const SPX_L uint8_t *tl, int dt, const MwDst &d, float (&part)[4], float (&cr)[4]) {
@@ -1795,8 +1888,9 @@ constexpr int WS_BYTES = MsGeo<1, TT != T_Q4K>::BYTES;  // a wavefront's LDS
 __host__ __device__ inline size_t ws_bytes(int tt) { return tt == T_Q4K ? WS_BYTES<T_Q4K> : WS_BYTES<0>; }
 
 // The walk of one wavefront over its tiles 0 .. ntiles - 1, all eight classes: tile i's bytes from src(i), its vectors from dst(i), done(i, out) with the tile's
-// results (matrix row lane & 15, vector 4 (lane >> 4) + t). tl: the wavefront's WS_BYTES.
-template <int NB, int TT, class Src, class Dst, class Done>
+// results (matrix row lane & 15, vector 4 (lane >> 4) + t). tl: the wavefront's WS_BYTES. SMALL: one
+// block's loads in flight instead of two, ms_step's registers: four wavefronts a SIMD.
+template <int NB, int TT, bool SMALL = false, class Src, class Dst, class Done>
 __device__ __forceinline__ void ws_walk(SPX_L uint8_t *tl, int ntiles, Src src, Dst dst, Done done) {
   if (ntiles <= 0) return;
   WsRaw<NB, TT> ra, rb;
@@ -1823,10 +1917,15 @@ __device__ __forceinline__ void ws_walk(SPX_L uint8_t *tl, int ntiles, Src src, 
   auto step = [&](WsRaw<NB, TT> &r) SPX_AI {
     r.put(tl, dc.dt);
     fetch(r);
-    MwProd<1> pr;
-    if (TT == T_Q4K || (TT == 0 && dc.dt == T_Q4K)) ms_prod<T_Q4K, 1, TT != T_Q4K, 1, 0>(tl, dc, b, 0, pr);
-    else ms_prod<T_Q6K, 1, true, 1, 0>(tl, dc, b, 0, pr);
-    mw_chain<1, 0>(pr, acc, cr);
+    if constexpr (SMALL) {
+      if (TT == T_Q4K || (TT == 0 && dc.dt == T_Q4K)) ms_step<T_Q4K, TT != T_Q4K>(tl, dc, b, acc, cr);
+      else ms_step<T_Q6K, true>(tl, dc, b, acc, cr);
+    } else {
+      MwProd<1> pr;
+      if (TT == T_Q4K || (TT == 0 && dc.dt == T_Q4K)) ms_prod<T_Q4K, 1, TT != T_Q4K, 1, 0>(tl, dc, b, 0, pr);
+      else ms_prod<T_Q6K, 1, true, 1, 0>(tl, dc, b, 0, pr);
+      mw_chain<1, 0>(pr, acc, cr);
+    }
     if (++b < NB) return;
     b = 0;
     float out[4];
@@ -1839,12 +1938,14 @@ __device__ __forceinline__ void ws_walk(SPX_L uint8_t *tl, int ntiles, Src src, 
   };
   clear();
   fetch(ra);
-  fetch(rb);
+  if (!SMALL) fetch(rb);
   for (;;) {
     step(ra);
     if (i >= ntiles) break;
-    step(rb);
-    if (i >= ntiles) break;
+    if (!SMALL) {
+      step(rb);
+      if (i >= ntiles) break;
+    }
   }
 }
 
@@ -2211,15 +2312,23 @@ __global__ __launch_bounds__(256) void kp_moe_combine(const float *yd, const flo
   gst<float>(y + (int64_t)b * ld_y + i, nk > 0 ? acc : __int_as_float(0x7fc00000));
 }
 
-// Gate / up + SwiGLU of a prefill pass on the matrix cores over a job list of at most sixteen
-// users a job (MoE: kp_route's, in global memory; dense, jobs null: rows 16j .. 16j + 15 as
-// job j): items (job, 16 h rows), workgroup b the items
-// [b n / G, (b + 1) n / G), job by job: the job's users' Q8_K rows are staged in LDS (slot =
-// the user's place in the job), then wavefront w walks the job's items w, w + NW, ... of the
-// range (ws_walk). Each h value has the bits of kd_gateup_mqs's.
+// Gate / up + SwiGLU over a job list of at most sixteen users a job on the matrix cores (prefill
+// passes and spx_moe_dev: kp_route's / kp_jobs' list in global memory; dense, jobs null: rows
+// 16j .. 16j + 15 as job j). Workgroup: KP_CH items (16 h rows each) of one job; the job's users'
+// Q8_K rows are staged in LDS (slot = the user's place in the job), then each wavefront walks one
+// tile, the items' gate tiles on wavefronts 0 .. KP_CH - 1 and their up tiles on the rest; the up
+// results go through LDS to the gate's wavefront. Each h value has the bits of kd_gateup_mqs's.
+// A tile's walk is a chain (a block's load, its LDS turn, ~200 vector instructions), so what bounds
+// this is how many walks a CU has under way, not the matrix cores: two workgroups a CU (128
+// registers, 62 KB of LDS at 2048 columns) and more workgroups than slots, so that one's staging runs
+// beside another's walk and the last round is short. One workgroup a CU with two blocks in flight a
+// wavefront, each walking gate and up of every eighth item of a contiguous range: 58.7 us a 128-row
+// layer of 768 x 2048 Q4_K experts, 42.7 us for nine rows; two a CU 48.6 and 35.6; a tile a
+// wavefront 48.3 and 30.8. (The same sums as f16 contractions, a third fewer vector
+// instructions but twice the LDS and so one workgroup a CU: 56.9 and 41.2.)
+constexpr int KP_CH = DEC_MM_NW / 2;
 template <int T, int NB>
-__global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void kp_gateup_mq(const DecGateUpMArgs a,
-                                                                                                     const Job *jobs,
+__global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void kp_gateup_mq(const DecGateUpMArgs a, const Job *jobs,
                                                                                                      const int *njobs) {
   constexpr int NW = DEC_MM_NW, JR = 2 + 2 * MAX_M;
   extern __shared__ __align__(16) uint8_t smem[];
@@ -2230,45 +2339,43 @@ __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(
   const MwLds L = mw_lds(smem, MAX_M, nb);
   SPX_L uint8_t *tl = (SPX_L uint8_t *)(smem + mw_tail_off(MAX_M, nb)) + wave * WS_BYTES<T>;  // (over lbs, once lc is built)
   const int nj = jobs ? gld<int>(njobs) : (m + MAX_M - 1) / MAX_M;
-  const int n = TX * nj, G = gridDim.x;
-  const int i0 = (int)((int64_t)blockIdx.x * n / G), i1 = (int)((int64_t)(blockIdx.x + 1) * n / G);
-  for (int s0 = i0; s0 < i1;) {
-    const int j = s0 / TX, s1 = min(i1, (j + 1) * TX);
-    __syncthreads();  // the previous job's users are done with
-    if ((int)threadIdx.x < JR) {
-      const int f = threadIdx.x;
-      sj[f] = jobs ? gld<int>(reinterpret_cast<const int *>(jobs + j) + f)
-                   : f == 0 ? 0 : f == 1 ? min(MAX_M, m - MAX_M * j) : MAX_M * j + (f - 2) % MAX_M;
-    }
-    __syncthreads();
-    const int nv = __builtin_amdgcn_readfirstlane(min(max(sj[1], 0), MAX_M));
-    const int e = __builtin_amdgcn_readfirstlane(min(max(sj[0], 0), a.gate.n_expert - 1));
-    stage_q8<NW * 64>(a.y, (const SPX_L int *)(sj + 2), nv, cols, L.lq, L.ld, L.lbs, mw_vs(nb) / 4);
-    __syncthreads();
-    mq_corr_stage(nv, nb, L.lbs, L.lc);
-    __syncthreads();
-    const int cnt = s1 - s0, nit = wave < cnt ? (cnt - wave + NW - 1) / NW : 0;
-    const MqVec vv = mq_vecs(nv, MqIdentity{});
-    float g[4];
-    auto src = [&](int k) SPX_AI {  // tile k: item s0 + wave + NW (k / 2), gate (k even) or up
-      const int x = s0 + wave + NW * (k >> 1) - j * TX;
-      return ws_src((k & 1) ? a.up.pl : a.gate.pl, T, (int64_t)e * a.gate.rows + (int64_t)x * 16, min(16, n_ff - x * 16), NB);
-    };
-    auto dst = [&](int) SPX_AI { return mw_dst(L, vv, NB, T); };
-    auto done = [&](int k, const float (&out)[4]) SPX_AI {
+  const int nch = (TX + KP_CH - 1) / KP_CH, j = (int)blockIdx.x / nch;
+  if (j >= nj) return;
+  if ((int)threadIdx.x < JR) {
+    const int f = threadIdx.x;
+    sj[f] = jobs ? gld<int>(reinterpret_cast<const int *>(jobs + j) + f)
+                 : f == 0 ? 0 : f == 1 ? min(MAX_M, m - MAX_M * j) : MAX_M * j + (f - 2) % MAX_M;
+  }
+  __syncthreads();
+  const int nv = __builtin_amdgcn_readfirstlane(min(max(sj[1], 0), MAX_M));
+  const int e = __builtin_amdgcn_readfirstlane(min(max(sj[0], 0), a.gate.n_expert - 1));
+  stage_q8<NW * 64>(a.y, (const SPX_L int *)(sj + 2), nv, cols, L.lq, L.ld, L.lbs, mw_vs(nb) / 4);
+  __syncthreads();
+  mq_corr_stage(nv, nb, L.lbs, L.lc);
+  __syncthreads();
+  const MqVec vv = mq_vecs(nv, MqIdentity{});
+  const int it = wave % KP_CH, x = ((int)blockIdx.x - j * nch) * KP_CH + it;
+  const bool up = wave >= KP_CH;
+  float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto src = [&](int) SPX_AI { return ws_src(up ? a.up.pl : a.gate.pl, T, (int64_t)e * a.gate.rows + (int64_t)x * 16, min(16, n_ff - x * 16), NB); };
+  auto dst = [&](int) SPX_AI { return mw_dst(L, vv, NB, T); };
+  auto done = [&](int, const float (&out)[4]) SPX_AI {
 #pragma unroll
-      for (int t = 0; t < 4; t++)
-        if (!(k & 1)) g[t] = out[t];
-      if (!(k & 1)) return;
-      const int x = s0 + wave + NW * (k >> 1) - j * TX, r = lane & 15;
+    for (int t = 0; t < 4; t++) o[t] = out[t];
+  };
+  ws_walk<NB, T, true>(tl, x < TX ? 1 : 0, src, dst, done);
+  SPX_L float *xu = (SPX_L float *)(smem + mw_tail_off(MAX_M, nb)) + it * 256;
+  __syncthreads();  // every walk has read its LDS
+  if (up)
 #pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const int v = 4 * (lane >> 4) + t;
-        if (v < nv && x * 16 + r < n_ff) gst<float>(a.h + (int64_t)sj[2 + MAX_M + v] * n_ff + x * 16 + r, g[t] / (1.0f + expf(-g[t])) * out[t]);
-      }
-    };
-    ws_walk<NB, T>(tl, 2 * nit, src, dst, done);
-    s0 = s1;
+    for (int t = 0; t < 4; t++) xu[t * 64 + lane] = o[t];
+  __syncthreads();
+  if (up || x >= TX) return;
+  const int r = x * 16 + (lane & 15);
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    const int v = 4 * (lane >> 4) + t;
+    if (v < nv && r < n_ff) gst<float>(a.h + (int64_t)sj[2 + MAX_M + v] * n_ff + r, o[t] / (1.0f + expf(-o[t])) * xu[t * 64 + lane]);
   }
 }
 
@@ -2668,8 +2775,8 @@ hipError_t launch_kp_gateup_mq(const DecGateUpMArgs &a, const Job *jobs, const i
       max_jobs < 1 || max_jobs > 512 || (jobs && !njobs))
     return hipErrorInvalidValue;
   const size_t sm = mw_tail_off(MAX_M, nb) + std::max((size_t)MAX_M * nb * 64, DEC_MM_NW * ws_bytes(a.gate.dtype));
-  const int njob = jobs ? max_jobs : (a.m + MAX_M - 1) / MAX_M, items = ((a.n_ff + 15) / 16) * njob;
-  const dim3 grid((unsigned)std::max(1, std::min((items + DEC_MM_NW - 1) / DEC_MM_NW, cu_count()))), b(DEC_MM_NW * 64);
+  const int njob = jobs ? max_jobs : (a.m + MAX_M - 1) / MAX_M, nch = ((a.n_ff + 15) / 16 + KP_CH - 1) / KP_CH;
+  const dim3 grid((unsigned)(nch * njob)), b(DEC_MM_NW * 64);
   if (a.gate.dtype != T_Q4K && a.gate.dtype != T_Q6K) return hipErrorInvalidValue;
   return with_nb(nb, [&](auto NBc) {
     constexpr int NB = decltype(NBc)::value;

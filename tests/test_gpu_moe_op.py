@@ -121,3 +121,23 @@ def test_moe_dev_bad_rows_nan(ctx):
     good = ops.moe_dev(ctx, ex["gate"][1], ex["up"][1], ex["down"][1], x[[0, 3]], torch.from_numpy(chosen[[0, 3]]).cuda(),
                        torch.from_numpy(weights[[0, 3]]).cuda()).cpu().numpy()
     assert np.array_equal(good.view(np.uint32), y[[0, 3]].view(np.uint32))
+
+
+@pytest.mark.parametrize("fmt", [(R.Q4K, R.Q6K), (R.Q6K, R.Q4K)], ids=["q4k-q6k", "q6k-q4k"])
+@pytest.mark.parametrize("dim,nff,ne,k,m", [(2048, 768, 4, 2, 40), (256, 1024, 256, 32, 3), (1024, 512, 2, 1, 33), (4096, 256, 3, 3, 16)])
+def test_moe_dev_job_edges(ctx, fmt, dim, nff, ne, k, m):
+    """Experts of more than sixteen users (a job of sixteen and one of the rest), of exactly one job's
+    sixteen, of one user; rows of 1, 4, 8 and 16 blocks; every expert chosen by a row: the bits of
+    spx_moe on the same rows, sixteen a call or fewer."""
+    from spindle_amd import ops
+    ex = _experts(ctx, fmt[0], fmt[1], dim, nff, ne, seed=dim + m)
+    rng = np.random.default_rng(nff + m)
+    x = torch.from_numpy(rng.standard_normal((m, dim)).astype(np.float32)).cuda()
+    chosen = np.stack([rng.permutation(ne)[:k] for _ in range(m)]).astype(np.int32)
+    weights = rng.dirichlet(np.ones(k), m).astype(np.float32)
+    mats = [ex[n][1] for n in ("gate", "up", "down")]
+    y = ops.moe_dev(ctx, *mats, x, torch.from_numpy(chosen).cuda(), torch.from_numpy(weights).cuda()).cpu().numpy()
+    step = min(16, 256 // k)
+    for a in range(0, m, step):
+        want = ops.moe(ctx, *mats, x[a:a + step].contiguous(), chosen[a:a + step], weights[a:a + step]).cpu().numpy()
+        assert np.array_equal(want.view(np.uint32), y[a:a + step].view(np.uint32)), a
