@@ -617,9 +617,9 @@ extern "C" int spx_moe(spx_ctx *ctx, const spx_tensor *gate, const spx_tensor *u
   return 0;
 }
 
-// The routed experts with the routing in device memory: nothing waits on the host. The routing
-// goes into the pipeline's layout (kp_moe_in), the job list is built on the device (kp_jobs: at
-// most 16 users a job), x is quantized to Q8_K, and the prefill pass's grouped kernels run on
+// The routed experts with the routing in device memory: nothing waits on the host. One launch checks
+// the routing, builds its job list (at most 16 users a job) and quantizes x to Q8_K (kp_moe_front),
+// and the prefill pass's grouped kernels run on
 // the int8 matrix cores (kp_gateup_mq, kp_down_mq or kd_down_m: the reference's per-lane integer dots and fp32
 // chains); kp_moe_combine sums each row's choices in order.
 extern "C" int spx_moe_dev(spx_ctx *ctx, const spx_tensor *gate, const spx_tensor *up, const spx_tensor *down, const float *x,
@@ -639,24 +639,22 @@ extern "C" int spx_moe_dev(spx_ctx *ctx, const spx_tensor *gate, const spx_tenso
   const int nv = m * k, max_jobs = std::min(512, std::min(ne, nv) + nv / MAX_M);
   size_t yq_b = 0;
   (void)q8kp_layout(nullptr, m, dim, &yq_b);
-  const size_t sz[8] = {al256(sizeof(int) * m * 32), al256(sizeof(float) * m * 32), al256(sizeof(int) * m), al256(sizeof(Job) * max_jobs),
+  const size_t sz[7] = {al256(sizeof(float) * m * 32), al256(sizeof(int) * m), al256(sizeof(Job) * max_jobs),
                         al256(sizeof(int) * 4), al256(yq_b), al256(sizeof(float) * nv * n_ff), al256(sizeof(float) * nv * dim)};
   size_t tot = 0;
   for (size_t v : sz) tot += v;
   uint8_t *w = static_cast<uint8_t *>(ws_get(ctx, tot));
   if (!w) return fail("spx_moe_dev: workspace allocation failed");
-  uint8_t *p[8];
-  for (int i = 0, o = 0; i < 8; o += (int)sz[i], i++) p[i] = w + o;
-  int *ch32 = reinterpret_cast<int *>(p[0]), *nkeep = reinterpret_cast<int *>(p[2]), *njobs = reinterpret_cast<int *>(p[4]);
-  float *w32 = reinterpret_cast<float *>(p[1]), *h = reinterpret_cast<float *>(p[6]), *yd = reinterpret_cast<float *>(p[7]);
-  Job *jobs = reinterpret_cast<Job *>(p[3]);
+  uint8_t *p[7];
+  for (int i = 0, o = 0; i < 7; o += (int)sz[i], i++) p[i] = w + o;
+  int *nkeep = reinterpret_cast<int *>(p[1]), *njobs = reinterpret_cast<int *>(p[3]);
+  float *w32 = reinterpret_cast<float *>(p[0]), *h = reinterpret_cast<float *>(p[5]), *yd = reinterpret_cast<float *>(p[6]);
+  Job *jobs = reinterpret_cast<Job *>(p[2]);
   hipStream_t s = ctx->stream;
-  SPX_HIP(launch_kp_moe_in(chosen, weights, m, k, ne, ch32, w32, nkeep, s));
   DecRouteArgs rt{};
-  rt.n_expert = ne; rt.n_used = k; rt.m = m; rt.chosen = ch32; rt.weights = w32; rt.nkeep = nkeep; rt.jobs = jobs; rt.njobs = njobs;
-  SPX_HIP(launch_kp_jobs(rt, s));
-  const Q8KP yq = q8kp_layout(p[5], m, dim, &yq_b);
-  SPX_HIP(launch_q8kp_quantize(x, dim, ld_x, m, yq, s));
+  rt.n_expert = ne; rt.n_used = k; rt.m = m; rt.weights = w32; rt.nkeep = nkeep; rt.jobs = jobs; rt.njobs = njobs;
+  const Q8KP yq = q8kp_layout(p[4], m, dim, &yq_b);
+  SPX_HIP(launch_kp_moe_front(rt, chosen, weights, x, ld_x, (int)dim, yq, s));
   DecGateUpMArgs ga{};
   ga.gate = gate->v; ga.up = up->v; ga.y = yq; ga.h = h; ga.n_ff = (int)n_ff; ga.m = m;
   SPX_HIP(launch_kp_gateup_mq(ga, jobs, njobs, max_jobs, s));

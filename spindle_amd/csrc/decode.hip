@@ -1288,10 +1288,6 @@ __device__ __forceinline__ int mq_sbyte(uint4 v, int i) { return (int)(int8_t)mq
 struct MqIdentity {
   __device__ __forceinline__ int operator()(int v) const { return v; }
 };
-struct MqRows {
-  const SPX_L int *r;
-  __device__ __forceinline__ int operator()(int v) const { return r[v]; }
-};
 
 // The correction operands of the MFMA path, per (vector, 256-block) 12 words next to the Q8_K
 // image: the sixteen 16-element bsums split as bs = 64 hi + lo (lo = bs & 63, hi = bs >> 6:
@@ -2107,19 +2103,17 @@ __global__ __launch_bounds__(MW_NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
   }
 }
 
-// Routing + gate/up + SwiGLU over the jobs on the matrix cores (kd_gateup_m's prologue and job
-// list) on staged tiles: items (job, 16 h rows), rounds of two items' gate tiles, then their up
+// Dense gate/up + SwiGLU of up to 16 rows on the matrix cores on staged tiles: items of 16 h rows,
+// rounds of two items' gate tiles, then their up
 // tiles (MsLoad: a round's bytes come into LDS at once, the next round's loads fly during this one); wavefronts
 // 0-3 take the first item's tile, 4-7 the second's, a quarter of the lane classes each, their
 // partial sums meeting in LDS; part 0 applies SwiGLU. Workgroup b takes item pairs b, b + G, ...
 template <int T, int NB>
 __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void kd_gateup_mqs(const DecGateUpMArgs a) {
-  constexpr int NW = DEC_MM_NW, JR = 2 + 2 * MAX_M;
+  constexpr int NW = DEC_MM_NW;
   static_assert(NW == 8, "two items of four wavefronts");
   using G = MsGeo<NB, T == T_Q6K>;
   extern __shared__ __align__(16) uint8_t smem[];
-  __shared__ signed char slot_of[MAX_M * 256];
-  __shared__ int wcount[NW];
   __shared__ float xch[2][NW][4][64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int g = wave >> 2, c = wave & 3;
@@ -2127,26 +2121,14 @@ __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(
   const int TX = (n_ff + 15) / 16;
   const MwLds L = mw_lds(smem, m, NB);
   SPX_L uint8_t *tl = (SPX_L uint8_t *)(smem + mw_tail_off(m, NB));  // (over lbs, once lc is built)
-  SPX_L int *sj = (SPX_L int *)(smem + mw_tail_off(m, NB) + (((size_t)std::max(m * NB * 64, 2 * G::BYTES) + 15) & ~(size_t)15));
-  int nj = 1;
   StageQ8<NW * 64> st;
-  if (a.rt.logits) {
-    float lv[2][4];
-    route_load<NW>(a.rt, lv);
-    st.get(a.y, m, cols);
-    nj = route_jobs<NW>(a.rt, lv, sj, (SPX_L signed char *)slot_of, (SPX_L int *)wcount, blockIdx.x == 0);
-  } else {
-    st.get(a.y, m, cols);
-    for (int i = threadIdx.x; i < JR; i += blockDim.x) sj[i] = i == 0 ? 0 : i == 1 ? m : i < 2 + MAX_M ? i - 2 : i - 2 - MAX_M;
-    __syncthreads();
-  }
-  const int n = TX * nj, R = gridDim.x, np = (n + 1) / 2, nr = (int)blockIdx.x < np ? (np - (int)blockIdx.x + R - 1) / R : 0;
+  st.get(a.y, m, cols);
+  const int n = TX, R = gridDim.x, np = (n + 1) / 2, nr = (int)blockIdx.x < np ? (np - (int)blockIdx.x + R - 1) / R : 0;
   // round k: item pair blockIdx.x + R (k / 2), gate (k even) or up tiles
   auto item = [&](int k, int u) SPX_AI { return min(2 * ((int)blockIdx.x + R * (k >> 1)) + u, n - 1); };
   auto msrc = [&](int k, int u) SPX_AI {
-    const int i = item(k, u), j = i / TX, x = i - j * TX;
-    const int e = __builtin_amdgcn_readfirstlane(min(max(sj[j * JR], 0), a.gate.n_expert - 1));
-    return MsSrc{(k & 1) ? a.up.pl : a.gate.pl, (int64_t)e * a.gate.rows + (int64_t)x * 16, min(16, n_ff - x * 16)};
+    const int x = item(k, u);
+    return MsSrc{(k & 1) ? a.up.pl : a.gate.pl, (int64_t)x * 16, min(16, n_ff - x * 16)};
   };
   MsLoad<NB, NW * 64, T == T_Q6K, 2> ld;
   if (nr > 0) ld.get(T, msrc(0, 0), msrc(0, 1));
@@ -2154,14 +2136,15 @@ __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(
   __syncthreads();
   mq_corr_stage(m, NB, L.lbs, L.lc);
   __syncthreads();  // lbs read: the tiles may take its place
+  const MqVec vv = mq_vecs(m, MqIdentity{});
   float gv[4];
   for (int k = 0; k < 2 * nr; k++) {
     ld.put(tl, T);
     __syncthreads();
     if (k + 1 < 2 * nr) ld.get(T, msrc(k + 1, 0), msrc(k + 1, 1));
-    const int i = item(k, g), j = i / TX, x = i - j * TX;
+    const int x = item(k, g);
     float part[4], cr[4], out[4];
-    ms_tile_part<NB, T, 4>(c, tl + g * G::BYTES, T, mw_dst(L, mq_vecs(sj[j * JR + 1], MqRows{sj + j * JR + 2}), NB, T), part, cr);
+    ms_tile_part<NB, T, 4>(c, tl + g * G::BYTES, T, mw_dst(L, vv, NB, T), part, cr);
     mw_meet<4>((SPX_L float *)&xch[k & 1][4 * g][0][0], c, part, cr, out);  // (its barrier: the tiles are read)
     if (c != 0) continue;
     if (!(k & 1)) {
@@ -2170,12 +2153,12 @@ __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(
       continue;
     }
     if (2 * ((int)blockIdx.x + R * (k >> 1)) + g >= n) continue;
-    const int nv = sj[j * JR + 1], r = lane & 15;
+    const int r = lane & 15;
 #pragma unroll
     for (int t = 0; t < 4; t++) {
       const int v = 4 * (lane >> 4) + t;
-      if (v < nv && x * 16 + r < n_ff)
-        gst<float>(a.h + (int64_t)sj[j * JR + 2 + MAX_M + v] * n_ff + x * 16 + r, gv[t] / (1.0f + expf(-gv[t])) * out[t]);
+      if (v < m && x * 16 + r < n_ff)
+        gst<float>(a.h + (int64_t)v * n_ff + x * 16 + r, gv[t] / (1.0f + expf(-gv[t])) * out[t]);
     }
   }
 }
@@ -2202,24 +2185,70 @@ __global__ __launch_bounds__(256) void kp_route_rows(const DecRouteArgs a) {
   if (lane == 0) gst<int>(a.nkeep + b, keep);
 }
 
+// The same and the job list (route_jobs: an expert's users are one job) for up to sixteen rows, in one
+// workgroup, a row a wavefront: a launch less than kp_route_rows + kp_jobs, whose first loads and last
+// stores are most of their 3.6 + 4.7 us.
+__global__ __launch_bounds__(MAX_M * 64) void kp_route_few(const DecRouteArgs a) {
+  __shared__ int sj[256 * (2 + 2 * MAX_M)];
+  __shared__ signed char slot_of[MAX_M * 256];
+  __shared__ int wcount[MAX_M];
+  float lv[2][4];
+  route_load<MAX_M>(a, lv);
+  const int nj = route_jobs<MAX_M>(a, lv, (SPX_L int *)sj, (SPX_L signed char *)slot_of, (SPX_L int *)wcount, true);
+  if (threadIdx.x == 0) gst<int>(a.njobs + 2, nj);
+}
+
 // The job list of the routed rows in global memory: expert e's users in row order, sixteen a
 // job, jobs in expert order (user (b, slot): vec = b, out = b * n_used + slot). A bit mask of
 // the rows per expert gives each user its rank, so every user is placed by its own thread.
 // njobs[0] = the job count, njobs[2] = the experts with users; expert_count counts each once.
 // Every workgroup of the grid (kp_jobs_grid) builds the masks and the job offsets; workgroup g
 // places the users of slots 256 (g + G k) + thread and writes the jobs of experts e = g mod G.
-__global__ __launch_bounds__(256) void kp_jobs(const DecRouteArgs a) {
+// RAW: the choices and weights are a caller's ([m][n_used], raw_ch / raw_w), row b's checked here: an
+// expert id out of range or chosen twice leaves the row no choices (nkeep 0); workgroup 0 also
+// writes the rows' nkeep and weights for the combine.
+template <bool RAW>
+__device__ __forceinline__ void jobs_body(const DecRouteArgs &a, const int *raw_ch, const float *raw_w, int g, int G) {
   __shared__ unsigned long long mask[256][PMAX / 64];
   __shared__ int jbase[257];
   __shared__ int sch[PMAX * 32], snk[PMAX];  // the rows' choices (-1: none)
   const int tid = threadIdx.x, m = a.m, nu = a.n_used;
   for (int i = tid; i < 256 * (PMAX / 64); i += 256) (&mask[0][0])[i] = 0ull;
-  if (tid < m) snk[tid] = gld<int>(a.nkeep + tid);
+  if (!RAW && tid < m) snk[tid] = gld<int>(a.nkeep + tid);
   {
     constexpr int NL = PMAX * 32 / 256;  // every load in flight at once
     int v[NL];
 #pragma unroll
-    for (int k = 0; k < NL; k++) v[k] = tid + 256 * k < m * 32 ? gld<int>(a.chosen + tid + 256 * k) : 0;
+    for (int k = 0; k < NL; k++) {
+      const int i = tid + 256 * k;
+      if constexpr (RAW) v[k] = i < m * 32 && (i & 31) < nu ? gld<int>(raw_ch + (int64_t)(i >> 5) * nu + (i & 31)) : -1;
+      else v[k] = i < m * 32 ? gld<int>(a.chosen + i) : 0;
+    }
+    if (RAW && g == 0)
+      for (int i = tid; i < m * nu; i += 256) gst<float>(a.weights + i / nu * 32 + i % nu, gld<float>(raw_w + i));
+    if constexpr (RAW) {
+#pragma unroll
+      for (int k = 0; k < NL; k++)
+        if (tid + 256 * k < m * 32) sch[tid + 256 * k] = v[k];
+      __syncthreads();
+      if (tid < m) {
+        unsigned long long seen[4] = {0ull, 0ull, 0ull, 0ull};
+        bool ok = true;
+        for (int j = 0; j < nu; j++) {
+          const int e = sch[tid * 32 + j];
+          ok = ok && e >= 0 && e < a.n_expert;
+          const unsigned long long bit = 1ull << (e & 63);
+#pragma unroll
+          for (int w = 0; w < 4; w++)
+            if (w == ((e >> 6) & 3)) {
+              ok = ok && !(seen[w] & bit);
+              seen[w] |= bit;
+            }
+        }
+        snk[tid] = ok ? nu : 0;
+        if (g == 0) gst<int>(a.nkeep + tid, ok ? nu : 0);
+      }
+    }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NL; k++) {
@@ -2251,7 +2280,6 @@ __global__ __launch_bounds__(256) void kp_jobs(const DecRouteArgs a) {
   int off = 0;
   for (int w = 0; w < wave; w++) off += wsum[w];
   jbase[tid] = off + incl - nje;
-  const int G = gridDim.x, g = blockIdx.x;
   if (tid == 255 && g == 0) {
     gst<int>(a.njobs, off + incl);
     gst<int>(a.njobs + 2, wnx[0] + wnx[1] + wnx[2] + wnx[3]);
@@ -2282,22 +2310,18 @@ __global__ __launch_bounds__(256) void kp_jobs(const DecRouteArgs a) {
   }
 }
 
-// spx_moe_dev's routing in device memory: row b's k choices (chosen / weights [m][k]) into the
-// pipeline's layout (ch32 / w32 [m][32], nkeep [m] = k), a row with an expert id out of range
-// or chosen twice kept with no choices (nkeep 0: its output is NaN); one thread a row.
-__global__ __launch_bounds__(256) void kp_moe_in(const int *chosen, const float *weights, int m, int k, int ne, int *ch32, float *w32,
-                                                 int *nkeep) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= m) return;
-  bool ok = true;
-  for (int j = 0; j < k; j++) {
-    const int e = gld<int>(chosen + (int64_t)b * k + j);
-    ok = ok && e >= 0 && e < ne;
-    for (int i = 0; i < j; i++) ok = ok && gld<int>(chosen + (int64_t)b * k + i) != e;
-    gst<int>(ch32 + b * 32 + j, ok ? e : 0);
-    gst<float>(w32 + b * 32 + j, gld<float>(weights + (int64_t)b * k + j));
-  }
-  gst<int>(nkeep + b, ok ? k : 0);
+__global__ __launch_bounds__(256) void kp_jobs(const DecRouteArgs a) { jobs_body<false>(a, nullptr, nullptr, blockIdx.x, gridDim.x); }
+
+// What comes before spx_moe_dev's experts, in one launch: workgroups 0 .. G - 1 the caller's routing
+// checked and its job list, the others x's rows as Q8_K, a wavefront a 256-block (x, ld_x, dim).
+// Nine rows of eight choices: the three launches it stands for took 6.3 + 4.6 + 4.8 us.
+__global__ __launch_bounds__(256) void kp_moe_front(const DecRouteArgs a, const int *raw_ch, const float *raw_w, int G, const float *x, int64_t ld_x,
+                                                    int dim, Q8KP y) {
+  if ((int)blockIdx.x < G) return jobs_body<true>(a, raw_ch, raw_w, blockIdx.x, G);
+  const int nb = dim >> 8, gb = ((int)blockIdx.x - G) * 4 + ((int)threadIdx.x >> 6);
+  if (gb >= nb * a.m) return;
+  const float4 xv = gld<float4>(x + (int64_t)(gb / nb) * ld_x + (gb % nb) * 256 + 4 * (threadIdx.x & 63));
+  q8k_block_store(xv, q8k_amax(xv), y.q + (int64_t)gb * 64, y.d + gb, reinterpret_cast<int *>(y.bs + (int64_t)gb * 8));
 }
 // y[b] = sum over j < nkeep[b], in j order, of w32[b][j] * yd[b k + j] (each product and sum
 // rounded, from 0: the combine of moe_forward_batch :1133-1140); NaN for a row kept with no
@@ -2711,21 +2735,15 @@ int dec_mq_grid(int tiles, int m) {
   return std::max(8, std::min((need + 7) / 8 * 8, per));
 }
 
-hipError_t launch_dec_gateup_mq(const DecGateUpMArgs &args, int max_jobs, hipStream_t s) {
-  DecGateUpMArgs a = args;
-  a.max_jobs = max_jobs;
+hipError_t launch_dec_gateup_mq(const DecGateUpMArgs &a, hipStream_t s) {
   const int nb = (int)(a.gate.cols >> 8);
-  if (a.gate.cols % 256 || nb > DEC_MAXNB || a.gate.nb != nb || a.up.nb != nb || a.gate.dtype != a.up.dtype || a.m < 1 || a.m > MAX_M || max_jobs < 1 ||
-      max_jobs > 512 || (a.rt.logits && (max_jobs > a.gate.n_expert || a.rt.m != a.m || a.rt.n_expert < 1 || a.rt.n_expert > 256 || a.rt.n_used < 1 ||
-                                         a.rt.n_used > 32 || a.rt.n_used > a.rt.n_expert)))
+  if (a.gate.cols % 256 || nb > DEC_MAXNB || a.gate.nb != nb || a.up.nb != nb || a.gate.dtype != a.up.dtype || a.m < 1 || a.m > MAX_M)
     return hipErrorInvalidValue;
   if (a.gate.dtype != T_Q4K && a.gate.dtype != T_Q6K) return hipErrorInvalidValue;
-  // staged tiles: two items a round, one workgroup a CU; every workgroup routes the pass (the
-  // items beyond the job count end at once)
-  const size_t jb = (size_t)(a.rt.logits ? max_jobs : 1) * (2 + 2 * MAX_M) * 4;
-  const size_t sm = mw_tail_off(a.m, nb) + ((std::max((size_t)a.m * nb * 64, 2 * ms_tile_bytes(nb, a.gate.dtype == T_Q6K)) + 15) & ~(size_t)15) + jb;
+  // staged tiles: two items a round, one workgroup a CU
+  const size_t sm = mw_tail_off(a.m, nb) + std::max((size_t)a.m * nb * 64, 2 * ms_tile_bytes(nb, a.gate.dtype == T_Q6K));
   if (sm > 136 * 1024) return hipErrorInvalidValue;
-  const int items = ((a.n_ff + 15) / 16) * (a.rt.logits ? max_jobs : 1);
+  const int items = (a.n_ff + 15) / 16;
   const dim3 grid((unsigned)std::max(1, std::min((items + 1) / 2, cu_count()))), b(DEC_MM_NW * 64);
   auto go = [&](auto kern) {
     SPX_DLDS(kern, sm);
@@ -2744,22 +2762,22 @@ hipError_t launch_kp_route(const DecRouteArgs &a, hipStream_t s) {
   if (a.m < 1 || a.m > PMAX || a.n_expert < 1 || a.n_expert > 256 || a.n_used < 1 || a.n_used > 32 || a.n_used > a.n_expert || !a.jobs ||
       !a.njobs)
     return hipErrorInvalidValue;
+  if (a.m <= MAX_M) {
+    hipLaunchKernelGGL(kp_route_few, dim3(1), dim3(MAX_M * 64), 0, s, a);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(kp_route_rows, dim3((a.m + 3) / 4), dim3(256), 0, s, a);
   hipLaunchKernelGGL(kp_jobs, dim3(kp_jobs_grid(a.m)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
-hipError_t launch_kp_moe_in(const int *chosen, const float *weights, int m, int k, int ne, int *ch32, float *w32, int *nkeep, hipStream_t s) {
-  if (m < 1 || m > PMAX || k < 1 || k > 32 || ne < 1 || ne > 256) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(kp_moe_in, dim3((m + 255) / 256), dim3(256), 0, s, chosen, weights, m, k, ne, ch32, w32, nkeep);
-  return hipGetLastError();
-}
-
-hipError_t launch_kp_jobs(const DecRouteArgs &a, hipStream_t s) {
-  if (a.m < 1 || a.m > PMAX || a.n_expert < 1 || a.n_expert > 256 || a.n_used < 1 || a.n_used > 32 || !a.jobs || !a.njobs || !a.chosen ||
-      !a.nkeep)
+hipError_t launch_kp_moe_front(const DecRouteArgs &a, const int *chosen, const float *weights, const float *x, int64_t ld_x, int dim, Q8KP y,
+                               hipStream_t s) {
+  if (a.m < 1 || a.m > PMAX || a.n_expert < 1 || a.n_expert > 256 || a.n_used < 1 || a.n_used > 32 || !a.jobs || !a.njobs || !a.weights || !a.nkeep ||
+      dim < 256 || dim % 256)
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(kp_jobs, dim3(kp_jobs_grid(a.m)), dim3(256), 0, s, a);
+  const int G = (int)kp_jobs_grid(a.m);
+  hipLaunchKernelGGL(kp_moe_front, dim3(G + (dim / 256 * a.m + 3) / 4), dim3(256), 0, s, a, chosen, weights, G, x, ld_x, dim, y);
   return hipGetLastError();
 }
 

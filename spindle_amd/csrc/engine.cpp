@@ -845,15 +845,19 @@ int enqueue_pass_m(spx_engine *E, int m) {
         DecRouterMArgs ra{ly.router->v, E->xn2, E->rlog, c.n_expert, dim, m};
         SPX_HIP(launch_dec_router_m(ra, s));
       }
-      {  // routing + jobs (every workgroup) and the grouped gate/up
+      {  // routing + jobs and the grouped gate/up
         ProfScope ps(E, PC_GATEUP, wbytes(ly.gate) + wbytes(ly.up), l, true);
         ga.rt = DecRouteArgs{E->rlog, c.n_expert, c.n_expert_used, c.expert_norm, m, c.moe_prune, E->chosen, E->weights, E->nkeep,
                              E->jobs, ly.njobs, E->expert_count + (size_t)l * c.n_expert};
-        if (big) {
+        // matrix cores: routing and job list in a launch of their own, then the job-list kernel. (Both in
+        // the staged-tile kernel's prologue, every workgroup routing for itself, Qwen3-30B-A3B 4 layers,
+        // us a pass with it / so: 2 rows 363 / 358, 4 rows 447 / 446, 6 rows 501 / 472, 9 rows 559 / 520,
+        // 16 rows 636 / 597.)
+        if (big || mqk(spx_engine::MQ_GATEUP)) {
           SPX_HIP(launch_kp_route(ga.rt, s));
-          SPX_HIP(launch_kp_gateup_mq(ga, E->jobs, ly.njobs, maxj, s));
+          SPX_HIP(launch_kp_gateup_mq(ga, E->jobs, ly.njobs, big ? maxj : std::min(m * nu, c.n_expert), s));
         } else {
-          SPX_HIP(mqk(spx_engine::MQ_GATEUP) ? launch_dec_gateup_mq(ga, std::min(m * nu, c.n_expert), s) : launch_dec_gateup_m(ga, std::min(m * nu, c.n_expert), s));
+          SPX_HIP(launch_dec_gateup_m(ga, std::min(m * nu, c.n_expert), s));
         }
       }
       if (int r = snap_ffn(E, l, m)) return r;
@@ -867,7 +871,7 @@ int enqueue_pass_m(spx_engine *E, int m) {
       {
         ProfScope ps(E, PC_GATEUP, wbytes(ly.gate) + wbytes(ly.up));
         if (big) SPX_HIP(launch_kp_gateup_mq(ga, nullptr, nullptr, 1, s));
-        else SPX_HIP(mqk(spx_engine::MQ_GATEUP) ? launch_dec_gateup_mq(ga, 1, s) : launch_dec_gateup_m(ga, 1, s));
+        else SPX_HIP(mqk(spx_engine::MQ_GATEUP) ? launch_dec_gateup_mq(ga, s) : launch_dec_gateup_m(ga, 1, s));
         SPX_HIP(launch_q8kp_quantize(E->h, nff, nff, m, E->hq, s));
       }
       if (int r = snap_ffn(E, l, m)) return r;

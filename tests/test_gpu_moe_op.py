@@ -141,3 +141,29 @@ def test_moe_dev_job_edges(ctx, fmt, dim, nff, ne, k, m):
     for a in range(0, m, step):
         want = ops.moe(ctx, *mats, x[a:a + step].contiguous(), chosen[a:a + step], weights[a:a + step]).cpu().numpy()
         assert np.array_equal(want.view(np.uint32), y[a:a + step].view(np.uint32)), a
+
+
+@pytest.mark.parametrize("m,k,ne", [(128, 8, 256), (17, 32, 32), (128, 1, 3)])
+def test_moe_dev_routing_checked(ctx, m, k, ne):
+    """The routing check at its sizes' edges (one workgroup to sixteen, ids in every 64-bit word of the
+    seen mask): rows with a negative id, an id past the last or a repeated id are NaN, all others have
+    the bits of a call without the bad rows."""
+    from spindle_amd import ops
+    ex = _experts(ctx, R.Q4K, R.Q6K, 256, 256, ne, seed=m + k)
+    mats = [ex[n][1] for n in ("gate", "up", "down")]
+    rng = np.random.default_rng(m * k)
+    x = torch.from_numpy(rng.standard_normal((m, 256)).astype(np.float32)).cuda()
+    chosen = np.stack([rng.permutation(ne)[:k] for _ in range(m)]).astype(np.int32)
+    weights = rng.dirichlet(np.ones(k), m).astype(np.float32)
+    bad = {0: -1, m // 2: ne, m - 1: -2 ** 31, 3: 2 ** 31 - 1}
+    for b, e in bad.items():
+        chosen[b, k - 1] = e
+    if k > 1:
+        bad[5] = chosen[5, 0]
+        chosen[5, k - 1] = chosen[5, 0]
+    good = [b for b in range(m) if b not in bad]
+    call = lambda rows: ops.moe_dev(ctx, *mats, x[rows].contiguous(), torch.from_numpy(chosen[rows]).cuda(),
+                                    torch.from_numpy(weights[rows]).cuda()).cpu().numpy()
+    y = call(list(range(m)))
+    assert np.isnan(y[list(bad)]).all()
+    assert np.array_equal(y[good].view(np.uint32), call(good).view(np.uint32))
