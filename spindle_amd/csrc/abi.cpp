@@ -393,7 +393,8 @@ static int mv_launch(spx_ctx *ctx, const spx_tensor *w, int expert, int m, const
   a.m = m;
   a.G = G;
   a.R = R;
-  a.fx = w->v.dtype == T_Q8_0 && m >= FX_MIN_ROWS ? 1 : 0;
+  // (its loads of x have 32-bit byte offsets: vectors further apart keep the per-lane walk)
+  a.fx = w->v.dtype == T_Q8_0 && m >= FX_MIN_ROWS && m * ld_x < (int64_t)1 << 29 ? 1 : 0;
   SPX_HIP(launch_mv(a, m, mode, nullptr, a.seg[0].wgs, ctx->stream));
   return 0;
 }

@@ -70,6 +70,27 @@ def test_q8_0_non_finite(ctx):
     w.free()
 
 
+@pytest.mark.parametrize("ld", [2 ** 28 - 4, 2 ** 28])
+def test_q8_0_far_apart_vectors(ctx, ld):
+    """Two vectors 1 GiB apart: on either side of where the matrix-core kernel's 32-bit byte offsets
+    end (test_q8_0_edges' bound, which the per-lane walk's 32 additions a block keep too)."""
+    from spindle_amd import ops
+    from spindle_amd._lib import check, lib
+    import ctypes as C
+    rng = np.random.default_rng(9)
+    raw, wd = _q8_0(rng, 1024, 48)
+    w = ops.Tensor(ctx, M.Q8_0, 1024, 48, raw)
+    x = rng.standard_normal((2, 1024)).astype(np.float32)
+    buf, y = torch.empty(ld + 1024, device="cuda"), torch.empty(2, 48, device="cuda")
+    buf[:1024], buf[ld:] = torch.from_numpy(x[0]).cuda(), torch.from_numpy(x[1]).cuda()
+    torch.cuda.synchronize()
+    check(lib.spx_matvec(ctx.h, w.h, 0, C.c_void_p(buf.data_ptr()), ld, 2, C.c_void_p(y.data_ptr()), 48))
+    torch.cuda.synchronize()
+    want, scale = x.astype(np.float64) @ wd.T, np.abs(x.astype(np.float64)) @ np.abs(wd).T
+    assert np.all(np.abs(y.cpu().numpy() - want) <= (96 + 32 + 16) * 2.0 ** -23 * scale)
+    w.free()
+
+
 # dense Q8_0 (attention with q/k norms), dense Q5_0, Q8_0 experts, Q5_0 experts
 # (a model with K-quant matrices too runs passes of at most 16)
 CASES = {
