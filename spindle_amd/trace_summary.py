@@ -2,9 +2,9 @@
 
 A pass is the kernels from k_embed to k_argmax_final (or to the next k_embed: a prompt chunk of
 spx_engine_feed runs no LM head); passes are grouped by kernel count, their
-first matrix kernel (k_mvr<M> / k_mvt<M> / k_mv_f<M>: M = the pass's row bucket; kd_mv / kd_mm /
+first matrix kernel (k_mvr<M> / k_mvt<M> / k_mv_f<M>: M = the pass's row bucket; k_fx_mv: the bf16 matrix cores; kd_mv / kd_mm /
 kd_mq: the decode, lane-exact multi-row and int8-MFMA multi-row kernels) and their row count
-(k_embed's grid: 256 threads a row). For each group: pass span vs busy time, and (groups of at
+(k_embed's grid: a workgroup a row). For each group: pass span vs busy time, and (groups of at
 least 10 passes) the median per-pass time of every kernel.
 
   python3 -m spindle_amd.trace_summary <run_kernel_trace.csv> <summary.txt>
@@ -37,8 +37,8 @@ lines.append(f"kernels in trace: {len(rows)}; forward passes found: {len(passes)
 # classify by kernel count
 groups = collections.defaultdict(list)
 for p in passes:
-    sig = next((short(r[2]) for r in p if short(r[2]).startswith(("k_mvr", "k_mvt", "k_mv_f", "kd_mv", "kd_mm", "kd_mq"))), "none")
-    groups[(len(p), sig, "rows %d" % (p[0][3] // 256))].append(p)
+    sig = next((short(r[2]) for r in p if short(r[2]).startswith(("k_mvr", "k_mvt", "k_mv_f", "k_fx_mv", "kd_mv", "kd_mm", "kd_mq"))), "none")
+    groups[(len(p), sig, "rows %d" % (p[0][3] // max(p[0][4], 1)))].append(p)
 for n, ps in sorted(groups.items()):
     spans = [(p[-1][1] - p[0][0]) / 1e3 for p in ps]
     busy = [sum(r[1] - r[0] for r in p) / 1e3 for p in ps]

@@ -202,7 +202,7 @@ def test_verify_pass_at_context(ctx, key):
     """M=9 at the config's context: the lane-exact pass equals nine one-row passes bitwise (the
     reference's batch invariance, quant_q8k.rs:413-442, moe_batch_fused :4696-4736). The default
     pass on the matrix cores: for the K-quant model (int8, one lane class a wavefront) the same
-    bits too; for the Q8_0 models (fp32 matrix cores: the same products summed in a fixed order
+    bits too; for the Q8_0 models (bf16 matrix cores: the same products summed in a fixed order
     of their own) logits within 1e-3, picks equal except near-ties under 1e-4."""
     S = setup(ctx, key)
     cfg, eng = S.cfg, S.eng

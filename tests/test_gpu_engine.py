@@ -240,7 +240,7 @@ def test_speculation_is_exact_on_gpu(ctx, name, mode, monkeypatch):
     every projection; the default thresholds leave small passes on the lane kernels)."""
     cfg = M.TINY[name].replace(sigma=0.06)
     if mode == "matrix" and not all(t in (M.Q4K, M.Q6K) for t in (cfg.t_q, cfg.t_k, cfg.t_v, cfg.t_o, cfg.t_gate, cfg.t_up, cfg.t_down)):
-        pytest.skip("float formats: the fp32 matrix cores sum in an order of their own (logits within 1e-3), not the one-row bits")
+        pytest.skip("float formats: the bf16 matrix cores sum in an order of their own (logits within 1e-3), not the one-row bits")
     w = M.synth_model(cfg, seed=22)
     prompt = _spec_prompt(cfg.vocab, 4)
     if mode == "matrix":

@@ -201,7 +201,7 @@ def test_int_matvec_real_shapes(ctx, dtype, n, rows, ne, mv_mode):
 @pytest.mark.parametrize("n,rows", [(1024, 2048), (2048, 1024), (1024, 3072), (3072, 1024)])
 def test_q8_0_multi_config2_shapes(ctx, n, rows):
     """Qwen3-0.6B's Q8_0 projections (q, attn_output, gate/up, down) at 2, 9 and 16 vectors:
-    the fp32 matrix-core kernel (k_mv_fq) against the reference's multi-row kernel
+    the bf16 matrix-core kernel (k_fx_mv) against the reference's multi-row kernel
     (quant_multi.rs, the oracle's or_matmul_rows_multi) within 1e-4 of the largest output, and
     within the reference's per-row tolerance 1e-4 * sum|w x| + 1e-6 of the f64 dot; a vector's
     bits the same in any batch of two or more."""
