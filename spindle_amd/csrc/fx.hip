@@ -458,7 +458,11 @@ static hipError_t fx_go(K kern, dim3 grid, size_t sm, hipStream_t s, A... args) 
   return hipGetLastError();
 }
 template <int T, int P, int NT, int NV>  // the wavefronts' stages, then their parts
-static constexpr size_t fx_lds() { return (size_t)FX_NW<P> * (FX_STAGE<T, NT, NV> > NT * NV * 1024 ? FX_STAGE<T, NT, NV> : NT * NV * 1024); }
+static constexpr size_t fx_lds() {
+  constexpr size_t n = (size_t)FX_NW<P> * (FX_STAGE<T, NT, NV> > NT * NV * 1024 ? FX_STAGE<T, NT, NV> : NT * NV * 1024);
+  static_assert(n + 512 <= 160 * 1024, "more than a CU's LDS (the kernels' static part is at most 512 bytes)");
+  return n;
+}
 
 // Workgroups of a launch over one matrix of at most 16 vectors (with greedy keys: its slots).
 static bool fx_wide(int64_t rows, int wg) { return (rows + 64 * wg - 1) / (64 * wg) >= 2 * cu_count_fx(); }
@@ -523,9 +527,16 @@ hipError_t launch_fx_gateup(const GUArgs &a, int m, const StepRec *st, int max_j
     const int tiles = (a.n_ff + 15) / 16;
     if (a.jobs) return go(Tc, Pc, integral_constant<int, 2>{}, integral_constant<int, 1>{});
     if (m <= MAX_M) return go(Tc, Pc, integral_constant<int, 1>{}, integral_constant<int, 1>{});
-    if constexpr (PP <= 8)
+    if constexpr (PP <= 8) {
       if ((tiles + 2 * WG - 1) / (2 * WG) * ((m + 31) / 32) >= cu) return go(Tc, Pc, integral_constant<int, 2>{}, integral_constant<int, 2>{});
-    return go(Tc, Pc, integral_constant<int, 1>{}, integral_constant<int, 2>{});
+      return go(Tc, Pc, integral_constant<int, 1>{}, integral_constant<int, 2>{});
+    } else {
+      // sixteen wavefronts: one vector group (two need more LDS than a CU has). Two row tiles from a
+      // workgroup a CU on: 4 layers of dim 2048, us a pass with two / one, 128 rows of n_ff 4096 572 / 613,
+      // 64 rows of 2048 (256 workgroups) 339 / 347, 64 rows of 1024 (128) 328 / 314.
+      if ((tiles + 1) / 2 * ((m + 15) / 16) >= cu) return go(Tc, Pc, integral_constant<int, 2>{}, integral_constant<int, 1>{});
+      return go(Tc, Pc, integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    }
   };
   return with_parts(DT, nb, shape);
 }
