@@ -2,13 +2,16 @@
 // matrix cores.
 //
 // A weight is an int8 code times its 32-column block's f16 scale d. A code (at most 8 significant
-// bits) is a bf16 exactly, and an fp32 activation is exactly the sum of three bf16 parts (8
-// significant bits each, fx_split), so one block's sum over code * x takes three
+// bits) is a bf16 exactly, and an fp32 activation is the sum of three bf16 parts (8 significant bits
+// each, fx_split), exactly down to |x| = 2^-110, so one block's sum over code * x takes three
 // v_mfma_f32_16x16x32_bf16 into one fp32 accumulator with every product exact, and the row then
 // takes acc = fma(d, sum, acc): the arithmetic of the per-lane kernels (quant.rs:48-161,
 // quant_multi.rs:168-190) in an order of its own. Against float64 its error is the fp32 matrix
 // cores' (v_mfma_f32_16x16x4f32, eight a block, the form before this one) or less, at 48 matrix-core
-// cycles a block and 16 x 16 outputs instead of 256.
+// cycles a block and 16 x 16 outputs instead of 256. Below 2^-110 the third part would need steps
+// finer than bf16's smallest, 2^-133, and an infinity has no parts: a part of a row that met either
+// walks its blocks again with a split that takes them whole (looked for once a part, not once a
+// block: 3072 -> 1024 by 9 rows 8.2 -> 7.6 us, Qwen3-0.6B's 128-row layers 680 -> 646 us for eight).
 //
 // Order of a row's sum, the same for every number of rows in the pass (2..128) and every tile
 // shape: its blocks are cut in P contiguous parts (fx_parts of the blocks a row), each part's
@@ -22,7 +25,7 @@
 // of x a row: 16 or fewer requests an instruction), parks them in its own LDS (swizzled, no
 // barrier) and reads the operands there, the next stage's loads (one tile: the next two's) in flight meanwhile. What
 // bounds the kernels then is the arrival of the weights at 2..16 rows (a launch moves 2-6 MB) and
-// the vector instructions: the split of x (44 of ~75 a block when a wavefront has one tile) and the
+// the vector instructions: the split of x (48 of ~71 a block when a wavefront has one tile) and the
 // int8 -> bf16 conversion, so in prefill passes a wavefront takes NT tiles of 16 rows x NV groups of
 // 16 vectors and pays each once per NT x NV products.
 #include "decode_dev.h"
@@ -34,7 +37,7 @@ namespace spx {
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 template <int P>
 constexpr int FX_NW = P > 8 ? P : 8;  // wavefronts a workgroup: FX_NW / P row groups of P parts
-// Wavefronts a SIMD that the registers are held to (no spills).
+// Wavefronts a SIMD that the registers are held to (no spills but four registers in Q5_0's four-tile form).
 template <int P, int NT, int NV>
 constexpr int FX_WPE = P > 8 || NT * NV <= 2 || NV == 1 ? 4 : 2;
 
@@ -48,32 +51,36 @@ struct FxX {
   uint4 hi, mid, lo;
 };
 // Eight fp32 values as three bf16 parts each: the top 16 bits of x, of the rest r = x - hi (exact,
-// at most 16 significant bits) and of r - mid (at most 8: all of it). An infinite x has the rest 0
-// (inf - inf would make a NaN of every sum it is in); a NaN stays one through r.
-__device__ __forceinline__ FxX fx_split(float4 a, float4 b) {
+// at most 16 significant bits) and of r - mid (at most 8). Two kinds of value come out wrong: of an
+// infinite x the rest is a NaN, and below |x| = 2^-110 the last part can need steps finer than
+// bf16's smallest, 2^-133; such bits are left in the low half of cut, and FIX (rest: 2^100 times what
+// was cut off, at most 16 significant bits) splits both kinds whole. All others have the same parts
+// either way.
+template <bool FIX>
+__device__ __forceinline__ FxX fx_split(float4 a, float4 b, uint32_t &cut, FxX *rest = nullptr) {
   const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
   uint32_t h[8], m[8], l[8];
-  float r[8];
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     h[i] = __float_as_uint(x[i]);
-    r[i] = x[i] - __uint_as_float(h[i] & 0xffff0000u);
+    float r = x[i] - __uint_as_float(h[i] & 0xffff0000u);
+    if (FIX) r = fabsf(x[i]) == INFINITY ? 0.0f : r;
+    m[i] = __float_as_uint(r);
+    l[i] = __float_as_uint(r - __uint_as_float(m[i] & 0xffff0000u));
+    cut |= l[i];
   }
-  // the rests' sum is a NaN exactly where some x is infinite or a NaN (each |rest| < 2^-7 |x|)
-  const float rs = ((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]));
-  if (__builtin_expect(__builtin_amdgcn_ballot_w64(rs != rs) != 0, 0)) {
+  auto pack = [](const uint32_t (&v)[8]) { return make_uint4(fx_hi2(v[0], v[1]), fx_hi2(v[2], v[3]), fx_hi2(v[4], v[5]), fx_hi2(v[6], v[7])); };
+  const FxX o{pack(h), pack(m), pack(l)};
+  if (FIX) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) r[i] = fabsf(x[i]) == INFINITY ? 0.0f : r[i];
+    for (int i = 0; i < 8; i++) {
+      const float t = fabsf(x[i]) < 0x1p-100f ? (__uint_as_float(l[i]) - __uint_as_float(l[i] & 0xffff0000u)) * 0x1p100f : 0.0f;
+      h[i] = __float_as_uint(t);
+      m[i] = __float_as_uint(t - __uint_as_float(h[i] & 0xffff0000u));
+    }
+    rest->hi = pack(h);
+    rest->mid = pack(m);
   }
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    m[i] = __float_as_uint(r[i]);
-    l[i] = __float_as_uint(r[i] - __uint_as_float(m[i] & 0xffff0000u));
-  }
-  FxX o;
-  o.hi = make_uint4(fx_hi2(h[0], h[1]), fx_hi2(h[2], h[3]), fx_hi2(h[4], h[5]), fx_hi2(h[6], h[7]));
-  o.mid = make_uint4(fx_hi2(m[0], m[1]), fx_hi2(m[2], m[3]), fx_hi2(m[4], m[5]), fx_hi2(m[6], m[7]));
-  o.lo = make_uint4(fx_hi2(l[0], l[1]), fx_hi2(l[2], l[3]), fx_hi2(l[4], l[5]), fx_hi2(l[6], l[7]));
   return o;
 }
 
@@ -86,23 +93,23 @@ __device__ __forceinline__ uint4 fx_codes(F code) {
   return make_uint4(fx_hi2(f[0], f[1]), fx_hi2(f[2], f[3]), fx_hi2(f[4], f[5]), fx_hi2(f[6], f[7]));
 }
 
-// Two blocks (u = 0, 1) of one 16-row tile: as a wavefront loads them (go[0]: the first block of tile
-// row lane >> 2, go[1]: of row (lane & 31) >> 1, both relative to block g0 of the planes), in its LDS,
-// and as operands: row j = lane & 15, columns 8 kq .. + 7, kq = lane >> 4. bu: the two block indices.
+// Two blocks (u = 0, 1) of one 16-row tile: as a wavefront loads them (lane: block (lane >> 1) & 1 of
+// row lane >> 2; g: its index, relative to block g0 of the planes), in its LDS, and as operands:
+// row j = lane & 15, columns 8 kq .. + 7, kq = lane >> 4.
 template <int T> struct FxW;
 template <> struct FxW<T_Q8_0> {
   static constexpr int BYTES = 1024 + 64;  // codes [row][4 pieces of 16 bytes, piece c at c ^ (row >> 2)], d [row][u]
   uint4 c;
   uint16_t d;
-  __device__ __forceinline__ void load(const Planes &pl, int64_t g0, const uint32_t (&go)[2], const uint32_t (&bu)[2]) {
+  __device__ __forceinline__ void load(const Planes &pl, int64_t g0, uint32_t g) {
     const int lane = threadIdx.x & 63;
-    c = gld<uint4>(pl.p0 + g0 * 32 + (size_t)((go[0] + ((lane & 2) ? bu[1] : bu[0])) * 32 + 16 * (lane & 1)));
-    d = gld<uint16_t>(pl.p3 + g0 * 2 + (size_t)((go[1] + ((lane & 1) ? bu[1] : bu[0])) * 2));
+    c = gld<uint4>(pl.p0 + g0 * 32 + (size_t)(g * 32 + 16 * (lane & 1)));
+    d = gld<uint16_t>(pl.p3 + g0 * 2 + (size_t)(g * 2));
   }
   __device__ __forceinline__ void park(SPX_L uint8_t *s) const {
     const int lane = threadIdx.x & 63;
     lst<uint4>(s + (lane >> 2) * 64 + (((lane & 3) ^ (lane >> 4)) * 16), c);
-    lst<uint16_t>(s + 1024 + (lane & 31) * 2, d);
+    lst<uint16_t>(s + 1024 + (lane >> 1) * 2, d);
   }
   static __device__ __forceinline__ uint4 codes(const SPX_L uint8_t *s, int u, int j, int kq) {
     const uint2 w = lld<uint2>(s + j * 64 + (((2 * u + (kq >> 1)) ^ (j >> 2)) * 16) + 8 * (kq & 1));
@@ -115,18 +122,17 @@ template <> struct FxW<T_Q5_0> {  // columns 0..15: low nibbles, 16..31: high ni
   uint2 c;
   uint32_t qh;
   uint16_t d;
-  __device__ __forceinline__ void load(const Planes &pl, int64_t g0, const uint32_t (&go)[2], const uint32_t (&bu)[2]) {
+  __device__ __forceinline__ void load(const Planes &pl, int64_t g0, uint32_t g) {
     const int lane = threadIdx.x & 63;
-    c = gld<uint2>(pl.p0 + g0 * 16 + (size_t)((go[0] + ((lane & 2) ? bu[1] : bu[0])) * 16 + 8 * (lane & 1)));
-    const uint32_t g = go[1] + ((lane & 1) ? bu[1] : bu[0]);
+    c = gld<uint2>(pl.p0 + g0 * 16 + (size_t)(g * 16 + 8 * (lane & 1)));
     qh = gld<uint32_t>(pl.p1 + g0 * 4 + (size_t)(g * 4));
     d = gld<uint16_t>(pl.p3 + g0 * 2 + (size_t)(g * 2));
   }
   __device__ __forceinline__ void park(SPX_L uint8_t *s) const {
     const int lane = threadIdx.x & 63;
     lst<uint2>(s + lane * 8, c);
-    lst<uint32_t>(s + 512 + (lane & 31) * 4, qh);
-    lst<uint16_t>(s + 640 + (lane & 31) * 2, d);
+    lst<uint32_t>(s + 512 + (lane >> 1) * 4, qh);
+    lst<uint16_t>(s + 640 + (lane >> 1) * 2, d);
   }
   static __device__ __forceinline__ uint4 codes(const SPX_L uint8_t *s, int u, int j, int kq) {
     const uint2 w = lld<uint2>(s + j * 32 + 16 * u + 8 * (kq & 1));
@@ -153,19 +159,17 @@ __device__ __forceinline__ void fx_xrows(uint32_t (&xo)[NV][4], F row, int ld) {
 #pragma unroll
     for (int i = 0; i < 4; i++) xo[v][i] = (uint32_t)row(16 * v + 4 * i + (int)((threadIdx.x & 63) >> 4)) * (uint32_t)ld * 4u;
 }
-// Where its loads of NT tiles' rows start (FxW::load's go), tile t's rows r0 .. r0 + 15 of at most
+// The first block of lane's row of a tile (FxW::load's g less the block), the rows r0 .. r0 + 15 of at most
 // rows, blocks counted from row rf.
-__device__ __forceinline__ void fx_wrows(uint32_t (&go)[2], int r0, int rows, int rf, int nb) {
-  const int lane = threadIdx.x & 63;
-  go[0] = (uint32_t)(min(r0 + (lane >> 2), rows - 1) - rf) * (uint32_t)nb;
-  go[1] = (uint32_t)(min(r0 + ((lane & 31) >> 1), rows - 1) - rf) * (uint32_t)nb;
+__device__ __forceinline__ uint32_t fx_wrows(int r0, int rows, int rf, int nb) {
+  return (uint32_t)(min(r0 + (int)((threadIdx.x & 63) >> 2), rows - 1) - rf) * (uint32_t)nb;
 }
 
 // One wavefront's part: blocks [b0, b1) of NT 16-row tiles against NV groups of 16 vectors.
 // Tile t's planes are pl[t / TB], counted from block g0[t / TB] (both wave-uniform). s: the
 // wavefront's LDS (FX_STAGE bytes). acc[t][v][q]: row lane & 15 of vector 4 (lane >> 4) + q.
 template <int T, int NT, int NV, int TB>
-__device__ __forceinline__ void fx_part(SPX_L uint8_t *s, const Planes *pl, const int64_t *g0, const uint32_t (&go)[NT][2], const float *x,
+__device__ __forceinline__ void fx_part(SPX_L uint8_t *s, const Planes *pl, const int64_t *g0, const uint32_t (&go)[NT], const float *x,
                                         const uint32_t (&xo)[NV][4], int b0, int b1, f4v (&acc)[NT][NV]) {
   struct Raw {
     FxW<T> w[NT];
@@ -173,16 +177,19 @@ __device__ __forceinline__ void fx_part(SPX_L uint8_t *s, const Planes *pl, cons
   };
   const int lane = threadIdx.x & 63, j = lane & 15, kq = lane >> 4;
   SPX_L uint8_t *sx = s + NT * FxW<T>::BYTES;
+  auto clear = [&]() {
 #pragma unroll
-  for (int t = 0; t < NT; t++)
+    for (int t = 0; t < NT; t++)
 #pragma unroll
-    for (int v = 0; v < NV; v++) acc[t][v] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int v = 0; v < NV; v++) acc[t][v] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+  };
+  clear();
   const uint8_t *xb = reinterpret_cast<const uint8_t *>(x);
   auto load = [&](Raw &r, int b) {
-    const uint32_t bu[2] = {(uint32_t)b, (uint32_t)min(b + 1, b1 - 1)};
+    const uint32_t c = (uint32_t)min(b + 1, b1 - 1), bw = (lane & 2) ? c : (uint32_t)b;
 #pragma unroll
-    for (int t = 0; t < NT; t++) r.w[t].load(pl[t / TB], g0[t / TB], go[t], bu);
-    const uint32_t xc = ((lane & 8) ? bu[1] : bu[0]) * 128u + 16u * (lane & 7);
+    for (int t = 0; t < NT; t++) r.w[t].load(pl[t / TB], g0[t / TB], go[t] + bw);
+    const uint32_t xc = ((lane & 8) ? c : (uint32_t)b) * 128u + 16u * (lane & 7);
 #pragma unroll
     for (int v = 0; v < NV; v++)
 #pragma unroll
@@ -202,12 +209,13 @@ __device__ __forceinline__ void fx_part(SPX_L uint8_t *s, const Planes *pl, cons
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
+  uint32_t cut = 0;
   auto work = [&](int u) {
     FxX xs[NV];
 #pragma unroll
     for (int v = 0; v < NV; v++) {
       const SPX_L uint8_t *xr = sx + v * 4096 + j * 256;
-      xs[v] = fx_split(lld<float4>(xr + (((8 * u + 2 * kq) ^ j) * 16)), lld<float4>(xr + (((8 * u + 2 * kq + 1) ^ j) * 16)));
+      xs[v] = fx_split<false>(lld<float4>(xr + (((8 * u + 2 * kq) ^ j) * 16)), lld<float4>(xr + (((8 * u + 2 * kq + 1) ^ j) * 16)), cut);
     }
 #pragma unroll
     for (int t = 0; t < NT; t++) {
@@ -223,6 +231,29 @@ __device__ __forceinline__ void fx_part(SPX_L uint8_t *s, const Planes *pl, cons
         for (int q = 0; q < 4; q++) acc[t][v][q] = fmaf(d, m[q], acc[t][v][q]);
       }
     }
+  };
+  // The same with the values that it gets wrong whole: the bits of work for a vector without any.
+  auto work_fix = [&](int u) {
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      const SPX_L uint8_t *xr = sx + v * 4096 + j * 256;
+      FxX xr2;
+      const FxX xs = fx_split<true>(lld<float4>(xr + (((8 * u + 2 * kq) ^ j) * 16)), lld<float4>(xr + (((8 * u + 2 * kq + 1) ^ j) * 16)), cut, &xr2);
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        __builtin_amdgcn_sched_barrier(0);  // (one tile's registers at a time)
+        const SPX_L uint8_t *st = s + t * FxW<T>::BYTES;
+        const uint4 w = FxW<T>::codes(st, u, j, kq);
+        const float d = FxW<T>::scale(st, u, j);
+        const f4v z{0.0f, 0.0f, 0.0f, 0.0f}, m = fx_mfma(xs.hi, w, fx_mfma(xs.mid, w, fx_mfma(xs.lo, w, z))), c = fx_mfma(xr2.hi, w, fx_mfma(xr2.mid, w, z));
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          acc[t][v][q] = fmaf(d, m[q], acc[t][v][q]);
+          if (c[q] != 0.0f) acc[t][v][q] = fmaf(d, c[q] * 0x1p-100f, acc[t][v][q]);
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
   };
   if (b0 >= b1) return;
   if constexpr (NT * NV > 1) {  // the next stage's loads cover this one's products (other wavefronts' too)
@@ -251,6 +282,23 @@ __device__ __forceinline__ void fx_part(SPX_L uint8_t *s, const Planes *pl, cons
       if (b + 1 < b1) work(1);
       b += 2;
       if (b >= b1) break;
+    }
+  }
+  // an infinity or a NaN in x is a NaN in its vector's sums
+  float sum = 0.0f;
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int v = 0; v < NV; v++) sum = sum + ((acc[t][v][0] + acc[t][v][1]) + (acc[t][v][2] + acc[t][v][3]));
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64((cut & 0xffffu) != 0 || sum != sum) != 0, 0)) {
+    clear();
+#pragma unroll 1
+    for (int b = b0; b < b1; b += 2) {
+      Raw r;
+      load(r, b);
+      park(r);
+#pragma unroll 1
+      for (int u = 0; u < min(2, b1 - b); u++) work_fix(u);
     }
   }
 }
@@ -306,9 +354,9 @@ __global__ __launch_bounds__(FX_NW<P> * 64) __attribute__((amdgpu_waves_per_eu(F
     const int r1 = (int)sg.r1, r0 = (int)sg.r0 + wg * RW, rg = r0 + g * RG, rf = min(rg, r1 - 1);
     const Planes pl = sg.w.pl;
     const int64_t g0 = ((int64_t)sg.expert * sg.w.rows + rf) * nb;
-    uint32_t go[NT][2];
+    uint32_t go[NT];
 #pragma unroll
-    for (int u = 0; u < NT; u++) fx_wrows(go[u], rg + 16 * u, r1, rf, nb);
+    for (int u = 0; u < NT; u++) go[u] = fx_wrows(rg + 16 * u, r1, rf, nb);
     f4v acc[NT][NV];
     fx_part<T, NT, NV, NT>(stage, &pl, &g0, go, a.x, xo, b0, b1, acc);
     __syncthreads();  // the stages' LDS takes the parts
@@ -368,9 +416,9 @@ __global__ __launch_bounds__(FX_NW<P> * 64) __attribute__((amdgpu_waves_per_eu(F
   const int r0 = blockIdx.x * RW, rg = r0 + g * RG, rf = min(rg, n_ff - 1);
   const Planes pl[2] = {a.gate.pl, a.up.pl};
   const int64_t gb = ((int64_t)e * n_ff + rf) * nb, g0[2] = {gb, gb};
-  uint32_t go[NT][2];
+  uint32_t go[NT];
 #pragma unroll
-  for (int u = 0; u < NT; u++) fx_wrows(go[u], rg + 16 * (u % NH), n_ff, rf, nb);
+  for (int u = 0; u < NT; u++) go[u] = fx_wrows(rg + 16 * (u % NH), n_ff, rf, nb);
   f4v acc[NT][NV];
   fx_part<T, NT, NV, NH>((SPX_L uint8_t *)smem + wave * FX_STAGE<T, NT, NV>, pl, g0, go, a.x, xo, b0, b1, acc);
   __syncthreads();  // the stages' LDS takes the parts
@@ -406,9 +454,9 @@ __global__ __launch_bounds__(FX_NW<P> * 64) __attribute__((amdgpu_waves_per_eu(F
   const int r0 = blockIdx.x * RW, rg = r0 + g * RG, rf = min(rg, dim - 1);
   const Planes pl = a.w.pl;
   const int64_t g0 = ((int64_t)e * dim + rf) * nb;
-  uint32_t go[NT][2];
+  uint32_t go[NT];
 #pragma unroll
-  for (int u = 0; u < NT; u++) fx_wrows(go[u], rg + 16 * u, dim, rf, nb);
+  for (int u = 0; u < NT; u++) go[u] = fx_wrows(rg + 16 * u, dim, rf, nb);
   f4v acc[NT][1];
   fx_part<T, NT, 1, NT>((SPX_L uint8_t *)smem + wave * FX_STAGE<T, NT, 1>, &pl, &g0, go, a.x, xo, b0, b1, acc);
   __syncthreads();  // the stages' LDS takes the parts

@@ -1,6 +1,7 @@
 """Float-activation products on the bf16 matrix cores (fx.hip): Q8_0 matvecs of 2..16 rows against
-float64 at the edges of their tiles and parts, non-finite activations, and prefill passes of float
-models (17..128 rows) against the same rows in passes of at most 16, bitwise."""
+float64 at the edges of their tiles and parts, activations of every size to the last bit and
+non-finite ones, and prefill passes of float models (17..128 rows) against the same rows in passes of
+at most 16, bitwise."""
 import numpy as np
 import pytest
 
@@ -68,6 +69,50 @@ def test_q8_0_non_finite(ctx):
             assert np.array_equal(got[v], want.astype(np.float32), equal_nan=True), v
     assert np.isnan(got[4]).all()
     w.free()
+
+
+# one, three and sixteen parts a row; the four-tile shape of large matrices
+@pytest.mark.parametrize("cols,rows", [(32, 17), (1056, 33), (2080, 40), (64, 33000)])
+def test_q8_0_whole_activations(ctx, cols, rows):
+    """One non-zero activation of 24 significant bits a vector, in each column of a block in turn and
+    from the smallest normal to the largest binade and down to the denormals (below 2^-110 its last
+    bits are finer than a bf16 holds): times a code of 1 or -1 and a scale of 1/2 it is exact, so
+    anything but the exact product is a bit lost. The vectors of a batch take different sizes."""
+    from spindle_amd import ops
+    rng = np.random.default_rng(cols)
+    raw = np.zeros((rows, cols // 32, 34), np.uint8)
+    raw[:, :, :2] = np.float16([0.5]).view(np.uint8)
+    code = rng.choice([1, -1], (rows, cols)).astype(np.int8)
+    raw[:, :, 2:] = code.reshape(rows, -1, 32).view(np.uint8)
+    w = ops.Tensor(ctx, M.Q8_0, cols, rows, raw.reshape(-1))
+    exps = [0, 126, -60, -100, -109, -111, -118, -125, -127, -133, -140]
+    for e0 in range(len(exps)):
+        x, want = np.zeros((32, cols), np.float32), np.zeros((32, rows), np.float32)
+        for c in range(32):
+            at = 32 * int(rng.integers(0, cols // 32)) + c
+            v = np.ldexp(1.0 + (rng.integers(0, 2 ** 22) * 2 + 1) * 2.0 ** -23, exps[(e0 + c) % len(exps)])
+            x[c, at] = np.float32(v)
+            want[c] = (x[c, at].astype(np.float64) * 0.5 * code[:, at]).astype(np.float32)
+        for a, b in ((0, 16), (16, 25), (25, 32)):
+            got = ops.matvec(ctx, w, torch.from_numpy(x[a:b]).cuda()).cpu().numpy()
+            assert np.array_equal(got, want[a:b]), (e0, a, np.argwhere(got != want[a:b])[:4])
+    w.free()
+
+
+@pytest.mark.parametrize("m", [9, 128])
+def test_tiny_activations_logits(ctx, m):
+    """A model whose activations are around 2^-115: the LM head's rows over the pass's own hidden rows,
+    in float64, to the rounding of their sums (test_q8_0_edges)."""
+    cfg = M.TINY["tiny-qwen3"].replace(max_seq=320, embedding_scale=2.0 ** -125, dim=1024)
+    w = M.synth_model(cfg, seed=3)
+    eng = M.Engine(ctx, cfg, w)
+    _, hid, lg = eng.forward(np.random.default_rng(4).integers(0, cfg.vocab, m), 0, hidden=True, logits=True)
+    spec, data = w["token_embd.weight"]
+    wd = ffi.dequant(spec.dtype, data, spec.rows, spec.cols).astype(np.float64).reshape(spec.rows, spec.cols)
+    h = hid.astype(np.float64)
+    assert 0 < np.abs(h).max() < 2.0 ** -110
+    assert np.all(np.abs(lg - h @ wd.T) <= (96 + cfg.dim // 32 + 16) * 2.0 ** -23 * (np.abs(h) @ np.abs(wd).T) + cfg.dim * 2.0 ** -150)
+    eng.close()
 
 
 @pytest.mark.parametrize("ld", [2 ** 28 - 4, 2 ** 28])
