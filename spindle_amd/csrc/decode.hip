@@ -693,11 +693,8 @@ __global__ __launch_bounds__(256) void kd_norm(const DecNormArgs a) {
   if (a.q_out.q) {
     in_quant<NW, KB>(in, r, (SPX_G uint32_t *)(a.q_out.q + (int64_t)b * a.dim / 4), (SPX_G float *)(a.q_out.d + (int64_t)b * nbq),
                      (SPX_G int *)(a.q_out.bs + (int64_t)b * nbq * 8), (SPX_L float *)bsum_, xn);
-  } else {  // fp32 only: quantize into a scratch image nobody reads
-    __shared__ uint32_t sq[DEC_MAXNB * 64];
-    __shared__ float sd[DEC_MAXNB];
-    __shared__ int sb[DEC_MAXNB * 16];
-    in_quant<NW, KB>(in, r, (SPX_L uint32_t *)sq, (SPX_L float *)sd, (SPX_L int *)sb, (SPX_L float *)bsum_, xn);
+  } else {
+    in_norm<NW, KB>(in, r, (SPX_L float *)bsum_, xn);
   }
 }
 

@@ -134,40 +134,44 @@ __device__ __forceinline__ void in_load(const DecIn &in, InRow<KB> &r) {
 }
 
 // rmsnorm (:569-575) as the norm tails compute it (per 256 block a wavefront tree, then the
-// blocks in order; inv = 1 / sqrt(S / cols + eps) correctly rounded; x * inv * w), then
-// quantize_avx2 of each block into the LDS image (lq, ld, lbs). xn_out: the normalised row.
-template <int NW, int KB, class QP, class DP, class BP>
-__device__ __forceinline__ void in_quant(const DecIn &in, InRow<KB> &r, QP lq, DP ld, BP lbs, SPX_L float *bsum, float *xn_out) {
+// blocks in order; inv = 1 / sqrt(S / cols + eps) correctly rounded; x * inv * w) of a row in
+// registers. xn_out: the normalised row in memory too.
+template <int NW, int KB>
+__device__ __forceinline__ void in_norm(const DecIn &in, InRow<KB> &r, SPX_L float *bsum, float *xn_out) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nbq = in.cols >> 8;
-  if (in.nw) {
 #pragma unroll
-    for (int k = 0; k < KB; k++) {
-      const int tb = wave + NW * k;
-      if (tb < nbq) {
-        float p = r.v[k].x * r.v[k].x;
-        p = fmaf(r.v[k].y, r.v[k].y, p);
-        p = fmaf(r.v[k].z, r.v[k].z, p);
-        p = fmaf(r.v[k].w, r.v[k].w, p);
-        p = wave_sum(p);
-        if (lane == 0) bsum[tb] = p;
-      }
-    }
-    __syncthreads();
-    float S = 0.0f;
-    for (int k = 0; k < nbq; k++) S = S + bsum[k];
-    const float inv = inv_rms(S, (float)in.cols, in.eps);
-#pragma unroll
-    for (int k = 0; k < KB; k++) {
-      const int tb = wave + NW * k;
-      if (tb < nbq) {
-        float4 v = r.v[k];
-        const float4 w = r.w[k];
-        v.x = v.x * inv * w.x; v.y = v.y * inv * w.y; v.z = v.z * inv * w.z; v.w = v.w * inv * w.w;
-        r.v[k] = v;
-        if (xn_out) gst<float4>(xn_out + 4 * (tb * 64 + lane), v);
-      }
+  for (int k = 0; k < KB; k++) {
+    const int tb = wave + NW * k;
+    if (tb < nbq) {
+      float p = r.v[k].x * r.v[k].x;
+      p = fmaf(r.v[k].y, r.v[k].y, p);
+      p = fmaf(r.v[k].z, r.v[k].z, p);
+      p = fmaf(r.v[k].w, r.v[k].w, p);
+      p = wave_sum(p);
+      if (lane == 0) bsum[tb] = p;
     }
   }
+  __syncthreads();
+  float S = 0.0f;
+  for (int k = 0; k < nbq; k++) S = S + bsum[k];
+  const float inv = inv_rms(S, (float)in.cols, in.eps);
+#pragma unroll
+  for (int k = 0; k < KB; k++) {
+    const int tb = wave + NW * k;
+    if (tb < nbq) {
+      float4 v = r.v[k];
+      const float4 w = r.w[k];
+      v.x = v.x * inv * w.x; v.y = v.y * inv * w.y; v.z = v.z * inv * w.z; v.w = v.w * inv * w.w;
+      r.v[k] = v;
+      if (xn_out) gst<float4>(xn_out + 4 * (tb * 64 + lane), v);
+    }
+  }
+}
+// The same (unless in.nw is null), then quantize_avx2 of each block into the LDS image (lq, ld, lbs).
+template <int NW, int KB, class QP, class DP, class BP>
+__device__ __forceinline__ void in_quant(const DecIn &in, InRow<KB> &r, QP lq, DP ld, BP lbs, SPX_L float *bsum, float *xn_out) {
+  const int wave = threadIdx.x >> 6, nbq = in.cols >> 8;
+  if (in.nw) in_norm<NW, KB>(in, r, bsum, xn_out);
 #pragma unroll
   for (int k = 0; k < KB; k++) {
     const int tb = wave + NW * k;
