@@ -642,14 +642,16 @@ __global__ __launch_bounds__(512) void kd_down(const DecDownArgs a) {
 // ================================================================== passes of 2..16 rows
 // ------------------------------------------------------------------ norm of m rows
 // One workgroup per row: residual row -> rmsnorm (the norm tails' fixed-order sum) -> fp32
-// normalised row and / or its Q8_K, in global memory.
+// normalised row and / or its Q8_K, in global memory. RAG: rows of any multiple of four values (in_has),
+// fp32 only.
+template <bool RAG>
 __global__ __launch_bounds__(256) void kd_norm(const DecNormArgs a) {
   constexpr int NW = 4, KB = DEC_MAXNB / NW;
   __shared__ float bsum_[DEC_MAXNB];
-  const int b = blockIdx.x, nbq = a.dim >> 8;
+  const int b = blockIdx.x;
   const DecIn in{(a.yd ? a.res_in : a.x) + (int64_t)b * a.dim, a.nw, a.eps, a.dim};
   InRow<KB> r;
-  in_load<NW, KB>(in, r);
+  in_load<NW, KB, RAG>(in, r);
   if (a.yd) {  // the MoE combine of row b: kept choices in choice order, then the residual add
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nk = gld<int>(a.nkeep + b);
     const float *yr = a.yd + (int64_t)b * a.n_used * a.dim;
@@ -666,7 +668,7 @@ __global__ __launch_bounds__(256) void kd_norm(const DecNormArgs a) {
 #pragma unroll
         for (int k = 0; k < KB; k++) {
           const int tb = wave + NW * k;
-          yv[t][k] = tb < nbq ? gld<float4>(yr + (int64_t)i * a.dim + 4 * (tb * 64 + lane)) : make_float4(0.f, 0.f, 0.f, 0.f);
+          yv[t][k] = in_has<RAG>(tb, a.dim) ? gld<float4>(yr + (int64_t)i * a.dim + 4 * (tb * 64 + lane)) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
       }
 #pragma unroll
@@ -681,7 +683,7 @@ __global__ __launch_bounds__(256) void kd_norm(const DecNormArgs a) {
 #pragma unroll
     for (int k = 0; k < KB; k++) {
       const int tb = wave + NW * k;
-      if (tb < nbq) {
+      if (in_has<RAG>(tb, a.dim)) {
         float4 x = r.v[k];
         x.x = x.x + a.rscale * acc[k].x; x.y = x.y + a.rscale * acc[k].y; x.z = x.z + a.rscale * acc[k].z; x.w = x.w + a.rscale * acc[k].w;
         r.v[k] = x;
@@ -690,11 +692,12 @@ __global__ __launch_bounds__(256) void kd_norm(const DecNormArgs a) {
     }
   }
   float *xn = a.xn_out ? a.xn_out + (int64_t)b * a.dim : nullptr;
-  if (a.q_out.q) {
+  if (!RAG && a.q_out.q) {
+    const int nbq = a.dim >> 8;
     in_quant<NW, KB>(in, r, (SPX_G uint32_t *)(a.q_out.q + (int64_t)b * a.dim / 4), (SPX_G float *)(a.q_out.d + (int64_t)b * nbq),
                      (SPX_G int *)(a.q_out.bs + (int64_t)b * nbq * 8), (SPX_L float *)bsum_, xn);
   } else {
-    in_norm<NW, KB>(in, r, (SPX_L float *)bsum_, xn);
+    in_norm<NW, KB, RAG>(in, r, (SPX_L float *)bsum_, xn);
   }
 }
 
@@ -2609,8 +2612,9 @@ hipError_t launch_dec_down(const DecDownArgs &a, hipStream_t s) {
 
 // ------------------------------------------------------------------ launchers, m rows
 hipError_t launch_dec_norm(const DecNormArgs &a, int m, hipStream_t s) {
-  if (a.dim % 256 || a.dim > 256 * DEC_MAXNB || !a.nw || m < 1 || m > PMAX) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(kd_norm, dim3(m), dim3(256), 0, s, a);
+  if (a.dim % 4 || (a.q_out.q && a.dim % 256) || a.dim > 256 * DEC_MAXNB || !a.nw || m < 1 || m > PMAX) return hipErrorInvalidValue;
+  if (a.dim % 256) hipLaunchKernelGGL(kd_norm<true>, dim3(m), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(kd_norm<false>, dim3(m), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -2817,7 +2821,7 @@ hipError_t launch_kp_down_mq(const DecDownMArgs &a, hipStream_t s) {
 }
 
 hipError_t launch_dec_router_m(const DecRouterMArgs &a, hipStream_t s) {
-  if (a.dim % 256 || a.dim > 256 * DEC_MAXNB || a.m < 1 || a.m > PMAX) return hipErrorInvalidValue;
+  if (a.dim % 4 || a.dim > 256 * DEC_MAXNB || a.m < 1 || a.m > PMAX) return hipErrorInvalidValue;
   hipLaunchKernelGGL(kd_router_m, dim3(a.n_expert, (a.m + MAX_M - 1) / MAX_M), dim3(256), 0, s, a);
   return hipGetLastError();
 }

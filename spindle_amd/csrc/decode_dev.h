@@ -118,15 +118,22 @@ struct InRow {
   float4 v[KB], w[KB];
 };
 
-template <int NW, int KB>
+// The 256-value blocks of a row of cols values, and whether this lane has a float4 in block tb. RAG: the
+// last block may be part-filled (cols % 4 == 0; without RAG cols % 256 == 0); what is not there counts as zero.
+template <bool RAG>
+__device__ __forceinline__ int in_blocks(int cols) { return RAG ? (cols + 255) >> 8 : cols >> 8; }
+template <bool RAG>
+__device__ __forceinline__ bool in_has(int tb, int cols) { return RAG ? 4 * (tb * 64 + (int)(threadIdx.x & 63)) < cols : tb < cols >> 8; }
+
+template <int NW, int KB, bool RAG = false>
 __device__ __forceinline__ void in_load(const DecIn &in, InRow<KB> &r) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nbq = in.cols >> 8;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
   for (int k = 0; k < KB; k++) {
     const int tb = wave + NW * k;
     r.v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
     r.w[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (tb < nbq) {
+    if (in_has<RAG>(tb, in.cols)) {
       r.v[k] = gld<float4>(in.x + 4 * (tb * 64 + lane));
       if (in.nw) r.w[k] = gld<float4>(in.nw + 4 * (tb * 64 + lane));
     }
@@ -136,9 +143,9 @@ __device__ __forceinline__ void in_load(const DecIn &in, InRow<KB> &r) {
 // rmsnorm (:569-575) as the norm tails compute it (per 256 block a wavefront tree, then the
 // blocks in order; inv = 1 / sqrt(S / cols + eps) correctly rounded; x * inv * w) of a row in
 // registers. xn_out: the normalised row in memory too.
-template <int NW, int KB>
+template <int NW, int KB, bool RAG = false>
 __device__ __forceinline__ void in_norm(const DecIn &in, InRow<KB> &r, SPX_L float *bsum, float *xn_out) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nbq = in.cols >> 8;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nbq = in_blocks<RAG>(in.cols);
 #pragma unroll
   for (int k = 0; k < KB; k++) {
     const int tb = wave + NW * k;
@@ -158,7 +165,7 @@ __device__ __forceinline__ void in_norm(const DecIn &in, InRow<KB> &r, SPX_L flo
 #pragma unroll
   for (int k = 0; k < KB; k++) {
     const int tb = wave + NW * k;
-    if (tb < nbq) {
+    if (in_has<RAG>(tb, in.cols)) {
       float4 v = r.v[k];
       const float4 w = r.w[k];
       v.x = v.x * inv * w.x; v.y = v.y * inv * w.y; v.z = v.z * inv * w.z; v.w = v.w * inv * w.w;

@@ -338,12 +338,8 @@ bool fx_on(const spx_engine *E, const spx_tensor *t) {
   return E->mq && (t->v.dtype == T_Q8_0 || (t->v.dtype == T_Q5_0 && E->all_float));
 }
 
-// A MoE layer whose passes of 2..128 rows run on the bf16 matrix cores: float experts, and a row
-// width that the multi-row router and norm take.
-bool fx_moe(const spx_engine *E, const LayerW &ly) {
-  return ly.moe && fx_on(E, ly.gate) && fx_on(E, ly.up) && fx_on(E, ly.down) && ly.router->v.dtype == T_F32 &&
-         E->c.dim % 256 == 0 && E->c.dim <= 256 * DEC_MAXNB;
-}
+// A MoE layer whose passes of 2..128 rows run on the bf16 matrix cores: float experts of any width.
+bool fx_moe(const spx_engine *E, const LayerW &ly) { return ly.moe && fx_on(E, ly.gate) && fx_on(E, ly.up) && fx_on(E, ly.down); }
 
 // One forward pass of m rows at the step record's start position: embeddings through the
 // LM head and the greedy pick (forward_slice / forward_batch_slice + compute_logits_batch).
@@ -456,7 +452,7 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
     const int gmode = m <= 2 ? mode_of(E, ly.gate, m) : 0;  // grouped experts: row-parallel at decode, tiles for verify
     if (ly.moe) {  // moe_forward / moe_forward_batch (:925-1392)
       const int nu = c.n_expert_used, ne = c.n_expert;
-      if (fx_moe(E, ly) && m >= FX_MIN_ROWS) {
+      if (m >= FX_MIN_ROWS && fx_moe(E, ly)) {
         // float experts, 2..128 rows: the router's rows, the routing and a job list of at most 16
         // users a job (the K-quant prefill passes' kernels), the experts on the bf16 matrix cores,
         // then the combine in choice order and the next norm in one launch
@@ -1233,7 +1229,6 @@ int spx_engine_prepare(spx_engine *E) {
     for (auto &ly : E->L) {
       for (const spx_tensor *t : {ly.wq, ly.wk, ly.wv, ly.wo, ly.gate, ly.up, ly.down}) ok = ok && fx_type(t->v.dtype);
       ok = ok && ly.wk->v.dtype == ly.wq->v.dtype && ly.wv->v.dtype == ly.wq->v.dtype;
-      ok = ok && (!ly.moe || (ly.router->v.dtype == T_F32 && c.dim % 256 == 0 && c.dim <= 256 * DEC_MAXNB));
       ok = ok && (!ly.q_bias || (c.n_heads / c.n_kv_heads) * c.head_dim <= 2048);
     }
     E->fx_pf = ok;

@@ -143,6 +143,9 @@ CASES = {
     "llama-q5_0": M.TINY["tiny-llama"].replace(sigma=0.05, max_seq=320, t_down=M.Q5_0),
     "granite": M.TINY["tiny-granite"].replace(sigma=0.05, max_seq=320),
     "granite-q5_0": M.TINY["tiny-granite"].replace(sigma=0.05, max_seq=320, t_gate=M.Q5_0, t_up=M.Q5_0, t_down=M.Q5_0, moe_prune=0.3),
+    # rows of a full and a part-filled 256-value block, and of five
+    "granite-288": M.TINY["tiny-granite"].replace(sigma=0.05, max_seq=320, dim=288, n_ff=96),
+    "granite-1056": M.TINY["tiny-granite"].replace(sigma=0.03, max_seq=320, dim=1056, n_ff=160, n_expert=32, n_expert_used=8),
     "wide": M.TINY["tiny-qwen3"].replace(sigma=0.03, max_seq=320, dim=1024, n_heads=16, n_kv_heads=8, head_dim=128, n_ff=2048),
     # sixteen parts a row: the gate/up of 17 rows in one-tile workgroups, of 128 in two-tile ones
     "dim2048": M.TINY["tiny-qwen3"].replace(sigma=0.02, max_seq=320, dim=2048, n_heads=16, n_kv_heads=8, head_dim=128, n_ff=1024),
