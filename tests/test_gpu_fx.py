@@ -179,3 +179,28 @@ def test_float_prefill_equals_16_row_passes(ctx, case):
         assert all(0 < n <= cfg.n_expert for n in a.last_experts())
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("case", list(CASES))
+def test_float_passes_match_oracle(ctx, case):
+    """Passes of 2, 9 and 40 rows against the oracle on the GPU's own KV cache, so that a wrong code or
+    scale of either format cannot hide in both sides: logits within 1e-3 of the largest (the bar of
+    test_gpu_engine). In the median 1e-4: the pass's own keys and values are rounded to f16 on both
+    sides, and where two sums differ by ~2^-22 a share of 2^-22 / 2^-11 of them rounds to the other
+    neighbour, 2^-10 away: 2^-10 sqrt(2^-11) = 2e-5 of their root mean square, a layer and for keys
+    and values each."""
+    from oracle.model import OracleModel
+    cfg = CASES[case]
+    w = M.synth_model(cfg, seed=73)
+    eng, om = M.Engine(ctx, cfg, w), OracleModel(cfg, w)
+    ids, pos, errs = np.random.default_rng(74).integers(0, cfg.vocab, 67), 16, []
+    eng.forward(ids[:16], 0)
+    for m in (2, 9, 40):
+        om.k_cache[:], om.v_cache[:] = eng.kv_cache()
+        _, _, lg = eng.forward(ids[pos:pos + m], pos, hidden=True, logits=True)
+        want = om.logits(om.forward(ids[pos:pos + m], pos)).astype(np.float64)
+        errs += list(np.abs(lg - want).max(1) / np.maximum(1.0, np.abs(want).max(1)))
+        pos += m
+    print(case, "median %.1e max %.1e" % (np.median(errs), np.max(errs)))
+    assert np.max(errs) <= 1e-3 and np.median(errs) <= 1e-4
+    eng.close()
