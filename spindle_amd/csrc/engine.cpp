@@ -142,9 +142,10 @@ struct spx_engine {
   float *dbg = nullptr;
   int64_t dbg_off[13] = {};
   // captured passes by LM-head selection and rows: [0] every row's logits and pick, [1] the
-  // last row's only, [2] none (spx_engine_feed's chunks)
-  hipGraphExec_t graph[3][PMAX + 1] = {};
+  // last row's only, [2] none (spx_engine_feed's chunks); [3], [4]: [0], [1] with want_hid
+  hipGraphExec_t graph[5][PMAX + 1] = {};
   int lm_sel = 0;       // LM-head selection of the pass being enqueued (as graph's first index)
+  bool want_hid = false;  // its last kernel leaves the hidden rows in host memory (up to 16 rows, when the call wants them)
   int n_used = 0;
   // kernel-class timing (eager passes only): event pairs recorded around each launch
   struct ProfRec { int cls, layer; double bytes; bool per_expert; hipEvent_t a, b; };
@@ -327,10 +328,10 @@ int mv_res(spx_engine *E, const spx_tensor *w, const float *x, int64_t ld_x, flo
 // 128-row pass would read the bus from 128 workgroups; a copy before it costs 5 us of its 860.
 const StepRec *step_src(const spx_engine *E, int m, bool advance = false) { return advance || m > MAX_M ? nullptr : E->st_host; }
 
-// Where the last kernel of a pass leaves n rows' picks and (up to 16 rows) their hidden states, rows
-// row0 .. of xn.
-HostOut host_out(spx_engine *E, int n, int row0) {
-  return HostOut{E->picks_host, n <= MAX_M ? E->hidden_host : nullptr, E->xn + (int64_t)row0 * E->c.dim, E->c.dim};
+// Where the last kernel of a pass leaves its rows' picks and (want_hid) their hidden states, rows row0 ..
+// of xn.
+HostOut host_out(spx_engine *E, int row0) {
+  return HostOut{E->picks_host, E->want_hid ? E->hidden_host : nullptr, E->xn + (int64_t)row0 * E->c.dim, E->c.dim};
 }
 
 // A matrix whose passes of two rows and more run on the bf16 matrix cores (fx.hip).
@@ -578,7 +579,7 @@ int enqueue_forward(spx_engine *E, int m, bool advance = false) {
   }
   {
     ProfScope ps(E, PC_ARGMAX, 0);
-    SPX_HIP(launch_argmax_final(E->best, E->nbest, E->amax, last ? nullptr : E->st_dev, advance ? E->hist : nullptr, lm, advance ? HostOut{} : host_out(E, lm, m - lm), s));
+    SPX_HIP(launch_argmax_final(E->best, E->nbest, E->amax, last ? nullptr : E->st_dev, advance ? E->hist : nullptr, lm, advance ? HostOut{} : host_out(E, m - lm), s));
   }
   return 0;
 }
@@ -714,7 +715,7 @@ int enqueue_decode(spx_engine *E, bool advance, int nv = 1) {
   E->nbest = grid;
   {
     ProfScope ps(E, PC_ARGMAX, 0);
-    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, last ? nullptr : E->st_dev, advance ? E->hist : nullptr, nl, advance ? HostOut{} : host_out(E, nl, 0), s));
+    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, last ? nullptr : E->st_dev, advance ? E->hist : nullptr, nl, advance ? HostOut{} : host_out(E, 0), s));
   }
   return 0;
 }
@@ -896,7 +897,7 @@ int enqueue_pass_m(spx_engine *E, int m) {
     SPX_HIP(launch_dec_mv(a, grid, s));
     E->nbest = grid;
     ProfScope pa(E, PC_ARGMAX, 0);
-    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, nullptr, nullptr, 1, host_out(E, 1, 0), s));
+    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, nullptr, nullptr, 1, host_out(E, 0), s));
     return 0;
   }
   {
@@ -913,7 +914,7 @@ int enqueue_pass_m(spx_engine *E, int m) {
   E->nbest = grid;
   {
     ProfScope ps(E, PC_ARGMAX, 0);
-    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, E->st_dev, nullptr, m, host_out(E, m, 0), s));
+    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, E->st_dev, nullptr, m, host_out(E, 0), s));
   }
   return 0;
 }
@@ -952,7 +953,7 @@ int enqueue_persist(spx_engine *E, bool advance) {
   E->nbest = grid;
   {
     ProfScope ps(E, PC_ARGMAX, 0);
-    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, E->st_dev, advance ? E->hist : nullptr, 1, advance ? HostOut{} : host_out(E, 1, 0), s));
+    SPX_HIP(launch_argmax_final(E->best, grid, E->amax, E->st_dev, advance ? E->hist : nullptr, 1, advance ? HostOut{} : host_out(E, 0), s));
   }
   return 0;
 }
@@ -991,7 +992,7 @@ int run_forward(spx_engine *E, int m, bool advance = false) {
   };
   if (!E->use_graphs || E->profiling || E->dbg_on) return enqueue();
   const int slot = advance ? 0 : m;
-  hipGraphExec_t &gx = E->graph[advance ? 0 : E->lm_sel][slot];
+  hipGraphExec_t &gx = E->graph[advance ? 0 : E->lm_sel + (E->want_hid ? 3 : 0)][slot];
   if (!gx) {
     SPX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     int r = enqueue();
@@ -1380,18 +1381,21 @@ int forward_sel(spx_engine *E, const int32_t *ids, int m, int start_pos, float *
   for (int i = 0; i < m; i++) E->st_host->ids[i] = ids[i];
   E->last_m = m;
   if (!step_src(E, m)) SPX_HIP(hipMemcpyAsync(E->st_dev, E->st_host, sizeof(StepRec), hipMemcpyHostToDevice, s));
+  const int nr = sel ? 1 : m;  // rows copied out (sel 1: the last row's, at row 0; the decode pipeline's norm writes row 0)
+  const bool hid_host = nr <= MAX_M;
   E->lm_sel = sel;
+  E->want_hid = hidden && hid_host && sel != 2;
   const int rf = run_forward(E, m);
   E->lm_sel = 0;
+  E->want_hid = false;
   if (rf) {
     (void)hipStreamSynchronize(s);  // what was queued still reads the record
     return rf;
   }
-  const int nr = sel ? 1 : m;  // rows copied out (sel 1: the last row's, at row 0; the decode pipeline's norm writes row 0)
   const int64_t hrow = sel && !(E->dec_ok && E->dec_on) ? m - 1 : 0;
-  // up to 16 hidden rows and the picks are in host memory when the pass ends; one row of logits takes
-  // the same way, more take a copy
-  const bool one_row = logits && nr == 1, hid_host = nr <= MAX_M;
+  // the picks and up to 16 wanted hidden rows are in host memory when the pass ends; one row of logits
+  // takes the same way, more take a copy
+  const bool one_row = logits && nr == 1;
   if (sel != 2) {
     if (hidden && !hid_host) SPX_HIP(hipMemcpyAsync(hidden, E->xn + hrow * E->c.dim, sizeof(float) * nr * E->c.dim, hipMemcpyDeviceToHost, s));
     if (one_row) SPX_HIP(launch_to_host(E->logits, E->logits_host, (E->c.vocab + 3) / 4 * 4, s));

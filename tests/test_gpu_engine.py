@@ -305,3 +305,29 @@ def test_draft_model_speculation(ctx, name):
     eng.set_draft(None)
     for e in (eng, same, other):
         e.close()
+
+
+@pytest.mark.parametrize("name", ["tiny-qwen3", "tiny-granite", "tiny-a3b"])
+def test_hidden_rows_on_request(ctx, name):
+    """Hidden rows asked for in one call and not in the next, the same pass size each time (one captured
+    pass serves both): a call that asks gets its own pass's rows, with the bits of an engine that is
+    always asked, and picks do not depend on it."""
+    cfg = M.TINY[name].replace(sigma=0.05)
+    w = M.synth_model(cfg, seed=31)
+    a, b = M.Engine(ctx, cfg, w), M.Engine(ctx, cfg, w)
+    ids, pos = np.random.default_rng(32).integers(0, cfg.vocab, 256), 0
+    for m in (1, 2, 9, 16, 17):
+        for ask in (True, False, False, True):
+            am, h, _ = a.forward(ids[pos:pos + m], pos, hidden=ask)
+            am2, h2, _ = b.forward(ids[pos:pos + m], pos, hidden=True)
+            assert np.array_equal(am, am2), (name, m)
+            if ask:
+                assert np.array_equal(h.view(np.uint32), h2.view(np.uint32)), (name, m)
+            pos += m
+    for n, ask in ((20, False), (20, True), (1, False), (1, True)):
+        p1, h, _ = a.feed(ids[pos:pos + n], pos, hidden=ask)
+        p2, h2, _ = b.feed(ids[pos:pos + n], pos, hidden=True)
+        assert p1 == p2 and (not ask or np.array_equal(h.view(np.uint32), h2.view(np.uint32))), (name, n)
+        pos += n
+    a.close()
+    b.close()
