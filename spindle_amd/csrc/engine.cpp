@@ -1396,14 +1396,19 @@ int forward_sel(spx_engine *E, const int32_t *ids, int m, int start_pos, float *
   // the picks and up to 16 wanted hidden rows are in host memory when the pass ends; one row of logits
   // takes the same way, more take a copy
   const bool one_row = logits && nr == 1;
-  if (sel != 2) {
-    if (hidden && !hid_host) SPX_HIP(hipMemcpyAsync(hidden, E->xn + hrow * E->c.dim, sizeof(float) * nr * E->c.dim, hipMemcpyDeviceToHost, s));
-    if (one_row) SPX_HIP(launch_to_host(E->logits, E->logits_host, (E->c.vocab + 3) / 4 * 4, s));
-    else if (logits) SPX_HIP(hipMemcpyAsync(logits, E->logits, sizeof(float) * nr * E->c.vocab, hipMemcpyDeviceToHost, s));
-  }
   const bool pers = persist_used(E, m);
-  if (pers) SPX_HIP(hipMemcpyAsync(E->perr_host, E->pa.err, sizeof(int), hipMemcpyDeviceToHost, s));
-  SPX_HIP(hipStreamSynchronize(s));
+  auto bring = [&]() -> int {
+    if (sel != 2) {
+      if (hidden && !hid_host) SPX_HIP(hipMemcpyAsync(hidden, E->xn + hrow * E->c.dim, sizeof(float) * nr * E->c.dim, hipMemcpyDeviceToHost, s));
+      if (one_row) SPX_HIP(launch_to_host(E->logits, E->logits_host, (E->c.vocab + 3) / 4 * 4, s));
+      else if (logits) SPX_HIP(hipMemcpyAsync(logits, E->logits, sizeof(float) * nr * E->c.vocab, hipMemcpyDeviceToHost, s));
+    }
+    if (pers) SPX_HIP(hipMemcpyAsync(E->perr_host, E->pa.err, sizeof(int), hipMemcpyDeviceToHost, s));
+    return 0;
+  };
+  const int rb = bring();
+  SPX_HIP(hipStreamSynchronize(s));  // (also where a copy failed: the pass reads the record)
+  if (rb) return rb;
   if (pers)
     if (int r = persist_check(E)) return r;
   if (sel != 2) {
