@@ -120,8 +120,8 @@ struct spx_engine {
   // device state
   __half *kc = nullptr, *vc = nullptr;
   float2 *rope = nullptr;
-  // host memory that the device reads and writes: a pass's step record, its picks, hidden rows (up to
-  // 16) and one row of logits
+  // host memory that the device reads and writes, one allocation from st_host on: a pass's step record,
+  // its picks, hidden rows (up to 16) and one row of logits
   StepRec *st_dev = nullptr, *st_host = nullptr;
   int *picks_host = nullptr;
   float *hidden_host = nullptr, *logits_host = nullptr;
@@ -1182,10 +1182,16 @@ int spx_engine_prepare(spx_engine *E) {
   if (!ok) return fail("spx_engine_prepare: out of device memory");
   for (auto &ly : E->L)
     if (ly.moe && !(ly.njobs = E->dalloc<int>(3))) return fail("out of device memory");
-  SPX_HIP(hipHostMalloc(&E->st_host, sizeof(StepRec)));
-  SPX_HIP(hipHostMalloc(&E->picks_host, sizeof(int) * PMAX));
-  SPX_HIP(hipHostMalloc(&E->hidden_host, sizeof(float) * MAX_M * c.dim));
-  SPX_HIP(hipHostMalloc(&E->logits_host, sizeof(float) * ((c.vocab + 3) / 4 * 4)));
+  {  // one allocation: each takes 12 us (and as long to free), whatever its size here
+    auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    const size_t rec = al(sizeof(StepRec)), picks = al(sizeof(int) * PMAX), hid = al(sizeof(float) * MAX_M * c.dim), log = al(sizeof(float) * ((c.vocab + 3) / 4 * 4));
+    uint8_t *h = nullptr;
+    SPX_HIP(hipHostMalloc(&h, rec + picks + hid + log));
+    E->st_host = reinterpret_cast<StepRec *>(h);
+    E->picks_host = reinterpret_cast<int *>(h + rec);
+    E->hidden_host = reinterpret_cast<float *>(h + rec + picks);
+    E->logits_host = reinterpret_cast<float *>(h + rec + picks + hid);
+  }
   // RoPE table: inv_freq = 1/theta^(2i/hd) (Rope::new :1399-1402); angle = pos * inv_freq.
   const int half = c.head_dim / 2;
   std::vector<float2> tab((size_t)c.max_seq * half);
@@ -1914,8 +1920,7 @@ int spx_engine_destroy(spx_engine *E) {
   for (auto ev : E->ev_pool) (void)hipEventDestroy(ev);
   for (auto &kv : E->mats) spx_tensor_free(E->ctx, kv.second);
   for (void *p : E->allocs) (void)hipFree(p);
-  for (void *h : {(void *)E->st_host, (void *)E->picks_host, (void *)E->hidden_host, (void *)E->logits_host})
-    if (h) (void)hipHostFree(h);
+  if (E->st_host) (void)hipHostFree(E->st_host);  // (and what lies behind it)
   if (E->perr_host) (void)hipHostFree(E->perr_host);
   delete E;
   return 0;
