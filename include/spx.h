@@ -156,7 +156,10 @@ int spx_engine_decode_pipeline(spx_engine *e, int *active);  /* *active = 1: the
  * sums to rounding (a matvec within ~1e-6 relative of the lane-exact result; a whole pass can
  * differ more where that moves a downstream Q8_K code or a near-tied expert choice, and greedy
  * picks only at near-ties). 0: the lane-exact dot chains, the same bits as one-row passes, so
- * speculation reproduces plain greedy decoding bit for bit. No counterpart in the reference (a
+ * speculation reproduces plain greedy decoding bit for bit. Models without K-quant matrices
+ * run their Q8_0 and Q5_0 matrices (mixed models their Q8_0 ones) in passes of two rows and more
+ * on the bf16 matrix cores, every product whole and the sums in an order of their own; 0: the
+ * one-row order there too. No counterpart in the reference (a
  * choice between two implementations of its batched kernel). */
 int spx_engine_set_mfma(spx_engine *e, int on);
 /* One-row passes (decode) with each layer as one cooperative launch of co-resident workgroups
@@ -173,8 +176,9 @@ int spx_engine_persist_active(spx_engine *e, int *active);
  * chunks of up to 128 rows :3090-3101 — then compute_logits_batch :3588-3602 and the greedy
  * pick of sample_from_logits :3624-3671). K/V of every row are written before any row
  * attends, row b sees positions <= start_pos + b. A pass of more than 16 rows runs on the
- * prefill kernels (K-quant models, matrix cores on), else as consecutive passes of at most
- * 16 rows; either way each row gets the bits it would get in a pass of 16. Optional host
+ * prefill kernels (matrix cores on; K-quant models, and models whose matrices are all Q8_0 or
+ * Q5_0), else as consecutive passes of at most 16 rows; either way each row gets the bits it
+ * would get in a pass of 2..16 (but for the attention of K-quant prefill). Optional host
  * outputs: hidden [m][dim] (after output_norm), logits [m][vocab], argmax [m]. Synchronous. */
 int spx_engine_forward(spx_engine *e, const int32_t *ids, int m, int start_pos, float *hidden,
                        float *logits, int32_t *argmax);

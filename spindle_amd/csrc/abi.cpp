@@ -660,8 +660,12 @@ extern "C" int spx_moe_dev(spx_ctx *ctx, const spx_tensor *gate, const spx_tenso
   ga.gate = gate->v; ga.up = up->v; ga.y = yq; ga.h = h; ga.n_ff = (int)n_ff; ga.m = m;
   SPX_HIP(launch_kp_gateup_mq(ga, jobs, njobs, max_jobs, s));
   DecDownMArgs da{down->v, h, jobs, njobs, yd, max_jobs};
-  // below 12 rows the lane kernel (as the passes choose; 128 experts, 8 a row, us a call with it / on
-  // the matrix cores: 1 row 43.5 / 46.7, 4 rows 64.0 / 71.5, 9 rows 87.5 / 93.5, 16 rows 114.5 / 113.0)
+  // Below 12 rows the lane kernel, as the passes choose. What decides is the users an expert has, which
+  // the host does not see. us a call, calls back to back, with the lane kernel / on the matrix cores,
+  // 768 x 2048 experts chosen at random: of 128, 8 a row, 1 row 28.9 / 31.8, 4 rows 42.9 / 49.7, 8 rows
+  // 57.9 / 61.2, 12 rows 71.1 / 78.1, 16 rows 81.2 / 85.2; of 32 (four users each at 16 rows) 8 rows
+  // 46.6 / 48.3, 12 rows 50.2 / 52.9, 14 rows 50.9 / 47.6, 16 rows 53.4 / 48.0. In a model's passes rows
+  // share experts as those of 32 do or more, and the lines cross at 12 (mq_rows).
   if (m < 12) {
     da.max_jobs = std::min(ne, nv);  // (at most 16 rows: one job an expert)
     SPX_HIP(launch_dec_down_m(da, s));

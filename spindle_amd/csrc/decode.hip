@@ -1883,9 +1883,10 @@ template <int TT>
 constexpr int WS_BYTES = MsGeo<1, TT != T_Q4K>::BYTES;  // a wavefront's LDS
 __host__ __device__ inline size_t ws_bytes(int tt) { return tt == T_Q4K ? WS_BYTES<T_Q4K> : WS_BYTES<0>; }
 
-// The walk of one wavefront over its tiles 0 .. ntiles - 1, all eight classes: tile i's bytes from src(i), its vectors from dst(i), done(i, out) with the tile's
-// results (matrix row lane & 15, vector 4 (lane >> 4) + t). tl: the wavefront's WS_BYTES. SMALL: one
-// block's loads in flight instead of two, ms_step's registers: four wavefronts a SIMD.
+// The walk of one wavefront over its tiles 0 .. ntiles - 1, all eight classes: tile i's bytes from
+// src(i), its vectors from dst(i), done(i, out) with the tile's results (matrix row lane & 15, vector
+// 4 (lane >> 4) + t). tl: the wavefront's WS_BYTES. SMALL: one block's loads in flight instead of two,
+// ms_step's registers: four wavefronts a SIMD.
 template <int NB, int TT, bool SMALL = false, class Src, class Dst, class Done>
 __device__ __forceinline__ void ws_walk(SPX_L uint8_t *tl, int ntiles, Src src, Dst dst, Done done) {
   if (ntiles <= 0) return;
@@ -2349,7 +2350,9 @@ __global__ __launch_bounds__(256) void kp_moe_combine(const float *yd, const flo
 // wavefront, each walking gate and up of every eighth item of a contiguous range: 58.7 us a 128-row
 // layer of 768 x 2048 Q4_K experts, 42.7 us for nine rows; two a CU 48.6 and 35.6; a tile a
 // wavefront 48.3 and 30.8. (The same sums as f16 contractions, a third fewer vector
-// instructions but twice the LDS and so one workgroup a CU: 56.9 and 41.2.)
+// instructions but twice the LDS and so one workgroup a CU: 56.9 and 41.2.) Rows of 4096 columns leave
+// LDS for one workgroup a CU; spx_moe_dev of 64 such experts, 8 a row, us a call with the contiguous
+// ranges / so: 9 rows 152 / 108, 16 rows 197 / 122, 128 rows 291 / 197.
 constexpr int KP_CH = DEC_MM_NW / 2;
 template <int T, int NB>
 __global__ __launch_bounds__(DEC_MM_NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void kp_gateup_mq(const DecGateUpMArgs a, const Job *jobs,

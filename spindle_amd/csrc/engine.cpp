@@ -69,12 +69,18 @@ struct spx_engine {
   bool mq = true;          // passes of 2..16 rows on the int8 matrix cores (SPX_MQ, spx_engine_set_mfma)
   // passes of 2..16 rows: the matrix-core kernels from this many rows, per projection (q|k|v,
   // attention output, gate/up, routed down, LM head; SPX_MQ_ROWS "a,b,c,d,e"); below, the
-  // lane-exact kernels (the same bits). Qwen3-30B-A3B shapes, us per launch (matrix cores vs
-  // lane-exact): rows 2: 11.2/8.2, 9.9/6.4, 17.4/14.9, 9.4 (lane), 114/93; rows 9: 12.0/13.5,
-  // 12.6/11.3, 23.0/31.5, 19.8/16.8, 117/191; rows 16: 12.4/27.7, 13.9/15.1, 26.2/72.8,
-  // 22.0/25.4, 119/420.
+  // lane-exact kernels (the same bits). Qwen3-30B-A3B shapes, us per launch by event pairs in eager
+  // passes (matrix cores / lane-exact; the gate/up with its routing launch):
+  //   rows       3           4           5           6           9          12          16
+  //   q|k|v      12.4/10.7   12.4/11.4   12.7/11.9   12.7/12.5   13.2/15.7  13.5/17.6   13.7/29.5
+  //   output     12.5/9.0    12.9/9.4    13.4/10.0   13.6/10.5   14.7/13.2  15.1/14.6   16.1/17.0
+  //   gate/up    23.2/21.7   24.6/24.6   25.1/29.1   25.6/31.9   28.0/43.8  29.3/52.1   30.4/93.5
+  //   down       18.1/13.0   18.6/14.4   19.7/15.6   20.2/16.7   22.2/20.6  23.5/24.3   25.3/29.5
+  //   LM head    89.6/111    90.1/122    90.6/133    90.5/144    92.2/201   93.0/235    95.6/436
+  // (12, 20 and 25 distinct experts a layer at 3, 9 and 16 rows. The fewer users an expert has, the
+  // longer the lane kernel of the down holds: spx_moe_dev.)
   enum { MQ_QKV, MQ_WO, MQ_GATEUP, MQ_DOWN, MQ_LM, MQ_KINDS };
-  int mq_rows[MQ_KINDS] = {6, 12, 5, 12, 4};
+  int mq_rows[MQ_KINDS] = {6, 12, 5, 12, 3};
   bool mq_shapes = true;   // every K-quant matrix's blocks-a-row count is one the matrix-core kernels take (dec_mq_nb_ok)
   int mv_mode = -1, lm_mode = -1, tail_max = 2, down_mode = 0;  // launch-shape overrides (SPX_MV_MODE, SPX_LM_MODE, SPX_TAIL_MAX, SPX_DOWN_MODE)
   int pf_attn = 4;          // prefill passes: 4 K / V rows prepared + the position slices (k_attn_fs: bits of its own, no partials), 3 the chunk loop (k_attn_fl), 2 the multi-tile
