@@ -2746,7 +2746,8 @@ hipError_t launch_dec_gateup_mq(const DecGateUpMArgs &a, hipStream_t s) {
   if (a.gate.dtype != T_Q4K && a.gate.dtype != T_Q6K) return hipErrorInvalidValue;
   // staged tiles: two items a round, one workgroup a CU
   const size_t sm = mw_tail_off(a.m, nb) + std::max((size_t)a.m * nb * 64, 2 * ms_tile_bytes(nb, a.gate.dtype == T_Q6K));
-  if (sm > 136 * 1024) return hipErrorInvalidValue;
+  // (rows of 4096 columns: from 13 rows of Q4_K, 6 of Q6_K the two tiles leave no room for the vectors)
+  if (sm > 136 * 1024) return launch_kp_gateup_mq(a, nullptr, nullptr, 1, s);
   const int items = (a.n_ff + 15) / 16;
   const dim3 grid((unsigned)std::max(1, std::min((items + 1) / 2, cu_count()))), b(DEC_MM_NW * 64);
   auto go = [&](auto kern) {

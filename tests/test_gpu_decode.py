@@ -241,6 +241,24 @@ def test_multi_row_passes_mfma(ctx, case, monkeypatch):
     b.close()
 
 
+@pytest.mark.parametrize("fmt", [M.Q4K, M.Q6K], ids=["q4k", "q6k"])
+def test_wide_dense_passes_mfma(ctx, fmt):
+    """Dense gate/up rows of 4096 columns, where two staged tiles and the rows' Q8_K do not fit the LDS
+    from 13 rows (Q4_K) or 6 (Q6_K): every pass size runs, with the lane-exact kernels' bits."""
+    cfg = M.TINY["tiny-qwen3"].replace(sigma=0.02, **KQ).replace(dim=4096, n_ff=1024, t_gate=fmt, t_up=fmt, n_layers=1)
+    w = M.synth_model(cfg, seed=39)
+    a, b = M.Engine(ctx, cfg, w), M.Engine(ctx, cfg, w)
+    b.set_mfma(False)
+    ids, pos = np.random.default_rng(8).integers(0, cfg.vocab, 120), 0
+    for m in (5, 6, 12, 13, 16, 9):
+        am0, h0, l0 = a.forward(ids[pos:pos + m], pos, hidden=True, logits=True)
+        am1, h1, l1 = b.forward(ids[pos:pos + m], pos, hidden=True, logits=True)
+        assert _same(h0, h1) and _same(l0, l1) and np.array_equal(am0, am1), (m, _rel(h0, h1), _rel(l0, l1))
+        pos += m
+    a.close()
+    b.close()
+
+
 @pytest.mark.parametrize("case", list(CASES))
 def test_persistent_pass_bitwise(ctx, case):
     """One-row passes with their layers as cooperative launches (persist.hip) against the decode
